@@ -3258,131 +3258,225 @@ extern "C" int fitsne_symmetrize(const uint32_t *row_P, const uint32_t *col_P, c
     return FITSNE_OK;
 }
 
-extern "C" int fitsne_knn_exact(const double *X, int N, int D, int K, int32_t *idx, double *dist) {
+// The FP64 kernel over all queries, or over the nq listed ones, from device X (rows) into idx and dist.  tmp:
+// device memory for X transposed and the parts' lists.
+static int knn_fp64(fitsne_ctx *c, const double *X, DBuf &tmp, int N, int D, int K, int *idx, double *dist,
+                    const int *qlist, int nq) {
+    int B = 128;
+    while (B < 2 * K || B < K + kWave) B *= 2;
+    // a list too short to fill the chip at kKnnQ queries per wavefront: a query at a time, over parts of
+    // at least 1024 points
+    int parts = 1;
+    if (qlist && nq < 2048) parts = std::min((N + 1023) / 1024, (4096 + nq - 1) / nq);
+    const int per = ((N + parts - 1) / parts + kWave - 1) / kWave * kWave;
+    parts = (N + per - 1) / per;
+    const size_t nd = (size_t)N * D, np = parts > 1 ? (size_t)nq * parts * K : 0;
+    TRY(ensure(tmp, sizeof(double) * (nd + np) + sizeof(int) * np));
+    double *XT = tmp.as<double>(), *pd = XT + nd;
+    int *pi = reinterpret_cast<int *>(pd + np);
+    launch(c, "transpose64", k_transpose_f64, dim3((N + 31) / 32, (D + 31) / 32), dim3(256), 0, X, (long)N, D, XT);
+    const size_t lds = (size_t)B * (sizeof(double) + sizeof(int));
+    if (parts > 1) {
+        launch(c, "knn64_part", k_knn_f64<1, true>, dim3(nq, parts), dim3(kWave), lds, X, (const double *)XT, N, D, K,
+               B, pi, pd, qlist, nq, per);
+        launch(c, "knn64_merge", k_knn_merge, dim3(nq), dim3(kWave), lds, (const int *)pi, (const double *)pd,
+               parts * K, K, B, idx, dist, qlist);
+    } else {
+        launch(c, "knn64", k_knn_f64<kKnnQ, false>, dim3((nq + kKnnQ - 1) / kKnnQ), dim3(kWave), kKnnQ * lds, X,
+               (const double *)XT, N, D, K, B, idx, dist, qlist, nq, 0);
+    }
+    HIPTRY(hipGetLastError());
+    return FITSNE_OK;
+}
+
+// ---------------------------------------------------------------- kNN by the matrix-core filter
+
+// One device allocation of a call, released on every return; take() deals it out in 256-byte steps.
+struct KnnSlab {
+    DBuf b;
+    size_t at = 0;
+    ~KnnSlab() { release(b); }
+    template <typename T>
+    size_t need(size_t n) {
+        const size_t o = at;
+        at += (sizeof(T) * n + 255) & ~(size_t)255;
+        return o;
+    }
+    template <typename T>
+    T *ptr(size_t o) const { return reinterpret_cast<T *>(static_cast<char *>(b.p) + o); }
+};
+
+struct KnnPlan {
+    int N, D, K, nch, stride, NS, npad, nspad, cap, qblocks, parts, per;
+};
+
+// The threshold sample's stride and the list length.  About 33 strides of all points lie nearer than the
+// cut (kKmRank of 64 classes: 64 (H64 - H38) sample points), give or take a fifth.  A list is short only if
+// the nearest K points' sample (K / stride <= 9 of them on average) hits kKmRank classes, and too long only if that
+// of the nearest 77 strides hits fewer: both below 1e-6 per query (which is then recomputed in FP64).  A
+// stride of at least 8 keeps the threshold pass a small part of the candidate pass.
+static KnnPlan knn_plan(int N, int D, int K) {
+    KnnPlan p{};
+    p.N = N;
+    p.D = D;
+    p.K = K;
+    p.nch = (D + kKmAug + 15) / 16;
+    p.stride = std::max(8, (K + 8) / 9);
+    p.cap = p.stride <= 10 ? 768 : p.stride <= 20 ? 1536 : 2304;
+    p.NS = (N + p.stride - 1) / p.stride;
+    p.npad = (N + kKmWg - 1) / kKmWg * kKmWg;
+    p.nspad = (p.NS + 31) / 32 * 32;
+    p.qblocks = p.npad / kKmWg;
+    // enough workgroups for several rounds of the chip, each with at least 16 tiles to sweep
+    const int tiles = (N + 31) / 32;
+    const int parts = std::max(1, std::min(tiles / 16, (2048 + p.qblocks - 1) / p.qblocks));
+    p.per = ((tiles + parts - 1) / parts + 1) / 2 * 2;
+    p.parts = (tiles + p.per - 1) / p.per;
+    return p;
+}
+
+struct KnnDev {
+    const double *X;
+    f16x8 *XC, *XS;
+    f16x4 *QA;
+    double *nrm;
+    float *cut;
+    unsigned long long *cand;
+    int *cnt;
+    KnnScale *sc;
+};
+
+template <int NCH>
+static void knn_passes(fitsne_ctx *c, const KnnPlan &p, const KnnDev &d) {
+    const size_t lds = sizeof(f16x8) * 2 * kKmCt<NCH> * NCH * 2 * kWave;
+    launch(c, "knn_query", k_knn_query, dim3(p.npad / 256), dim3(256), 0, (const double *)d.nrm, p.N, p.npad,
+           (const float *)nullptr, d.QA);
+    launch(c, "knn_tau", k_knn_tau<NCH>, dim3(p.qblocks), dim3(kKmThreads), lds, (const f16x8 *)d.XC,
+           (const f16x4 *)d.QA, p.N, p.D, (const f16x8 *)d.XS, p.NS, p.stride, d.cut);
+    launch(c, "knn_query", k_knn_query, dim3(p.npad / 256), dim3(256), 0, (const double *)d.nrm, p.N, p.npad,
+           (const float *)d.cut, d.QA);
+    launch(c, "knn_collect", k_knn_collect<NCH>, dim3(p.qblocks * p.parts), dim3(kKmThreads), lds,
+           (const f16x8 *)d.XC, (const f16x4 *)d.QA, p.N, p.D, p.qblocks, p.per, p.cap, d.cand, d.cnt);
+}
+
+// Neighbours by the filter, the queries it cannot settle by the FP64 kernel (their number into *nredo).
+// D <= kKmMaxD, K <= kKmMaxK.
+static int knn_filtered(fitsne_ctx *c, const double *X, int N, int D, int K, int32_t *idx, double *dist, int *nredo) {
+    const KnnPlan p = knn_plan(N, D, K);
+    const size_t nd = (size_t)N * D, nk = (size_t)N * K, tile = (size_t)p.nch * 2 * kWave;
+    const int cblk = (N + kKmRows - 1) / kKmRows, eblk = (N + 255) / 256, tblk = p.npad / 32;
+    KnnSlab m;
+    const size_t oX = m.need<double>(nd), oXC = m.need<f16x8>(p.npad / 32 * tile), oXS = m.need<f16x8>(p.nspad / 32 * tile);
+    const size_t oQA = m.need<f16x4>(p.npad), oN = m.need<double>(N), oCut = m.need<float>(N);
+    const size_t oCand = m.need<unsigned long long>((size_t)N * p.cap), oCnt = m.need<int>(N);
+    const size_t oI = m.need<int>(nk), oD = m.need<double>(nk), oR = m.need<int>((size_t)N + 1);
+    const size_t oPart = m.need<double>(std::max((size_t)cblk * D + eblk, (size_t)tblk)), oMean = m.need<double>(D), oSc = m.need<KnnScale>(1);
+    TRY(ensure(m.b, m.at));
+    const KnnDev d{m.ptr<double>(oX), m.ptr<f16x8>(oXC), m.ptr<f16x8>(oXS), m.ptr<f16x4>(oQA), m.ptr<double>(oN),
+                   m.ptr<float>(oCut), m.ptr<unsigned long long>(oCand), m.ptr<int>(oCnt), m.ptr<KnnScale>(oSc)};
+    double *part = m.ptr<double>(oPart), *mean = m.ptr<double>(oMean);
+    int *redo = m.ptr<int>(oR), *nr = redo + N, *di = m.ptr<int>(oI);
+    double *dd = m.ptr<double>(oD);
+    HIPTRY(hipMemcpyAsync(m.ptr<double>(oX), X, sizeof(double) * nd, hipMemcpyHostToDevice, c->stream));
+    launch(c, "fill", k_fill<int>, dim3(1), dim3(kWave), 0, nr, 1L, 0);
+    launch(c, "fill", k_fill<int>, dim3(std::min(blocks_for(N), 1024)), dim3(kThreads), 0, d.cnt, (long)N, 0);
+    launch(c, "knn_colsum", k_knn_colsum, dim3(cblk), dim3(256), 0, d.X, N, D, part);
+    launch(c, "knn_colmean", k_knn_colmean, dim3(1), dim3(1024), 0, (const double *)part, cblk, N, D, mean);
+    launch(c, "knn_extent", k_knn_extent, dim3(eblk), dim3(256), 0, d.X, N, D, (const double *)mean,
+           part + (size_t)cblk * D);
+    launch(c, "knn_scale", k_knn_scale, dim3(1), dim3(1024), 0, (const double *)(part + (size_t)cblk * D), eblk,
+           (const double *)mean, D, d.sc);
+    launch(c, "knn_prep", k_knn_prep, dim3(tblk), dim3(256), 0, d.X, N, D, p.nch, (const double *)mean,
+           (const KnnScale *)d.sc, p.stride, p.NS, p.nspad, d.XC, d.XS, d.nrm, part);
+    launch(c, "knn_nmax", k_knn_nmax, dim3(1), dim3(1024), 0, (const double *)part, tblk, d.sc);
+    switch (p.nch) {
+    case 1: knn_passes<1>(c, p, d); break;
+    case 2: knn_passes<2>(c, p, d); break;
+    case 3: knn_passes<3>(c, p, d); break;
+    case 4: knn_passes<4>(c, p, d); break;
+    case 5: knn_passes<5>(c, p, d); break;
+    case 6: knn_passes<6>(c, p, d); break;
+    case 7: knn_passes<7>(c, p, d); break;
+    case 8: knn_passes<8>(c, p, d); break;
+    default: knn_passes<9>(c, p, d); break;
+    }
+    auto rerank = p.cap == 768 ? k_knn_rerank<12> : p.cap == 1536 ? k_knn_rerank<24> : k_knn_rerank<36>;
+    launch(c, "knn_rerank", rerank, dim3(N), dim3(kWave), 0, d.X, N, D, K, 16 * p.nch,
+           (const unsigned long long *)d.cand, (const int *)d.cnt, (const float *)d.cut, (const double *)d.nrm,
+           (const KnnScale *)d.sc, di, dd, redo, nr);
+    HIPTRY(hipGetLastError());
+    int n = 0;
+    HIPTRY(hipMemcpyAsync(&n, nr, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPTRY(hipStreamSynchronize(c->stream));
+    if (n < 0 || n > N) return fail(FITSNE_E_HIP, "inconsistent recompute count");
+    KnnSlab xt;
+    if (n > 0) TRY(knn_fp64(c, d.X, xt.b, N, D, K, di, dd, redo, n));
+    HIPTRY(hipMemcpyAsync(idx, di, sizeof(int) * nk, hipMemcpyDeviceToHost, c->stream));
+    HIPTRY(hipMemcpyAsync(dist, dd, sizeof(double) * nk, hipMemcpyDeviceToHost, c->stream));
+    TRY(sync_ctx(c));
+    if (nredo) *nredo = n;
+    return FITSNE_OK;
+}
+
+static int knn_args(const double *X, int N, int D, int K, const int32_t *idx, const double *dist) {
     if (!X || !idx || !dist || N < 2 || D < 1 || K < 1) return fail(FITSNE_E_ARG, "invalid kNN arguments");
     if (K > N - 1) return fail(FITSNE_E_ARG, "K must be at most N - 1");
     if (K > 1000) return fail(FITSNE_E_UNSUPPORTED, "K above 1000 is not supported");
-    const size_t nd = (size_t)N * D;
+    return FITSNE_OK;
+}
+
+static int knn_finite(const double *X, size_t nd) {
     for (size_t i = 0; i < nd; i++)
         if (!std::isfinite(X[i])) return fail(FITSNE_E_ARG, "X contains non-finite values");
-    std::lock_guard<std::mutex> lk(g_mirror_mu);
-    fitsne_ctx *c;
-    TRY(mirror_ctx(&c, 1, 3, 1.0, 1, 1.0));
-    HIPTRY(hipSetDevice(c->device));
-    TRY(ensure(c->knnX, sizeof(double) * nd));
-    TRY(ensure(c->knnXT, sizeof(double) * nd));
+    return FITSNE_OK;
+}
+
+// X up, the FP64 kernel over all queries, neighbours down.
+static int knn_plain(fitsne_ctx *c, const double *X, int N, int D, int K, int32_t *idx, double *dist) {
+    TRY(ensure(c->knnX, sizeof(double) * (size_t)N * D));
     TRY(ensure(c->knnI, sizeof(int) * (size_t)N * K));
     TRY(ensure(c->knnD, sizeof(double) * (size_t)N * K));
-    HIPTRY(hipMemcpy(c->knnX.p, X, sizeof(double) * nd, hipMemcpyHostToDevice));
-    launch(c, "transpose64", k_transpose_f64, dim3((N + 31) / 32, (D + 31) / 32), dim3(256), 0,
-           c->knnX.as<const double>(), (long)N, D, c->knnXT.as<double>());
-    int B = 128;
-    while (B < 2 * K || B < K + kWave) B *= 2;
-    const size_t lds = (size_t)kKnnQ * B * (sizeof(double) + sizeof(int));
-    launch(c, "knn64", k_knn_f64, dim3((N + kKnnQ - 1) / kKnnQ), dim3(kWave), lds, c->knnX.as<const double>(),
-           c->knnXT.as<const double>(), N, D, K, B, c->knnI.as<int>(), c->knnD.as<double>(), (const int *)nullptr, N);
-    HIPTRY(hipGetLastError());
+    HIPTRY(hipMemcpy(c->knnX.p, X, sizeof(double) * (size_t)N * D, hipMemcpyHostToDevice));
+    TRY(knn_fp64(c, c->knnX.as<const double>(), c->knnXT, N, D, K, c->knnI.as<int>(), c->knnD.as<double>(), nullptr, N));
     HIPTRY(hipMemcpyAsync(idx, c->knnI.p, sizeof(int) * (size_t)N * K, hipMemcpyDeviceToHost, c->stream));
     HIPTRY(hipMemcpyAsync(dist, c->knnD.p, sizeof(double) * (size_t)N * K, hipMemcpyDeviceToHost, c->stream));
     return sync_ctx(c);
 }
 
-// ---------------------------------------------------------------- kNN for large N (FP32 MFMA candidates)
+// The filter's fewest points (its sample must hit kKmRank classes), and the least work fitsne_knn_exact
+// takes it for.  The filter's dozen launches cost 0.5 to 0.7 ms whatever the size; the FP64 kernel's time
+// goes with N (D + 40) while N is small (whole calls, D = 50, K = 90: 0.79 against 0.80 ms at N = 1,500, 1.92
+// against 0.89 at 5,000; D = 20, K = 30: 0.41 against 0.55 ms at 2,000, 0.79 against 0.54 at 5,000; D = 100,
+// K = 30: 0.63 against 0.59 ms at 1,024).
+constexpr int kKnnFilterMinN = 1024;
+constexpr long kKnnFilterWork = 150000;
 
-// Device buffers of one call, released on every return.
-struct KnnmBufs {
-    DBuf X, XT, XT4, nrm, nrm64, XS4, nrs, tau, cand, cnt, idx, dist, redo, nredo, nmax;
-    ~KnnmBufs() {
-        DBuf *all[] = {&X, &XT, &XT4, &nrm, &nrm64, &XS4, &nrs, &tau, &cand, &cnt, &idx, &dist, &redo, &nredo, &nmax};
-        for (DBuf *b : all) release(*b);
-    }
-};
-
-template <int NCH>
-static void knnm_passes(hipStream_t st, KnnmBufs &m, int N, int NS) {
-    const int nblk = (N + kKmWaves * kKmQ - 1) / (kKmWaves * kKmQ);
-    k_knnm_tau<NCH><<<dim3(nblk), dim3(kKmWaves * kWave), 0, st>>>(m.XT4.as<const float>(), N, m.nrm.as<const float>(),
-                                                                   m.XS4.as<const float>(), NS,
-                                                                   m.nrs.as<const float>(), m.tau.as<float>());
-    k_knnm_collect<NCH><<<dim3(nblk), dim3(kKmWaves * kWave), 0, st>>>(m.XT4.as<const float>(), N,
-                                                                       m.nrm.as<const float>(),
-                                                                       m.tau.as<const float>(), m.cand.as<int>(),
-                                                                       m.cnt.as<int>());
-}
-
-extern "C" int fitsne_knn_mfma(const double *X, int N, int D, int K, int32_t *idx, double *dist,
-                               long long *recomputed) {
-    if (!X || !idx || !dist || N < 2 || D < 1 || K < 1) return fail(FITSNE_E_ARG, "invalid kNN arguments");
-    if (K > N - 1) return fail(FITSNE_E_ARG, "K must be at most N - 1");
-    if (K > 1000) return fail(FITSNE_E_UNSUPPORTED, "K above 1000 is not supported");
-    if (D > 128) return fail(FITSNE_E_UNSUPPORTED, "the MFMA kNN takes D <= 128 (use fitsne_knn_exact)");
-    if (K > kKmCap / 2) return fail(FITSNE_E_UNSUPPORTED, "the MFMA kNN takes K <= 256 (use fitsne_knn_exact)");
-    const size_t nd = (size_t)N * D;
-    for (size_t i = 0; i < nd; i++)
-        if (!std::isfinite(X[i])) return fail(FITSNE_E_ARG, "X contains non-finite values");
-    const int need = (D + 3) / 4;
-    const int nch = need <= 8 ? 8 : need <= 13 ? 13 : need <= 16 ? 16 : need <= 25 ? 25 : 32;
-    const int NS = (N + kKmStride - 1) / kKmStride;
+extern "C" int fitsne_knn_exact(const double *X, int N, int D, int K, int32_t *idx, double *dist) {
+    TRY(knn_args(X, N, D, K, idx, dist));
+    TRY(knn_finite(X, (size_t)N * D));
     std::lock_guard<std::mutex> lk(g_mirror_mu);
     fitsne_ctx *c;
     TRY(mirror_ctx(&c, 1, 3, 1.0, 1, 1.0));
     HIPTRY(hipSetDevice(c->device));
-    hipStream_t st = c->stream;
-    KnnmBufs m;
-    TRY(ensure(m.X, sizeof(double) * nd));
-    TRY(ensure(m.XT4, sizeof(float4) * (size_t)nch * N));
-    TRY(ensure(m.nrm, sizeof(float) * N));
-    TRY(ensure(m.nrm64, sizeof(double) * N));
-    TRY(ensure(m.XS4, sizeof(float4) * (size_t)nch * NS));
-    TRY(ensure(m.nrs, sizeof(float) * NS));
-    TRY(ensure(m.tau, sizeof(float) * N));
-    TRY(ensure(m.cand, sizeof(int) * (size_t)N * kKmCap));
-    TRY(ensure(m.cnt, sizeof(int) * N));
-    TRY(ensure(m.idx, sizeof(int) * (size_t)N * K));
-    TRY(ensure(m.dist, sizeof(double) * (size_t)N * K));
-    TRY(ensure(m.redo, sizeof(int) * N));
-    TRY(ensure(m.nredo, sizeof(int)));
-    TRY(ensure(m.nmax, sizeof(double)));
-    HIPTRY(hipMemcpy(m.X.p, X, sizeof(double) * nd, hipMemcpyHostToDevice));
-    k_fill<int><<<dim3(1), dim3(kWave), 0, st>>>(m.nredo.as<int>(), 1, 0);
-    k_knnm_prep<<<dim3((N + 255) / 256), dim3(256), 0, st>>>(m.X.as<const double>(), N, D, nch, m.XT4.as<float4>(),
-                                                             m.nrm.as<float>(), m.nrm64.as<double>(), NS,
-                                                             m.XS4.as<float4>(), m.nrs.as<float>());
-    k_knnm_max<<<dim3(1), dim3(1024), 0, st>>>(m.nrm64.as<const double>(), (long)N, m.nmax.as<double>());
-    switch (nch) {
-    case 8: knnm_passes<8>(st, m, N, NS); break;
-    case 13: knnm_passes<13>(st, m, N, NS); break;
-    case 16: knnm_passes<16>(st, m, N, NS); break;
-    case 25: knnm_passes<25>(st, m, N, NS); break;
-    default: knnm_passes<32>(st, m, N, NS); break;
-    }
-    const double epsu = 2.0 * (4.0 * nch + 8.0) * std::ldexp(1.0, -24);
-    k_knnm_exact<<<dim3(N), dim3(kWave), 0, st>>>(m.X.as<const double>(), N, D, K, m.cand.as<const int>(),
-                                                  m.cnt.as<const int>(), m.tau.as<const float>(),
-                                                  m.nrm64.as<const double>(), m.nmax.as<const double>(), epsu,
-                                                  m.idx.as<int>(), m.dist.as<double>(), m.redo.as<int>(),
-                                                  m.nredo.as<int>());
-    HIPTRY(hipGetLastError());
-    int nredo = 0;
-    HIPTRY(hipMemcpyAsync(&nredo, m.nredo.p, sizeof(int), hipMemcpyDeviceToHost, st));
-    HIPTRY(hipStreamSynchronize(st));
-    if (nredo < 0 || nredo > N) return fail(FITSNE_E_HIP, "inconsistent recompute count");
-    if (nredo > 0) {  // the queries the candidate lists could not settle: the FP64 kernel over all points
-        TRY(ensure(m.XT, sizeof(double) * nd));
-        k_transpose_f64<<<dim3((N + 31) / 32, (D + 31) / 32), dim3(256), 0, st>>>(m.X.as<const double>(), (long)N, D,
-                                                                                m.XT.as<double>());
-        int B = 128;
-        while (B < 2 * K || B < K + kWave) B *= 2;
-        const size_t lds = (size_t)kKnnQ * B * (sizeof(double) + sizeof(int));
-        k_knn_f64<<<dim3((nredo + kKnnQ - 1) / kKnnQ), dim3(kWave), lds, st>>>(
-            m.X.as<const double>(), m.XT.as<const double>(), N, D, K, B, m.idx.as<int>(), m.dist.as<double>(),
-            m.redo.as<const int>(), nredo);
-        HIPTRY(hipGetLastError());
-    }
-    HIPTRY(hipMemcpyAsync(idx, m.idx.p, sizeof(int) * (size_t)N * K, hipMemcpyDeviceToHost, st));
-    HIPTRY(hipMemcpyAsync(dist, m.dist.p, sizeof(double) * (size_t)N * K, hipMemcpyDeviceToHost, st));
-    HIPTRY(hipStreamSynchronize(st));
-    if (recomputed) *recomputed = nredo;
+    if (N >= kKnnFilterMinN && D <= kKmMaxD && K <= kKmMaxK && (long)N * (D + 40) >= kKnnFilterWork)
+        return knn_filtered(c, X, N, D, K, idx, dist, nullptr);
+    return knn_plain(c, X, N, D, K, idx, dist);
+}
+
+extern "C" int fitsne_knn_mfma(const double *X, int N, int D, int K, int32_t *idx, double *dist,
+                               long long *recomputed) {
+    TRY(knn_args(X, N, D, K, idx, dist));
+    if (D > kKmMaxD) return fail(FITSNE_E_UNSUPPORTED, "the MFMA kNN takes D <= 128 (use fitsne_knn_exact)");
+    if (K > kKmMaxK) return fail(FITSNE_E_UNSUPPORTED, "the MFMA kNN takes K <= 256 (use fitsne_knn_exact)");
+    TRY(knn_finite(X, (size_t)N * D));
+    std::lock_guard<std::mutex> lk(g_mirror_mu);
+    fitsne_ctx *c;
+    TRY(mirror_ctx(&c, 1, 3, 1.0, 1, 1.0));
+    HIPTRY(hipSetDevice(c->device));
+    int n = N;
+    if (N >= kKnnFilterMinN) TRY(knn_filtered(c, X, N, D, K, idx, dist, &n));
+    else TRY(knn_plain(c, X, N, D, K, idx, dist));
+    if (recomputed) *recomputed = n;
     return FITSNE_OK;
 }
 

@@ -2,7 +2,7 @@
 //
 // TSNE::run finds each point's K nearest other points with a VP tree (tsne.cpp:1643-1726), whose
 // distance is sqrt(sum_d (x_d - y_d)^2) accumulated in order d = 0..D-1 without fused multiply-adds
-// (vptree.h:97-107).  Here one wavefront serves kKnnQ query points: every lane takes one candidate per
+// (vptree.h:97-107).  Here one wavefront serves kKnnQ query points (a query at a time in short lists): every lane takes one candidate per
 // round, accumulates its squared distances to the kKnnQ queries in the same order and rounding
 // (contraction to fused multiply-adds switched off; the root by the correctly rounded __dsqrt_rn),
 // and candidates below the query's current K-th distance are appended to an LDS buffer of B slots
@@ -75,42 +75,48 @@ __device__ void knn_compact(double *key, int *idx, int cnt, int B) {
     knn_sort(key, idx, B);
 }
 
-// One workgroup = one wavefront = kKnnQ queries: points blockIdx.x * kKnnQ + j, or, with a query list,
-// qlist[blockIdx.x * kKnnQ + j] for list positions below nq.  Dynamic LDS: kKnnQ * B * (8 + 4) bytes,
-// where B = power of two >= max(2K, K + 64, 128) so that a round of 64 appends always fits after a cut.
+// One workgroup = one wavefront = Q queries: points blockIdx.x * Q + j, or, with a query list,
+// qlist[blockIdx.x * Q + j] for list positions below nq.  Dynamic LDS: Q * B * (8 + 4) bytes, where
+// B = power of two >= max(2K, K + 64, 128) so that a round of 64 appends always fits after a cut.
+// PART: a short query list is swept by gridDim.y wavefronts per query, `per` points each, which leave their
+// K nearest as squared distances in part_d / part_i [query][part][K] for k_knn_merge: alone, a
+// wavefront took 175 ms over 300,000 points at D = 100 (the latency of its N / 64 * D steps).
+template <int Q, bool PART>
 __global__ __launch_bounds__(kWave) void k_knn_f64(const double *__restrict__ X, const double *__restrict__ XT,
                                                    int N, int D, int K, int B, int *__restrict__ out_idx,
                                                    double *__restrict__ out_dist, const int *__restrict__ qlist,
-                                                   int nq) {
+                                                   int nq, int per) {
     extern __shared__ double knn_smem[];
     double *bk = knn_smem;
-    int *bi = reinterpret_cast<int *>(knn_smem + (long)kKnnQ * B);
+    int *bi = reinterpret_cast<int *>(knn_smem + (long)Q * B);
     const int lane = threadIdx.x;
-    int qid[kKnnQ];  // the block's queries (-1: none)
+    const int lo = PART ? blockIdx.y * per : 0, hi = PART ? min(N, lo + per) : N;
+    int qid[Q];  // the block's queries (-1: none)
 #pragma unroll
-    for (int j = 0; j < kKnnQ; j++) {
-        const int s = blockIdx.x * kKnnQ + j;
+    for (int j = 0; j < Q; j++) {
+        const int s = blockIdx.x * Q + j;
         qid[j] = qlist ? (s < nq ? qlist[s] : -1) : (s < N ? s : -1);
     }
-    int cnt[kKnnQ];
-    double thr[kKnnQ];
+    int cnt[Q];
+    double thr[Q];
 #pragma unroll
-    for (int j = 0; j < kKnnQ; j++) {
+    for (int j = 0; j < Q; j++) {
         cnt[j] = 0;
         thr[j] = DBL_MAX;
     }
-    for (int c0 = 0; c0 < N; c0 += kWave) {
+    for (int c0 = lo; c0 < hi; c0 += kWave) {
         const int c = c0 + lane;
-        double acc[kKnnQ];
+        double acc[Q];
 #pragma unroll
-        for (int j = 0; j < kKnnQ; j++) acc[j] = 0.0;
-        if (c < N) {
+        for (int j = 0; j < Q; j++) acc[j] = 0.0;
+        if (c < hi) {
             // separate multiply and add, as the host's loop (no fused multiply-add)
 #pragma clang fp contract(off)
+#pragma unroll 4
             for (int d = 0; d < D; d++) {
                 const double xc = XT[(long)d * N + c];
 #pragma unroll
-                for (int j = 0; j < kKnnQ; j++) {
+                for (int j = 0; j < Q; j++) {
                     const int qi = qid[j] >= 0 ? qid[j] : 0;
                     const double diff = X[(long)qi * D + d] - xc;
                     acc[j] += diff * diff;
@@ -118,9 +124,9 @@ __global__ __launch_bounds__(kWave) void k_knn_f64(const double *__restrict__ X,
             }
         }
 #pragma unroll
-        for (int j = 0; j < kKnnQ; j++) {
+        for (int j = 0; j < Q; j++) {
             const int qi = qid[j];
-            const bool take = c < N && qi >= 0 && c != qi && acc[j] < thr[j];
+            const bool take = c < hi && qi >= 0 && c != qi && acc[j] < thr[j];
             const unsigned long long m = __ballot(take);
             if (m) {
                 const int pos = cnt[j] + __popcll(m & ((1ull << lane) - 1ull));
@@ -141,15 +147,60 @@ __global__ __launch_bounds__(kWave) void k_knn_f64(const double *__restrict__ X,
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kKnnQ; j++) {
+    for (int j = 0; j < Q; j++) {
         const int qi = qid[j];
         knn_compact(bk + j * B, bi + j * B, cnt[j], B);
-        if (qi >= 0)
+        if (qi >= 0) {
+            const long base = PART ? ((long)(blockIdx.x * Q + j) * gridDim.y + blockIdx.y) * K : (long)qi * K;
             for (int m = lane; m < K; m += kWave) {
-                out_idx[(long)qi * K + m] = bi[j * B + m];
-                out_dist[(long)qi * K + m] = __dsqrt_rn(bk[j * B + m]);  // correctly rounded, as the host's sqrt
+                out_idx[base + m] = bi[j * B + m];
+                // correctly rounded, as the host's sqrt
+                out_dist[base + m] = PART ? bk[j * B + m] : __dsqrt_rn(bk[j * B + m]);
             }
+        }
         __syncthreads();
+    }
+}
+
+// The K nearest of query qlist[blockIdx.x] from its parts' lists (n entries, padding as (DBL_MAX, INT_MAX)),
+// by the same buffer and order.  A cut keeps ties by the smaller index: entries equal to the threshold
+// distance are taken too.
+__global__ __launch_bounds__(kWave) void k_knn_merge(const int *__restrict__ part_i, const double *__restrict__ part_d,
+                                                     int n, int K, int B, int *__restrict__ out_idx,
+                                                     double *__restrict__ out_dist, const int *__restrict__ qlist) {
+    extern __shared__ double knn_smem[];
+    double *bk = knn_smem;
+    int *bi = reinterpret_cast<int *>(knn_smem + B);
+    const int lane = threadIdx.x;
+    const long base = (long)blockIdx.x * n;
+    int cnt = 0;
+    double thr = DBL_MAX;
+    for (int e0 = 0; e0 < n; e0 += kWave) {
+        const int e = e0 + lane;
+        const double d = e < n ? part_d[base + e] : DBL_MAX;
+        const bool take = e < n && d < DBL_MAX && d <= thr;
+        const unsigned long long m = __ballot(take);
+        if (!m) continue;
+        const int pos = cnt + __popcll(m & ((1ull << lane) - 1ull));
+        if (take) {
+            bk[pos] = d;
+            bi[pos] = part_i[base + e];
+        }
+        cnt += __popcll(m);
+        if (cnt > B - kWave) {
+            __syncthreads();
+            knn_compact(bk, bi, cnt, B);
+            cnt = K;
+            thr = bk[K - 1];
+            __syncthreads();
+        }
+    }
+    __syncthreads();
+    knn_compact(bk, bi, cnt, B);
+    const int q = qlist[blockIdx.x];
+    for (int m = lane; m < K; m += kWave) {
+        out_idx[(long)q * K + m] = bi[m];
+        out_dist[(long)q * K + m] = __dsqrt_rn(bk[m]);
     }
 }
 

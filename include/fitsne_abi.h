@@ -135,12 +135,13 @@ int fitsne_distances2similarities_batch(const double *D, double *P, int n_points
  * K <= min(N - 1, 1000); X must be finite. */
 int fitsne_knn_exact(const double *X, int N, int D, int K, int32_t *idx, double *dist);
 
-/* The same neighbours as fitsne_knn_exact, bit for bit, for large N: candidates from FP32 MFMA distances
- * (a sampled threshold, then every point below it), their FP64 distances in the reference's order, and
- * the FP64 kernel for any query whose candidates cannot be shown to contain its K nearest (their count,
- * or the K-th distance against the threshold minus the FP32 error bound).  D <= 128, K <= 256;
- * recomputed (nullable) receives the number of such queries.  Same role as fitsne_knn_exact: the exact
- * kNN of TSNE::run (tsne.cpp:1643-1726, vptree.h). */
+/* The same neighbours as fitsne_knn_exact, bit for bit, for large N: candidates from approximate distances on
+ * the matrix cores (a sampled threshold, then every point below it), their FP64 distances in the reference's
+ * order, and the FP64 kernel for any query whose candidates cannot be shown to contain its K nearest (their
+ * count, or the K-th distance against the threshold minus the error bound), and for all of them when N <
+ * 1024.  D <= 128, K <= 256; recomputed (nullable) receives the number of queries the FP64 kernel took.
+ * fitsne_knn_exact takes the same route where it is faster.  Same role: the exact kNN of TSNE::run
+ * (tsne.cpp:1643-1726, vptree.h). */
 int fitsne_knn_mfma(const double *X, int N, int D, int K, int32_t *idx, double *dist, long long *recomputed);
 
 /* symmetrizeMatrix (tsne.cpp:1730-1828) on the GPU: the same output rows, entry order and values

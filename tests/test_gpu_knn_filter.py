@@ -1,0 +1,77 @@
+"""The matrix-core filter behind fitsne_knn_mfma (N >= 1024) and fitsne_knn_exact (where it is faster), against
+the oracle's VP-tree distances and against the FP64 kernel (reached with K = 257): the same neighbours and
+distances, bit for bit.  Sizes at the edges of its tiles (32 points), workgroups (256 queries), chunks (16
+coordinates, six of them the norms'), list lengths and thresholds; data far off centre, of extreme magnitude,
+with repeated points and constant coordinates."""
+import numpy as np
+import pytest
+
+import fitsne_gpu as fg
+import orc
+
+pytestmark = pytest.mark.gpu
+
+
+def mixture(N, D, seed, k=12):
+    rng = np.random.default_rng(seed)
+    return rng.normal(0.0, 4.0, size=(k, D))[rng.integers(0, k, size=N)] + rng.normal(size=(N, D))
+
+
+def check(X, K, got):
+    idx, dist = got
+    ridx, rdist = orc.knn_exact(X, K)
+    assert np.array_equal(idx, ridx)
+    assert np.array_equal(dist, rdist)
+
+
+@pytest.mark.parametrize("N,D,K", [
+    (1024, 10, 5), (1025, 11, 90), (1055, 26, 13), (1087, 42, 104), (1280, 58, 105), (1281, 74, 150), (1311, 90, 208),
+    (1536, 106, 209), (1999, 122, 256), (2049, 128, 30), (3000, 1, 40), (3001, 2, 90)])
+def test_filter_matches_the_oracle(N, D, K):
+    X = mixture(N, D, N + D)
+    print(f"[gpu] knn filter N={N} D={D} K={K}", flush=True)
+    check(X, K, fg.knn_exact(X, K))
+    check(X, K, fg.knn_mfma(X, K)[:2])
+
+
+@pytest.mark.parametrize("N", [2, 33, 255, 256, 257, 511, 512, 513, 545, 1023])
+def test_small_inputs_match_the_oracle(N):
+    X = mixture(N, 7, N)
+    K = min(N - 1, 200)
+    print(f"[gpu] knn_mfma N={N} K={K}", flush=True)
+    i, d, _ = fg.knn_mfma(X, K)
+    check(X, K, (i, d))
+
+
+@pytest.mark.parametrize("name", ["offset", "far", "tiny", "huge", "repeated", "constant", "one_axis", "all_equal"])
+def test_filter_on_awkward_data(name):
+    X = mixture(1500, 20, 3)
+    if name == "offset":
+        X = X + 1e6
+    elif name == "far":  # centring leaves too few bits for the halves: the FP64 kernel takes it
+        X = X + 1e12
+    elif name == "tiny":
+        X = X * 1e-170
+    elif name == "huge":
+        X = X * 1e150
+    elif name == "repeated":
+        X[700:1400] = X[:700]
+    elif name == "constant":
+        X[:, 5:] = 3.0
+    elif name == "one_axis":
+        X[:, 1:] *= 1e-7
+    else:
+        X[:] = X[0]
+    print(f"[gpu] knn filter data={name}", flush=True)
+    check(X, 45, fg.knn_mfma(X, 45)[:2])
+
+
+@pytest.mark.parametrize("N,D,K", [(20011, 50, 90), (33000, 100, 150)])
+def test_filter_matches_the_fp64_kernel(N, D, K):
+    X = mixture(N, D, N, k=30)
+    print(f"[gpu] knn filter N={N} D={D} K={K} against the FP64 kernel", flush=True)
+    i_f, d_f, redo = fg.knn_mfma(X, K)
+    i_e, d_e = fg.knn_exact(X, 257)
+    assert np.array_equal(i_f, i_e[:, :K])
+    assert np.array_equal(d_f, d_e[:, :K])
+    assert redo <= N // 100
