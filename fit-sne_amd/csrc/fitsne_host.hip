@@ -165,7 +165,7 @@ struct fitsne_ctx {
     DBuf xs, ys, box, wx, wy, ch, w, V, potA, potB;
     // exact path (dense P in val): per-row attractive / repulsive sums and Z shares
     DBuf att, rep, zrow;
-    // Barnes-Hut: the host tree of the current Y and its device copy (pre-order), theta
+    // Barnes-Hut: theta, the host tree and the tree of the current Y on the device (pre-order)
     double theta = 0.5;
     BhTree<1> bh_tree1;
     BhTree<2> bh_tree2;
@@ -173,8 +173,13 @@ struct fitsne_ctx {
     std::vector<double> bh_y;
     void *bh_pin = nullptr;  // pinned host memory: Y, then the flattened tree
     size_t bh_pin_cap = 0;
-    size_t bh_nodes = 0;
-    DBuf bh_tree_d, bh_neg, bh_Q;
+    DBuf bh_cell, bh_leafpt, bh_neg, bh_Q;
+    // the GPU tree's workspaces: root, keys, point numbers (sorted behind the unsorted), positions' arrays, spans,
+    // lists, order by level, sort storage, update factors for bh_ab_n points
+    DBuf bh_root, bh_key, bh_idx, bh_pos, bh_span, bh_list, bh_order, bh_tmp, bh_ab;
+    int bh_ab_n = 0;
+    hipEvent_t bh_ev = nullptr;
+    bool bh_sorted = false;  // the current tree came from the GPU: bh_idx holds the points in key order
     // symmetrisation of a CSR P (mirror tier)
     DBuf sy_row, sy_col, sy_val, sy_erow, sy_keys, sy_keys2, sy_vals, sy_vals2, sy_partner, sy_cnt, sy_start,
         sy_okeys, sy_okeys2, sy_tmp, sy_scol, sy_sval;
@@ -1391,10 +1396,13 @@ static BhTree<D> &bh_tree_for(fitsne_ctx *c) {
     else return c->bh_tree3;
 }
 
-// The SPTree of the resident Y, built on the host in insertion order (from a cached host copy of Y) and
-// uploaded in pre-order, one copy each way through pinned memory.
 template <int D>
-static int bh_tree_of_Y(fitsne_ctx *c) {
+static BhCell<D> *bh_cells(const fitsne_ctx *c) { return c->bh_cell.as<BhCell<D>>(); }
+
+// The tree of the resident Y by the reference's insertions on the host, uploaded in pre-order; one copy each
+// way through pinned memory.
+template <int D>
+static int bh_tree_on_host(fitsne_ctx *c) {
     const int N = c->N;
     const size_t ybytes = sizeof(double) * (size_t)N * D;
     TRY(bh_pinned(c, ybytes));
@@ -1404,12 +1412,144 @@ static int bh_tree_of_Y(fitsne_ctx *c) {
     std::memcpy(c->bh_y.data(), c->bh_pin, ybytes);
     BhTree<D> &t = bh_tree_for<D>(c);
     t.build(c->bh_y.data(), N);
-    const size_t n = t.nodes.size(), tbytes = bh_flat_bytes(n, D);
-    TRY(bh_pinned(c, tbytes));
-    bh_flatten(t, BhFlatView(c->bh_pin, n, D));
-    TRY(ensure(c->bh_tree_d, tbytes));
-    HIPTRY(hipMemcpyAsync(c->bh_tree_d.p, c->bh_pin, tbytes, hipMemcpyHostToDevice, c->stream));
-    c->bh_nodes = n;
+    const size_t n = t.nodes.size();
+    TRY(bh_pinned(c, n * (sizeof(BhCell<D>) + sizeof(int))));
+    auto *cell = static_cast<BhCell<D> *>(c->bh_pin);
+    int *pt = reinterpret_cast<int *>(cell + n);
+    bh_flatten(t, cell, pt);
+    TRY(ensure(c->bh_cell, sizeof(BhCell<D>) * n));
+    TRY(ensure(c->bh_leafpt, sizeof(int) * n));
+    HIPTRY(hipMemcpyAsync(c->bh_cell.p, cell, sizeof(BhCell<D>) * n, hipMemcpyHostToDevice, c->stream));
+    HIPTRY(hipMemcpyAsync(c->bh_leafpt.p, pt, sizeof(int) * n, hipMemcpyHostToDevice, c->stream));
+    c->bh_sorted = false;
+    return FITSNE_OK;
+}
+
+// The tree of the resident Y (fitsne_bh.hpp): on the GPU unless it needs the reference's insertions.  beside():
+// work for a side stream that needs only P and Y.  Side streams: the exact mean, the check of the keys against
+// it and beside() on one, the root's center of mass on the other; the walk waits for both.  The host
+// reads back twice: the node count, which sizes what follows, and the check, by when the rest is queued.
+template <int D, typename F>
+static int bh_tree_of_Y(fitsne_ctx *c, F &&beside) {
+    const int N = c->N;
+    const double *Y = c->Y.as<const double>();
+    if (!c->astream) HIPTRY(hipStreamCreateWithFlags(&c->astream, hipStreamNonBlocking));
+    if (!c->kstream) HIPTRY(hipStreamCreateWithFlags(&c->kstream, hipStreamNonBlocking));
+    if (!c->bh_ev) HIPTRY(hipEventCreateWithFlags(&c->bh_ev, hipEventDisableTiming));  // the host reads a copy after it
+    if (c->bh_ab_n != N) {
+        TRY(ensure(c->bh_ab, sizeof(double2) * ((size_t)N + 1)));
+        launch(c, "bh_factors", k_bh_factors, dim3(blocks_for(N)), dim3(kThreads), 0, c->bh_ab.as<double2>(), N);
+        c->bh_ab_n = N;
+    }
+    const size_t n64 = sizeof(uint64_t) * (size_t)N, n32 = sizeof(int) * ((size_t)N + 1);
+    const int eblk = (N + kBhExtentPer - 1) / kBhExtentPer;
+    TRY(ensure(c->bh_root, 2 * sizeof(BhRoot) + sizeof(BhInfo) + 2 * sizeof(int) +
+                               sizeof(double) * (4 * kBhMaxDims + (size_t)eblk * 3 * D)));
+    auto *root = c->bh_root.as<BhRoot>(), *exact = root + 1;
+    auto *rcom = reinterpret_cast<double *>(exact + 1), *mean = rcom + kBhMaxDims, *ext = mean + kBhMaxDims;
+    double *part = ext + 2 * kBhMaxDims;
+    auto *info = reinterpret_cast<BhInfo *>(part + (size_t)eblk * 3 * D);
+    int *differs = reinterpret_cast<int *>(info + 1);
+    TRY(ensure(c->bh_key, 3 * n64));
+    TRY(ensure(c->bh_idx, 2 * n32));
+    TRY(ensure(c->bh_pos, 3 * n32 + (size_t)N));  // lcp, counts, offsets; lost levels
+    uint64_t *key = c->bh_key.as<uint64_t>(), *skey = key + N, *key2 = skey + N;
+    uint32_t *idx = c->bh_idx.as<uint32_t>(), *sidx = idx + N + 1;
+    int *lcp = c->bh_pos.as<int>(), *cnt = lcp + N + 1, *off = cnt + N + 1;
+    auto *lost = reinterpret_cast<unsigned char *>(off + N + 1);
+    constexpr unsigned bits = D * kBhLevels<D>;
+    size_t t1 = 0, t2 = 0;
+    HIPTRY(rocprim::radix_sort_pairs(nullptr, t1, key, skey, idx, sidx, (size_t)N, 0u, bits, c->stream));
+    HIPTRY(rocprim::exclusive_scan(nullptr, t2, cnt, off, 0, (size_t)N + 1, rocprim::plus<int>(), c->stream));
+    TRY(ensure(c->bh_tmp, std::max<size_t>(std::max(t1, t2), 16)));
+    struct Back {
+        BhInfo info;
+        int nodes, differs;
+    };
+    TRY(bh_pinned(c, sizeof(Back)));
+    auto *h = static_cast<volatile Back *>(c->bh_pin);
+    // a side stream's launches, behind the work queued so far
+    hipStream_t main = c->stream;
+    struct Restore {
+        fitsne_ctx *c;
+        hipStream_t s;
+        ~Restore() { c->stream = s; }
+    } restore{c, main};
+    HIPTRY(hipEventRecord(c->fork_ev, main));
+    HIPTRY(hipStreamWaitEvent(c->astream, c->fork_ev, 0));
+    HIPTRY(hipStreamWaitEvent(c->kstream, c->fork_ev, 0));
+    c->stream = c->astream;
+    launch(c, "bh_com_root", k_bh_com_root<D>, dim3(1), dim3(kWave), 0, Y, N, c->bh_ab.as<const double2>(), rcom);
+    HIPTRY(hipEventRecord(c->join_ev, c->astream));
+    c->stream = c->kstream;
+    launch(c, "bh_clear", k_bh_clear, dim3(1), dim3(1), 0, differs);
+    launch(c, "bh_mean", k_bh_mean<D>, dim3(1), dim3(256), 0, Y, N, mean);
+    c->stream = main;
+    launch(c, "bh_extent", k_bh_extent<D>, dim3(eblk), dim3(kThreads), 0, Y, N, part);
+    launch(c, "bh_approx_root", k_bh_approx_root<D>, dim3(1), dim3(kWave), 0, (const double *)part, eblk, N, root, ext,
+           info);
+    launch(c, "bh_keys", k_bh_keys<D>, dim3(blocks_for(N)), dim3(kThreads), 0, Y, N, (const BhRoot *)root, key, idx,
+           lost, info);
+    HIPTRY(rocprim::radix_sort_pairs(c->bh_tmp.p, t1, key, skey, idx, sidx, (size_t)N, 0u, bits, main));
+    launch(c, "bh_ties", k_bh_ties<D>, dim3(blocks_for(N)), dim3(kThreads), 0, Y, N, (const BhRoot *)root,
+           (const uint64_t *)skey, sidx, key2, lost, info);
+    launch(c, "bh_count", k_bh_count<D>, dim3(blocks_for((long)N + 1)), dim3(kThreads), 0, (const uint64_t *)skey,
+           (const uint64_t *)key2, (const uint32_t *)sidx, (const unsigned char *)lost, N, lcp, cnt, info);
+    // the check on the side stream, once the leaves' depths are there
+    HIPTRY(hipEventRecord(c->kl_go, main));
+    HIPTRY(hipStreamWaitEvent(c->kstream, c->kl_go, 0));
+    c->stream = c->kstream;
+    launch(c, "bh_check", k_bh_check<D>, dim3(blocks_for(N)), dim3(kThreads), 0, Y, N, (const double *)mean,
+           (const double *)ext, (const uint64_t *)skey, (const uint64_t *)key2, (const uint32_t *)sidx, (const int *)lcp,
+           exact, differs);
+    HIPTRY(hipMemcpyAsync((void *)&h->differs, differs, sizeof(int), hipMemcpyDeviceToHost, c->kstream));
+    HIPTRY(hipEventRecord(c->bh_ev, c->kstream));
+    const int rc = beside();
+    HIPTRY(hipEventRecord(c->kl_ev, c->kstream));
+    TRY(rc);
+    c->stream = main;
+    HIPTRY(rocprim::exclusive_scan(c->bh_tmp.p, t2, cnt, off, 0, (size_t)N + 1, rocprim::plus<int>(), main));
+    HIPTRY(hipMemcpyAsync((void *)&h->info, info, sizeof(BhInfo), hipMemcpyDeviceToHost, main));
+    HIPTRY(hipMemcpyAsync((void *)&h->nodes, off + N, sizeof(int), hipMemcpyDeviceToHost, main));
+    HIPTRY(hipGetLastError());
+    HIPTRY(hipStreamSynchronize(main));
+    const int nodes = h->nodes, deepest = h->info.deepest;
+    bool ok = !h->info.bad && nodes >= 1 && deepest < 2 * kBhLevels<D>;
+    if (ok) {
+        TRY(ensure(c->bh_cell, sizeof(BhCell<D>) * (size_t)nodes));
+        TRY(ensure(c->bh_leafpt, sizeof(int) * (size_t)nodes));
+        TRY(ensure(c->bh_span, sizeof(BhSpan) * (size_t)nodes));
+        TRY(ensure(c->bh_list, sizeof(int) * ((size_t)nodes * 2 + N)));
+        TRY(ensure(c->bh_order, sizeof(uint32_t) * (size_t)N * std::max(deepest, 1)));
+        auto *span = c->bh_span.as<BhSpan>();
+        auto *cell = bh_cells<D>(c);
+        int *huge = c->bh_list.as<int>(), *big = huge + nodes, *at = big + nodes;
+        auto *order = c->bh_order.as<uint32_t>();
+        launch(c, "bh_nodes", k_bh_nodes<D>, dim3(blocks_for(N)), dim3(kThreads), 0, (const uint64_t *)skey,
+               (const uint32_t *)sidx, (const int *)lcp, (const int *)off, Y, N, span, cell, c->bh_leafpt.as<int>(),
+               at, huge, big, info);
+        const uint32_t *in = sidx;
+        for (int d = deepest; d >= 1; d--) {
+            uint32_t *out = order + (size_t)(d - 1) * N;
+            launch(c, "bh_merge", k_bh_merge<D>, dim3(blocks_for(N)), dim3(kThreads), 0, (const BhSpan *)span,
+                   (const BhCell<D> *)cell, N, d, in, out, at);
+            in = out;
+        }
+        launch(c, "bh_com_long", k_bh_com_long<D>, dim3(2048), dim3(kWave), 0, (const int *)huge, (const int *)big,
+               (const BhInfo *)info, (const BhSpan *)span, (const uint32_t *)order, (long)N, Y,
+               c->bh_ab.as<const double2>(), cell);
+        launch(c, "bh_com_small", k_bh_com_small<D>, dim3(blocks_for(nodes)), dim3(kThreads), 0,
+               (const BhSpan *)span, nodes, (const uint32_t *)order, (long)N, Y, c->bh_ab.as<const double2>(), cell);
+        HIPTRY(hipEventSynchronize(c->bh_ev));  // the check's answer
+        ok = !h->differs;
+    }
+    HIPTRY(hipStreamWaitEvent(main, c->join_ev, 0));
+    HIPTRY(hipStreamWaitEvent(main, c->kl_ev, 0));
+    if (!ok) return bh_tree_on_host<D>(c);
+    launch(c, "bh_finish", k_bh_finish<D>, dim3(blocks_for(nodes)), dim3(kThreads), 0, c->bh_span.as<const BhSpan>(),
+           nodes, (const BhRoot *)exact, (const double *)rcom, bh_cells<D>(c));
+    HIPTRY(hipGetLastError());
+    c->bh_sorted = true;
     return FITSNE_OK;
 }
 
@@ -1418,11 +1558,10 @@ static int bh_walk(fitsne_ctx *c, bool forces) {
     const int N = c->N;
     TRY(ensure(c->bh_Q, sizeof(double) * (size_t)N));
     if (forces) TRY(ensure(c->bh_neg, sizeof(double) * (size_t)N * D));
-    const BhFlatView v(c->bh_tree_d.p, c->bh_nodes, D);
-    launch(c, "bh_nonedge", k_bh_nonedge<D>, dim3(blocks_for(N)), dim3(kThreads), 0, c->Y.as<const double>(), N,
-           (const double *)v.com, (const double *)v.maxw, (const unsigned *)v.cum, (const int *)v.leafpt,
-           (const int *)v.isleaf, (const int *)v.skip, c->theta, forces ? c->bh_neg.as<double>() : (double *)nullptr,
-           c->bh_Q.as<double>());
+    launch(c, "bh_nonedge", k_bh_nonedge<D>, dim3((N + kWave - 1) / kWave), dim3(kWave), 0, c->Y.as<const double>(),
+           N, (const BhCell<D> *)bh_cells<D>(c), c->bh_leafpt.as<const int>(),
+           c->bh_sorted ? c->bh_idx.as<const uint32_t>() + N + 1 : (const uint32_t *)nullptr, c->theta,
+           forces ? c->bh_neg.as<double>() : (double *)nullptr, c->bh_Q.as<double>());
     return FITSNE_OK;
 }
 
@@ -1431,12 +1570,15 @@ template <int D>
 static int pipeline_bh(fitsne_ctx *c, int mode, const fitsne_step_params *sp) {
     const int N = c->N;
     const long nd = (long)N * D;
-    TRY(bh_tree_of_Y<D>(c));
     TRY(ensure(c->pos, sizeof(double) * (size_t)nd));
     TRY(ensure(c->dC, sizeof(double) * (size_t)nd));
     TRY(ensure(c->zbuf, sizeof(double) * 4));
-    launch(c, "bh_edge", k_bh_edge<D>, dim3(blocks_for(N)), dim3(kThreads), 0, c->rowP.as<const int64_t>(),
-           c->colP.as<const uint32_t>(), c->val.as<const double>(), c->Y.as<const double>(), N, c->pos.as<double>());
+    TRY(bh_tree_of_Y<D>(c, [&]() {
+        launch(c, "bh_edge", k_bh_edge<D>, dim3(blocks_for(N)), dim3(kThreads), 0, c->rowP.as<const int64_t>(),
+               c->colP.as<const uint32_t>(), c->val.as<const double>(), c->Y.as<const double>(), N,
+               c->pos.as<double>());
+        return FITSNE_OK;
+    }));
     TRY(bh_walk<D>(c, true));
     launch(c, "bh_sumq", k_seq_sum, dim3(1), dim3(1024), 0, c->bh_Q.as<const double>(), N, c->zbuf.as<double>());
     launch(c, "bh_combine", k_bh_combine, dim3(std::min(blocks_for(nd), 4096)), dim3(kThreads), 0,
@@ -1468,7 +1610,7 @@ static int pipeline_bh(fitsne_ctx *c, int mode, const fitsne_step_params *sp) {
 template <int D>
 static int kl_bh_d(fitsne_ctx *c) {
     const int N = c->N;
-    TRY(bh_tree_of_Y<D>(c));
+    TRY(bh_tree_of_Y<D>(c, []() { return FITSNE_OK; }));
     TRY(bh_walk<D>(c, false));
     TRY(ensure(c->mean, sizeof(double) * kExMaxDims));
     launch(c, "bh_sumq", k_seq_sum, dim3(1), dim3(1024), 0, c->bh_Q.as<const double>(), N, c->mean.as<double>() + 2);
@@ -1608,7 +1750,8 @@ extern "C" int fitsne_ctx_destroy(fitsne_ctx *c) {
                    &c->inv_d, &c->colP2, &c->val2, &c->tmp, &c->fixgrid, &c->att, &c->rep, &c->zrow,
                    &c->sy_row, &c->sy_col, &c->sy_val, &c->sy_erow, &c->sy_keys, &c->sy_keys2, &c->sy_vals,
                    &c->sy_vals2, &c->sy_partner, &c->sy_cnt, &c->sy_start, &c->sy_okeys, &c->sy_okeys2, &c->sy_tmp,
-                   &c->sy_scol, &c->sy_sval, &c->bh_tree_d, &c->bh_neg, &c->bh_Q, &c->kline};
+                   &c->sy_scol, &c->sy_sval, &c->bh_cell, &c->bh_leafpt, &c->bh_neg, &c->bh_Q, &c->bh_root, &c->bh_key,
+                   &c->bh_idx, &c->bh_pos, &c->bh_span, &c->bh_list, &c->bh_order, &c->bh_tmp, &c->bh_ab, &c->kline};
     for (DBuf *b : all) release(*b);
     for (auto &kv : c->tw32) release(kv.second);
     for (auto &kv : c->tw64) release(kv.second);
@@ -1624,6 +1767,7 @@ extern "C" int fitsne_ctx_destroy(fitsne_ctx *c) {
     if (c->kern_ev) (void)hipEventDestroy(c->kern_ev);
     if (c->kl_go) (void)hipEventDestroy(c->kl_go);
     if (c->kl_ev) (void)hipEventDestroy(c->kl_ev);
+    if (c->bh_ev) (void)hipEventDestroy(c->bh_ev);
     if (c->astream) (void)hipStreamDestroy(c->astream);
     if (c->kstream) (void)hipStreamDestroy(c->kstream);
     if (c->h_mm) (void)hipHostFree(c->h_mm);
