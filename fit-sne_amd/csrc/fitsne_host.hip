@@ -162,7 +162,8 @@ struct fitsne_ctx {
     bool tw_fresh = false;  // a twiddle table was written on the stream since the last step's stages
     bool graph_ran = false;      // a captured step ran since the last error check
     // plain path extras
-    DBuf xs, ys, box, wx, wy, ch, w, V, potA, potB;
+    DBuf xs, ys, box, wx, wy, ch, w, V, potA;
+    DBuf bcount, bstart;  // points per box (zero between steps); places taken, then each box's first place in the list
     // exact path (dense P in val): per-row attractive / repulsive sums and Z shares
     DBuf att, rep, zrow;
     // Barnes-Hut: theta, the host tree and the tree of the current Y on the device (pre-order)
@@ -303,10 +304,17 @@ static int bits_for(unsigned long long v) {
     return b;
 }
 
-// lanes per CSR row: each lane carries 4 entries per pass, so 32 lanes cover 128 entries at once
+// lanes per CSR row of the KL kernel
 static int sw_for(long long nnz, int N) {
     const double avg = N > 0 ? (double)nnz / N : 0;
     return avg >= 64 ? 32 : 16;
+}
+
+// lanes per CSR row of the attractive kernel: each lane carries 8 entries per pass, so 16 lanes cover 128 entries
+// at once and 8 lanes 64.  (Rows of 84 entries: 16 lanes 99 us, 8 lanes 106; of 30: 53 and 42; N = 200,003.)
+static int att_lanes(long long nnz, int N) {
+    const double avg = N > 0 ? (double)nnz / N : 0;
+    return avg >= 64 ? 16 : 8;
 }
 
 // ---------------------------------------------------------------- min / max of the resident Y
@@ -522,6 +530,25 @@ static auto pick_interp_f64(int p) -> decltype(&k_interp_f64<3, D>) {
     }
 }
 
+template <int D>
+static auto pick_spread_box(int p) -> decltype(&k_spread_box_f64<3, D>) {
+    switch (p) {
+    case 2: return k_spread_box_f64<2, D>;
+    case 3: return k_spread_box_f64<3, D>;
+    case 4: return k_spread_box_f64<4, D>;
+    default: return k_spread_box_f64<5, D>;
+    }
+}
+template <int D, int NT>
+static auto pick_interp_box(int p) -> decltype(&k_interp_box_f64<3, D, NT>) {
+    switch (p) {
+    case 2: return k_interp_box_f64<2, D, NT>;
+    case 3: return k_interp_box_f64<3, D, NT>;
+    case 4: return k_interp_box_f64<4, D, NT>;
+    default: return k_interp_box_f64<5, D, NT>;
+    }
+}
+
 // Row blocks of about equal cost for the windowed attractive kernel (att_rows == kAttBalanced).  One
 // workgroup per CU holds a block, all start together, and the kernel lasts as long as its slowest block,
 // so the blocks are cut by a cost model instead of a row count: per block, a time per quad of entries,
@@ -704,7 +731,7 @@ static int launch_attractive(fitsne_ctx *c, TV scale, TV *pos, const DevGeo *dg 
             return FITSNE_OK;
         }
     }
-    const int sw = sw_for(c->nnz, c->N);
+    const int sw = att_lanes(c->nnz, c->N);
     const int rpb = kThreads / sw;
     const int nblk = (c->N + rpb - 1) / rpb;
     dim3 grid(8 * ((nblk + 7) / 8));
@@ -712,11 +739,11 @@ static int launch_attractive(fitsne_ctx *c, TV scale, TV *pos, const DevGeo *dg 
     auto cp = c->colP.as<const uint32_t>();
     auto vp = c->val.as<const TV>();
     auto yp = c->Y.as<const TV>();
-    if (sw == 32)
-        launch(c, "attractive", k_attractive<TV, int64_t, uint32_t, D, 32>, grid, dim3(kThreads), 0, rp, cp, vp, yp,
+    if (sw == 16)
+        launch(c, "attractive", k_attractive<TV, int64_t, uint32_t, D, 16>, grid, dim3(kThreads), 0, rp, cp, vp, yp,
                c->N, inv_df, df1, scale, pos);
     else
-        launch(c, "attractive", k_attractive<TV, int64_t, uint32_t, D, 16>, grid, dim3(kThreads), 0, rp, cp, vp, yp,
+        launch(c, "attractive", k_attractive<TV, int64_t, uint32_t, D, 8>, grid, dim3(kThreads), 0, rp, cp, vp, yp,
                c->N, inv_df, df1, scale, pos);
     return FITSNE_OK;
 }
@@ -1155,23 +1182,11 @@ static int tune_attractive(fitsne_ctx *c) {
 
 // ============================================================================ FP64 plain pipeline
 
-// One convolution pass of the plain path: charges `set` (nt terms) spread, convolved with kernel
-// spectrum KC (2D) or kernel kind (1D), interpolated into pot[N][nt] (zeroed first).
+// One convolution of the plain path: the grid's terms w[node][sin], nt of them, with kernel spectrum KC (2D)
+// or kernel kind (1D), into V[node][nt].  wait: an event to wait for before KC is read (nullable).
 template <int D>
-static int plain_pass(fitsne_ctx *c, const Geo &g, const cx<double> *tw, int set, int nt,
-                      const double *KC, int kind1d, int use_k1, DBuf &pot) {
-    const int N = c->N;
-    const long nodes = D == 2 ? (long)g.n1d * g.n1d : g.n1d;
-    TRY(ensure(c->ch, sizeof(double) * (size_t)N * nt));
-    TRY(ensure(c->w, sizeof(double) * nodes * nt));
-    TRY(ensure(c->V, sizeof(double) * nodes * nt));
-    TRY(ensure(pot, sizeof(double) * (size_t)N * nt));
-    launch(c, "charges", k_charges<D>, dim3(blocks_for(N)), dim3(kThreads), 0, c->Y.as<const double>(), N, set,
-           c->ch.as<double>());
-    launch(c, "fill", k_fill<double>, dim3(std::min(blocks_for(nodes * nt), 2048)), dim3(kThreads), 0,
-           c->w.as<double>(), nodes * nt, 0.0);
-    launch(c, "spread_f64", pick_spread_f64<D>(c->p), dim3(blocks_for(N)), dim3(kThreads), 0, c->box.as<const int>(),
-           c->wx.as<const double>(), c->wy.as<const double>(), c->ch.as<const double>(), nt, N, g, c->w.as<double>());
+static int plain_conv(fitsne_ctx *c, const Geo &g, const cx<double> *tw, const double *w, int sin, int nt,
+                      const double *KC, int kind1d, int use_k1, hipEvent_t wait, double *V) {
     if constexpr (D == 2) {
         const size_t plane = (size_t)g.H * g.n1d;
         TRY(ensure(c->spec, sizeof(cx<double>) * plane * nt));
@@ -1179,33 +1194,52 @@ static int plain_pass(fitsne_ctx *c, const Geo &g, const cx<double> *tw, int set
         const int gr_rows = 8 * ((g.n1d + 7) / 8), gr_cols = 8 * ((g.H + 7) / 8);
         const int lines = (nt + 1) / 2;
         launch(c, "rows_fwd64", k_rows_fwd<double, kRowThreads, kRowTot>, dim3(gr_rows), dim3(kRowThreads),
-               sizeof(cx<double>) * (lines + 1) * g.Mp, c->dgeo.as<const DevGeo>(), tw, c->w.as<const double>(), nt, nt,
+               sizeof(cx<double>) * (lines + 1) * g.Mp, c->dgeo.as<const DevGeo>(), tw, w, sin, nt,
                c->spec.as<cx<double>>(), (unsigned long long *)nullptr);
+        if (wait) HIPTRY(hipStreamWaitEvent(c->stream, wait, 0));
         const int cl = std::min(nt, kColTot64 / g.Mp);
         launch(c, "cols_plain64", k_cols_plain<double, kColThreads64, kColTot64>, dim3(gr_cols), dim3(kColThreads64),
                sizeof(cx<double>) * (cl + 1) * g.Mp, c->dgeo.as<const DevGeo>(), tw, c->spec.as<const cx<double>>(), nt, KC,
                c->ospec.as<cx<double>>());
         launch(c, "rows_inv64", k_rows_inv<double, kRowThreads, kRowTot>, dim3(gr_rows), dim3(kRowThreads),
                sizeof(cx<double>) * (lines + 1) * g.Mp, c->dgeo.as<const DevGeo>(), tw, c->ospec.as<const cx<double>>(), nt,
-               c->V.as<double>(), nt, (const double *)nullptr, 0, 0.0, (double *)nullptr);
+               V, nt, (const double *)nullptr, 0, 0.0, (double *)nullptr);
     } else {
         launch(c, "conv1d_f64", k_conv1d<double, kConv1dThreads, kMaxTot64>, dim3(1), dim3(kConv1dThreads),
-               sizeof(cx<double>) * g.Mp, c->dgeo.as<const DevGeo>(), tw, kind1d, kind1d, c->df, 0, c->w.as<const double>(), nt, nt, use_k1,
-               c->V.as<double>(), nt, (double *)nullptr, (const double *)nullptr, (const double *)nullptr);
+               sizeof(cx<double>) * g.Mp, c->dgeo.as<const DevGeo>(), tw, kind1d, kind1d, c->df, 0, w, sin, nt, use_k1,
+               V, nt, (double *)nullptr, (const double *)nullptr, (const double *)nullptr);
     }
-    launch(c, "fill", k_fill<double>, dim3(std::min(blocks_for((long)N * nt), 2048)), dim3(kThreads), 0,
-           pot.as<double>(), (long)N * nt, 0.0);
-    launch(c, "interp_f64", pick_interp_f64<D>(c->p), dim3(blocks_for(N)), dim3(kThreads), 0, c->box.as<const int>(),
-           c->wx.as<const double>(), c->wy.as<const double>(), c->V.as<const double>(), nt, N, g, pot.as<double>());
     return FITSNE_OK;
 }
 
+// The attractive term runs on the second stream beside the grid stages, the 2D kernel spectra on the third (unless
+// overlap is off).  It starts before the host has the last step's bounds, which the grid stages wait for.  (N =
+// 200,003, 84 entries per row: 346 us per step with the reading of Y, 396 with the term behind the bounds and
+// the spectra, 1644 one stage after the other with an atomic per point, node and term.)
 template <int D>
 static int pipeline_f64(fitsne_ctx *c, int mode, const fitsne_step_params *sp) {
     const int N = c->N, p = c->p;
     const bool df1 = c->df == 1.0;
     TRY(ensure(c->pos, sizeof(double) * (size_t)N * D));
+    const hipStream_t main = c->stream;
+    struct Restore {
+        fitsne_ctx *c;
+        hipStream_t s;
+        ~Restore() { c->stream = s; }
+    } restore{c, main};
+    const bool side = c->overlap;
+    if (side) {
+        if (!c->astream) HIPTRY(hipStreamCreateWithFlags(&c->astream, hipStreamNonBlocking));
+        if (D == 2 && !c->kstream) HIPTRY(hipStreamCreateWithFlags(&c->kstream, hipStreamNonBlocking));
+        HIPTRY(hipEventRecord(c->fork_ev, main));
+        HIPTRY(hipStreamWaitEvent(c->astream, c->fork_ev, 0));
+        c->stream = c->astream;
+    }
     TRY((launch_attractive<double, D>(c, 1.0, c->pos.as<double>())));
+    if (side) {
+        HIPTRY(hipEventRecord(c->join_ev, c->astream));
+        c->stream = main;
+    }
     double mn, mx;
     TRY(current_minmax<double>(c, &mn, &mx));
     Geo g;
@@ -1214,23 +1248,14 @@ static int pipeline_f64(fitsne_ctx *c, int mode, const fitsne_step_params *sp) {
     TRY(twiddles<double>(c, g.Mp, &tw));
     TRY(put_geo(c, g, true));
 
-    const double *xs = c->Y.as<const double>(), *ys = nullptr;
-    if constexpr (D == 2) {
-        TRY(ensure(c->xs, sizeof(double) * (size_t)N));
-        TRY(ensure(c->ys, sizeof(double) * (size_t)N));
-        launch(c, "split", k_split_f64, dim3(blocks_for(N)), dim3(kThreads), 0, c->Y.as<const double>(), N,
-               c->xs.as<double>(), c->ys.as<double>());
-        xs = c->xs.as<const double>();
-        ys = c->ys.as<const double>();
-    }
-    TRY(ensure(c->box, sizeof(int) * (size_t)N));
-    TRY(ensure(c->wx, sizeof(double) * (size_t)N * p));
-    TRY(ensure(c->wy, sizeof(double) * (size_t)N * p));
-    launch(c, "weights_f64", pick_weights<D>(p), dim3(blocks_for(N)), dim3(kThreads), 0, xs, ys, N, g,
-           (const double *)nullptr, (const double *)nullptr, c->box.as<int>(), c->wx.as<double>(), c->wy.as<double>());
-
     const int kind_q = df1 ? FITSNE_KERNEL_SQUARED_CAUCHY : FITSNE_KERNEL_SQUARED_GENERAL;
     const double *KQ = nullptr, *K1 = nullptr;
+    hipEvent_t wait = nullptr;
+    if (side && D == 2) {  // behind the geometry record, the twiddles and the last step
+        HIPTRY(hipEventRecord(c->geo_ev, main));
+        HIPTRY(hipStreamWaitEvent(c->kstream, c->geo_ev, 0));
+        c->stream = c->kstream;
+    }
     if constexpr (D == 2) {
         const size_t HH = (size_t)g.H * g.H;
         TRY(ensure(c->Trow, sizeof(cx<double>) * (size_t)g.H * g.n1d));
@@ -1243,38 +1268,72 @@ static int pipeline_f64(fitsne_ctx *c, int mode, const fitsne_step_params *sp) {
         launch(c, "kern_cols64", k_kern_cols<double, kKernThreads, kKernTot>, dim3(gr_cols), dim3(kKernThreads),
                sizeof(cx<double>) * (1 + 1) * g.Mp, c->dgeo.as<const DevGeo>(), tw, c->Trow.as<const cx<double>>(), 0, c->KQ.as<double>(),
                c->K1.as<double>(), (double *)nullptr, (double *)nullptr);
+        if (side) {
+            HIPTRY(hipEventRecord(c->kern_ev, c->kstream));
+            wait = c->kern_ev;
+        }
         KQ = c->KQ.as<const double>();
         K1 = c->K1.as<const double>();
     }
-    int zform, cform;
-    DBuf *potF = &c->potA;
-    if (df1) {
-        TRY((plain_pass<D>(c, g, tw, D == 2 ? 0 : 3, D == 2 ? 4 : 3, KQ, kind_q, 0, c->potA)));
-        zform = D == 2 ? 0 : 2;
-        cform = D == 2 ? 0 : 2;
-        potF = &c->potA;
-    } else {
-        TRY((plain_pass<D>(c, g, tw, D == 2 ? 1 : 4, D == 2 ? 3 : 2, KQ, kind_q, 0, c->potA)));
-        TRY((plain_pass<D>(c, g, tw, 2, 1, K1, FITSNE_KERNEL_GENERAL, 1, c->potB)));
-        zform = 1;
-        cform = D == 2 ? 1 : 3;
-        potF = &c->potA;
+    c->stream = main;
+    // points in box order
+    TRY(ensure(c->box, sizeof(int) * 3 * (size_t)N));
+    int *box = c->box.as<int>(), *rank = box + N, *order = rank + N;
+    const int nbox = g.nbox;
+    if (c->bcount.cap < sizeof(int) * (size_t)nbox) {  // zero between steps (the scan clears it)
+        release(c->bcount);
+        TRY(ensure(c->bcount, sizeof(int) * (size_t)nbox));
+        const long n = (long)(c->bcount.cap / sizeof(int));
+        launch(c, "fill", k_fill<int>, dim3(std::min(blocks_for(n), 2048)), dim3(kThreads), 0, c->bcount.as<int>(), n, 0);
     }
+    // df == 1: one set of charges gives Z and the forces; else [.., 1] gives the forces, and its last term,
+    // convolved with the general kernel, Z
+    const int set = df1 ? (D == 2 ? 0 : 3) : (D == 2 ? 1 : 4), nt = charge_terms(set);
+    const long nodes = D == 2 ? (long)g.n1d * g.n1d : g.n1d;
     const int nblk = blocks_for(N);
+    TRY(ensure(c->w, sizeof(double) * nodes * nt));
+    TRY(ensure(c->V, sizeof(double) * nodes * nt));
+    TRY(ensure(c->potA, sizeof(double) * (size_t)N * nt));
     TRY(ensure(c->part, sizeof(double) * (size_t)nblk * 2));
     TRY(ensure(c->zbuf, sizeof(double) * 4));
-    launch(c, "zterms64", k_zterms_f64, dim3(nblk), dim3(kThreads), 0, c->Y.as<const double>(),
-           (df1 ? c->potA : c->potB).as<const double>(), N, D, zform, c->part.as<double>());
-    launch(c, "zsum64", k_sum_final, dim3(1), dim3(kThreads), 0, c->part.as<const double>(), nblk, (double)N,
-           c->zbuf.as<double>());
     TRY(ensure(c->dC, sizeof(double) * (size_t)N * D));
-    launch(c, "combine64", k_combine_f64, dim3(nblk), dim3(kThreads), 0, c->Y.as<const double>(),
-           c->pos.as<const double>(), potF->as<const double>(), c->zbuf.as<const double>(), N, cform,
-           c->dC.as<double>());
-    if (mode == 1) {
-        launch(c, "update64", k_update_f64, dim3(nblk), dim3(kThreads), 0, c->Y.as<double>(), c->uY.as<double>(),
-               c->gains.as<double>(), c->dC.as<const double>(), N, D, sp->momentum, sp->learning_rate,
-               sp->max_step_norm, sp->plain_descent, c->part.as<double>());
+    double *w = c->w.as<double>(), *V = c->V.as<double>(), *pot = c->potA.as<double>(), *part = c->part.as<double>();
+    TRY(ensure(c->bstart, sizeof(int) * ((size_t)nbox + 1)));
+    int *used = c->bstart.as<int>(), *start = used + 1;
+    const double *Y = c->Y.as<const double>();
+    launch(c, "box64", k_box_f64<D>, dim3(nblk), dim3(kThreads), 0, Y, N, g, box, rank, c->bcount.as<int>(), used, w,
+           nodes * nt);
+    launch(c, "box_starts", k_box_starts, dim3(blocks_for(nbox)), dim3(kThreads), 0, c->bcount.as<int>(), nbox, used,
+           start);
+    launch(c, "box_order", k_box_order, dim3(nblk), dim3(kThreads), 0, (const int *)box, (const int *)rank,
+           (const int *)start, N, order);
+    launch(c, "spread64", pick_spread_box<D>(p), dim3(nblk), dim3(kThreads), 0, Y, (const int *)order, N, g, set, w);
+    TRY((plain_conv<D>(c, g, tw, w, nt, nt, KQ, kind_q, 0, wait, V)));
+    auto interp = [&](auto NT, int zform, double *out) {
+        launch(c, "interp64", pick_interp_box<D, decltype(NT)::value>(p), dim3(nblk), dim3(kThreads), 0, Y,
+               (const int *)order, N, g, (const double *)V, zform, out, part);
+    };
+    if (df1) {
+        if constexpr (D == 2) interp(std::integral_constant<int, 4>{}, 0, pot);
+        else interp(std::integral_constant<int, 3>{}, 2, pot);
+    } else {
+        if constexpr (D == 2) interp(std::integral_constant<int, 3>{}, -1, pot);
+        else interp(std::integral_constant<int, 2>{}, -1, pot);
+        TRY((plain_conv<D>(c, g, tw, w + (nt - 1), nt, 1, K1, FITSNE_KERNEL_GENERAL, 1, nullptr, V)));
+        interp(std::integral_constant<int, 1>{}, 1, (double *)nullptr);
+    }
+    const int cform = (D == 2 ? 0 : 2) + (df1 ? 0 : 1);
+    launch(c, "zsum64", k_sum_final, dim3(1), dim3(kThreads), 0, (const double *)part, nblk, (double)N,
+           c->zbuf.as<double>());
+    if (side) HIPTRY(hipStreamWaitEvent(main, c->join_ev, 0));
+    if (mode == 0) {
+        launch(c, "combine64", k_combine_f64, dim3(nblk), dim3(kThreads), 0, Y, c->pos.as<const double>(),
+               (const double *)pot, c->zbuf.as<const double>(), N, cform, c->dC.as<double>());
+    } else {
+        launch(c, "update64", k_combine_update_f64<D>, dim3(nblk), dim3(kThreads), 0, c->Y.as<double>(),
+               c->pos.as<const double>(), (const double *)pot, c->zbuf.as<const double>(), N, cform, c->dC.as<double>(),
+               c->uY.as<double>(), c->gains.as<double>(), sp->momentum, sp->learning_rate, sp->max_step_norm,
+               sp->plain_descent, part);
         TRY(ensure(c->mean, sizeof(double) * 2));
         const long n = (long)N * D;
         const int cblk = part_blocks(n);
@@ -1746,7 +1805,7 @@ extern "C" int fitsne_ctx_destroy(fitsne_ctx *c) {
                    &c->wkey, &c->wval, &c->wbmax, &c->wrstart, &c->knnX, &c->knnXT, &c->knnI, &c->knnD, &c->dgeo,
                    &c->dstep, &c->dtw, &c->dlive, &c->klpart, &c->gin, &c->gout, &c->spec, &c->ospec, &c->Trow, &c->KQ,
                    &c->K1, &c->KS, &c->KT, &c->zpart, &c->zbuf, &c->part, &c->mean, &c->mmpart, &c->mm, &c->mmu, &c->xs,
-                   &c->ys, &c->box, &c->wx, &c->wy, &c->ch, &c->w, &c->V, &c->potA, &c->potB,
+                   &c->ys, &c->box, &c->wx, &c->wy, &c->ch, &c->w, &c->V, &c->potA, &c->bcount, &c->bstart,
                    &c->inv_d, &c->colP2, &c->val2, &c->tmp, &c->fixgrid, &c->att, &c->rep, &c->zrow,
                    &c->sy_row, &c->sy_col, &c->sy_val, &c->sy_erow, &c->sy_keys, &c->sy_keys2, &c->sy_vals,
                    &c->sy_vals2, &c->sy_partner, &c->sy_cnt, &c->sy_start, &c->sy_okeys, &c->sy_okeys2, &c->sy_tmp,

@@ -83,13 +83,16 @@ __global__ void k_twiddles(cx<T> *tw, int n) {
 // pos_i = scale * sum_j p_ij q_ij (y_i - y_j), q_ij = 1 / (1 + |y_i - y_j|^2 / df)
 // (tsne.cpp:1121-1137, :965-980, :826-837, :721-732).  SW lanes per CSR row; each lane issues U
 // independent (column, value) loads before its U neighbour gathers, so a wave keeps U times more
-// memory requests in flight.  Column indices and values are streamed once (non-temporal loads).
+// memory requests in flight.  Bound: one L2 request per gathered neighbour.  Few lanes with U = 8 (no group
+// sum over 32 lanes, fewer idle slots) and loads that may stay in the cache between steps: FP64, 2D,
+// N = 200,003, random columns, 84 entries per row: 32 lanes with U = 4, streamed non-temporally, 137 us, this
+// 99 (columns near the row: 125 and 79); 300 per row 462 and 403; 30 per row (16 lanes before, 8 now) 56 and 42.
 template <typename TV, typename TI, typename TC, int D, int SW>
 __global__ __launch_bounds__(kThreads) void k_attractive(const TI *__restrict__ rowP, const TC *__restrict__ colP,
                                                          const TV *__restrict__ valP, const TV *__restrict__ Y,
                                                          int N, TV inv_df, int df_one, TV scale,
                                                          TV *__restrict__ pos) {
-    constexpr int U = 4;
+    constexpr int U = 8;
     // blocks of consecutive rows go to the same XCD, so each XCD's L2 holds the Y rows its
     // neighbours gather (the points are kept in spatial order)
     constexpr int RPB = kThreads / SW;
@@ -109,9 +112,10 @@ __global__ __launch_bounds__(kThreads) void k_attractive(const TI *__restrict__ 
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const long k = k0 + (long)u * SW;
-            const bool ok = k < end;
-            j[u] = ok ? (long)__builtin_nontemporal_load(&colP[k]) : row;  // row itself contributes 0
-            v[u] = ok ? __builtin_nontemporal_load(&valP[k]) : (TV)0;
+            const long kk = k < end ? k : end - 1;  // past the end: the last entry again, with p = 0
+            j[u] = (long)colP[kk];
+            v[u] = valP[kk];
+            v[u] = k < end ? v[u] : (TV)0;
         }
         TV yj[U][D];
 #pragma unroll
@@ -2315,24 +2319,6 @@ __global__ void k_fill(T *__restrict__ p, long n, T v) {
     for (long e = (long)blockIdx.x * kThreads + threadIdx.x; e < n; e += (long)gridDim.x * kThreads) p[e] = v;
 }
 
-// Charges of the reference (tsne.cpp:1057-1062, :904-908, :939-941, :786-790, :674-677, :689-691).
-// set: 0 = [1, x, y, x^2+y^2] (2D df=1), 1 = [x, y, 1] (2D df), 2 = [1] (general kernel),
-//      3 = [1, y, y^2] (1D df=1), 4 = [y, 1] (1D df).
-template <int D>
-__global__ __launch_bounds__(kThreads) void k_charges(const double *__restrict__ Y, int N, int set,
-                                                      double *__restrict__ ch) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= N) return;
-    const double x = Y[(long)i * D], y = D == 2 ? Y[(long)i * D + 1] : 0.0;
-    switch (set) {
-    case 0: ch[4L * i] = 1; ch[4L * i + 1] = x; ch[4L * i + 2] = y; ch[4L * i + 3] = x * x + y * y; break;
-    case 1: ch[3L * i] = x; ch[3L * i + 1] = y; ch[3L * i + 2] = 1; break;
-    case 2: ch[i] = 1; break;
-    case 3: ch[3L * i] = 1; ch[3L * i + 1] = x; ch[3L * i + 2] = x * x; break;
-    default: ch[2L * i] = x; ch[2L * i + 1] = 1; break;
-    }
-}
-
 // Box index, in-box coordinates and Lagrange weights per point (nbodyfft.cpp:85-127 / :349-371):
 // box[i], wx[j*N + i], wy[j*N + i] (SoA like the reference's interpolated_values).
 template <int P, int D>
@@ -2398,6 +2384,199 @@ __global__ __launch_bounds__(kThreads) void k_spread_f64(const int *__restrict__
     }
 }
 
+// ---- the FP64 path's grid stages, in box order
+// Points are listed by box (k_box_f64, k_box_starts, k_box_order), so that a box's charges are summed once per
+// wavefront instead of one FP64 atomic per point, node and term, and the interpolation's lanes read the same
+// nodes.
+
+// Box of every point (by nb + bx) and its rank among the box's points; cnt (zero before) counts them.  Clears
+// the grid w[0..nw) on the way.
+template <int D>
+__global__ __launch_bounds__(kThreads) void k_box_f64(const double *__restrict__ Y, int N, Geo g,
+                                                      int *__restrict__ box, int *__restrict__ rank,
+                                                      int *__restrict__ cnt, int *__restrict__ used,
+                                                      double *__restrict__ w, long nw) {
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i == 0) *used = 0;
+    if (i < N) {
+        double t;
+        int b = box_coord<D>(Y[(long)i * D], g, t);
+        if constexpr (D == 2) b += box_coord<D>(Y[2L * i + 1], g, t) * g.nb;
+        box[i] = b;
+        rank[i] = atomicAdd(&cnt[b], 1);
+    }
+    for (long e = i; e < nw; e += (long)gridDim.x * kThreads) w[e] = 0.0;
+}
+
+// A place in the list for every box: start[b], in box order within a wavefront's 64 boxes, and these in the order
+// in which they come (used: places taken so far, zero before).  Clears cnt.  (Any order of the boxes serves; an
+// exclusive scan by one workgroup of 1024 threads does not start before the attractive term, beside it on its
+// own stream, leaves a CU empty enough for it: 118 us at N = 200,000.)
+__global__ __launch_bounds__(kThreads) void k_box_starts(int *__restrict__ cnt, int nbox, int *__restrict__ used,
+                                                         int *__restrict__ start) {
+    const int b = blockIdx.x * kThreads + threadIdx.x, lane = threadIdx.x % kWave;
+    const int n = b < nbox ? cnt[b] : 0;
+    int x = n;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int y = __shfl_up(x, o, kWave);
+        if (lane >= o) x += y;
+    }
+    int first = 0;
+    if (lane == kWave - 1) first = atomicAdd(used, x);
+    first = __shfl(first, kWave - 1, kWave);
+    if (b < nbox) {
+        start[b] = first + x - n;
+        cnt[b] = 0;
+    }
+}
+
+// order[start[box] + rank] = i.
+__global__ __launch_bounds__(kThreads) void k_box_order(const int *__restrict__ box, const int *__restrict__ rank,
+                                                        const int *__restrict__ start, int N, int *__restrict__ order) {
+    const int i = blockIdx.x * kThreads + threadIdx.x;
+    if (i < N) order[start[box[i]] + rank[i]] = i;
+}
+
+// Charges of the reference (tsne.cpp:1057-1062, :904-908, :939-941, :786-790, :674-677, :689-691), by set:
+// 0 = [1, x, y, x^2+y^2] (2D df=1), 1 = [x, y, 1] (2D df), 2 = [1] (general kernel), 3 = [1, y, y^2] (1D
+// df=1), 4 = [y, 1] (1D df).  Their number:
+__host__ __device__ constexpr int charge_terms(int set) { return set == 0 ? 4 : set == 1 || set == 3 ? 3 : set == 2 ? 1 : 2; }
+
+// Spread (nbodyfft.cpp:129-147 / :373-382) of charge set `set` into w[node][nt], for points in
+// box order.  A wavefront takes 64 consecutive points: each lane computes one point's weights and charges
+// into LDS; then, box after box, lane v sums value v (node a P + c, term d) over the box's points and adds
+// it to the grid: one atomic per value and run of points instead of one per point.  Bound: the LDS reads,
+// three per point and value.  (N = 200,000, 2D, 3 nodes: 14 us; one atomic per point, node and term 600.)
+template <int P, int D>
+__global__ __launch_bounds__(kThreads) void k_spread_box_f64(const double *__restrict__ Y,
+                                                             const int *__restrict__ order, int N, Geo g, int set,
+                                                             double *__restrict__ w) {
+    constexpr int NW = kThreads / kWave, NN = D == 2 ? P * P : P, MV = (NN * 4 + kWave - 1) / kWave;
+    constexpr int ROW = D * P + 4 + (D * P) % 2 + 1;  // doubles per point; odd, so that rows spread over the banks
+    __shared__ double sh[NW][kWave * ROW];
+    const int wv = threadIdx.x / kWave, l = threadIdx.x % kWave, nt = charge_terms(set);
+    const long j = (long)blockIdx.x * kThreads + threadIdx.x;
+    if (j - l >= N) return;  // whole wavefront
+    double *row = sh[wv];
+    int bx = -1, by = 0;
+    if (j < N) {
+        const long i = order[j];
+        const double x = Y[i * D], y = D == 2 ? Y[i * D + 1] : 0.0;
+        double t, L[P];
+        bx = box_coord<D>(x, g, t);
+        lagrange<P, double>(t, g, L);
+#pragma unroll
+        for (int a = 0; a < P; a++) row[l * ROW + a] = L[a];
+        if constexpr (D == 2) {
+            by = box_coord<D>(y, g, t);
+            lagrange<P, double>(t, g, L);
+#pragma unroll
+            for (int a = 0; a < P; a++) row[l * ROW + P + a] = L[a];
+        }
+        double *q = row + l * ROW + D * P;
+        switch (set) {
+        case 0: q[0] = 1; q[1] = x; q[2] = y; q[3] = x * x + y * y; break;
+        case 1: q[0] = x; q[1] = y; q[2] = 1; break;
+        case 2: q[0] = 1; break;
+        case 3: q[0] = 1; q[1] = x; q[2] = x * x; break;
+        default: q[0] = x; q[1] = 1; break;
+        }
+    }
+    const int b = bx < 0 ? -1 : by * g.nb + bx;
+    const int pb = __shfl_up(b, 1, kWave);
+    unsigned long long heads = __ballot(j < N && (l == 0 || pb != b));
+    const int n = (int)min((long)kWave, N - (j - l));
+    // the wavefront's own LDS writes, read by its other lanes
+    __threadfence_block();
+    __builtin_amdgcn_wave_barrier();
+    // value v of the lane: weights at oa, oc and charge at od of a point's row, grid node at + the box's first
+    int oa[MV], oc[MV], od[MV];
+    long at[MV];
+#pragma unroll
+    for (int m = 0; m < MV; m++) {
+        const int v = m * kWave + l, node = v / nt, d = v - node * nt;
+        const int a = D == 2 ? node / P : node, c = D == 2 ? node - a * P : 0;
+        oa[m] = node < NN ? a : -1;
+        oc[m] = P + c;
+        od[m] = D * P + d;
+        at[m] = (D == 2 ? (long)a * g.n1d + c : (long)a) * nt + d;
+    }
+    while (heads) {
+        const int s = __ffsll((long long)heads) - 1;
+        heads &= heads - 1;
+        const int e = heads ? __ffsll((long long)heads) - 1 : n;
+        const int rbx = __shfl(bx, s, kWave), rby = __shfl(by, s, kWave);
+        const long first = (D == 2 ? (long)rbx * P * g.n1d + (long)rby * P : (long)rbx * P) * nt;
+#pragma unroll
+        for (int m = 0; m < MV; m++) {
+            if (oa[m] < 0) continue;
+            double acc = 0;
+#pragma unroll 4
+            for (int p = s; p < e; p++) {
+                const double *r = row + p * ROW;
+                if constexpr (D == 2) acc += r[oc[m]] * r[oa[m]] * r[od[m]];
+                else acc += r[oa[m]] * r[od[m]];
+            }
+            atomicAdd(&w[first + at[m]], acc);
+        }
+    }
+}
+
+// Interpolation (nbodyfft.cpp:222-239 / :439-447) of NT potentials for points in box order, into pot[i][NT]
+// (nullable), with the block partials of the Z terms (tsne.cpp:1101-1110 / :945-950 / :809-817 / :705-713).
+// zform: 0 = 2D expansion on [1,x,y,x^2+y^2]; 1 = sum of phi (general kernel); 2 = 1D expansion; -1 = none.
+template <int P, int D, int NT>
+__global__ __launch_bounds__(kThreads) void k_interp_box_f64(const double *__restrict__ Y,
+                                                             const int *__restrict__ order, int N, Geo g,
+                                                             const double *__restrict__ V, int zform,
+                                                             double *__restrict__ pot, double *__restrict__ part) {
+    const int j = blockIdx.x * kThreads + threadIdx.x;
+    double z = 0;
+    if (j < N) {
+        const long i = order[j];
+        const double x = Y[i * D], y = D == 2 ? Y[i * D + 1] : 0.0;
+        double t, Lx[P], Ly[P];
+        const int bx = box_coord<D>(x, g, t);
+        lagrange<P, double>(t, g, Lx);
+        int by = 0;
+        if constexpr (D == 2) {
+            by = box_coord<D>(y, g, t);
+            lagrange<P, double>(t, g, Ly);
+        }
+        double acc[NT];
+#pragma unroll
+        for (int d = 0; d < NT; d++) acc[d] = 0;
+#pragma unroll
+        for (int a = 0; a < P; a++) {
+            if constexpr (D == 2) {
+                const double *v = V + ((long)(bx * P + a) * g.n1d + by * P) * NT;
+#pragma unroll
+                for (int c = 0; c < P; c++)
+#pragma unroll
+                    for (int d = 0; d < NT; d++) acc[d] += Lx[a] * Ly[c] * v[c * NT + d];
+            } else {
+#pragma unroll
+                for (int d = 0; d < NT; d++) acc[d] += Lx[a] * V[((long)bx * P + a) * NT + d];
+            }
+        }
+        if (pot)
+#pragma unroll
+            for (int d = 0; d < NT; d++) pot[i * NT + d] = acc[d];
+        if constexpr (NT == 4) {
+            if (zform == 0) z = (1 + x * x + y * y) * acc[0] - 2 * (x * acc[1] + y * acc[2]) + acc[3];
+        }
+        if constexpr (NT == 3) {
+            if (zform == 2) z = (1 + x * x) * acc[0] - 2 * (x * acc[1]) + acc[2];
+        }
+        if (zform == 1) z = acc[0];
+    }
+    if (zform < 0) return;
+    __shared__ double sh[kThreads / kWave];
+    z = block_sum(z, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = z;
+}
+
 // Interpolate potentials back (nbodyfft.cpp:222-239 / :439-447), accumulating like the reference.
 template <int P, int D>
 __global__ __launch_bounds__(kThreads) void k_interp_f64(const int *__restrict__ box, const double *__restrict__ wx,
@@ -2425,30 +2604,6 @@ __global__ __launch_bounds__(kThreads) void k_interp_f64(const int *__restrict__
     for (int d = 0; d < nterms; d++) pot[(long)i * nterms + d] += acc[d];
 }
 
-// Per-point Z terms and block partials (tsne.cpp:1101-1110 / :945-950 / :809-817 / :705-713).
-// zform: 0 = 2D expansion on [1,x,y,x^2+y^2]; 1 = sum of phi (general kernel); 2 = 1D expansion.
-__global__ __launch_bounds__(kThreads) void k_zterms_f64(const double *__restrict__ Y, const double *__restrict__ pot,
-                                                         int N, int D, int zform, double *__restrict__ part) {
-    const int i = blockIdx.x * kThreads + threadIdx.x;
-    double s = 0;
-    if (i < N) {
-        if (zform == 0) {
-            const double x = Y[2L * i], y = Y[2L * i + 1];
-            const double *p = pot + 4L * i;
-            s = (1 + x * x + y * y) * p[0] - 2 * (x * p[1] + y * p[2]) + p[3];
-        } else if (zform == 1) {
-            s = pot[i];
-        } else {
-            const double y = Y[i];
-            const double *p = pot + 3L * i;
-            s = (1 + y * y) * p[0] - 2 * (y * p[1]) + p[2];
-        }
-    }
-    __shared__ double sh[kThreads / kWave];
-    s = block_sum(s, sh);
-    if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-
 __global__ void k_sum_final(const double *__restrict__ part, int nblk, double sub, double *__restrict__ out) {
     __shared__ double sh[kThreads / kWave];
     double s = 0;
@@ -2464,42 +2619,79 @@ __global__ void k_sum_final(const double *__restrict__ part, int nblk, double su
 // cform: 0 = 2D [1,x,y,..]: neg = (x phi0 - phi1, y phi0 - phi2) / Z, stride 4
 //        1 = 2D df [x,y,1]: neg = (x phi2 - phi0, y phi2 - phi1) / Z, stride 3
 //        2 = 1D [1,y,y^2]: neg = (y phi0 - phi1) / Z, stride 3;  3 = 1D df [y,1]: (y phi1 - phi0)/Z, stride 2
+__device__ __forceinline__ void combine_point(const double *__restrict__ Y, const double *__restrict__ pos,
+                                              const double *__restrict__ pot, double Z, long i, int cform,
+                                              double (&dy)[2]) {
+    switch (cform) {
+    case 0: {
+        const double *p = pot + 4L * i;
+        dy[0] = pos[2L * i] - (Y[2L * i] * p[0] - p[1]) / Z;
+        dy[1] = pos[2L * i + 1] - (Y[2L * i + 1] * p[0] - p[2]) / Z;
+        break;
+    }
+    case 1: {
+        const double *p = pot + 3L * i;
+        dy[0] = pos[2L * i] - (Y[2L * i] * p[2] - p[0]) / Z;
+        dy[1] = pos[2L * i + 1] - (Y[2L * i + 1] * p[2] - p[1]) / Z;
+        break;
+    }
+    case 2: dy[0] = pos[i] - (Y[i] * pot[3L * i] - pot[3L * i + 1]) / Z; break;
+    default: dy[0] = pos[i] - (Y[i] * pot[2L * i + 1] - pot[2L * i]) / Z; break;
+    }
+}
+
 __global__ __launch_bounds__(kThreads) void k_combine_f64(const double *__restrict__ Y, const double *__restrict__ pos,
                                                           const double *__restrict__ pot, const double *__restrict__ zbuf,
                                                           int N, int cform, double *__restrict__ dC) {
     const int i = blockIdx.x * kThreads + threadIdx.x;
     if (i >= N) return;
-    const double Z = zbuf[0];
-    switch (cform) {
-    case 0: {
-        const double x = Y[2L * i], y = Y[2L * i + 1];
-        const double *p = pot + 4L * i;
-        dC[2L * i] = pos[2L * i] - (x * p[0] - p[1]) / Z;
-        dC[2L * i + 1] = pos[2L * i + 1] - (y * p[0] - p[2]) / Z;
-        break;
-    }
-    case 1: {
-        const double x = Y[2L * i], y = Y[2L * i + 1];
-        const double *p = pot + 3L * i;
-        dC[2L * i] = pos[2L * i] - (x * p[2] - p[0]) / Z;
-        dC[2L * i + 1] = pos[2L * i + 1] - (y * p[2] - p[1]) / Z;
-        break;
-    }
-    case 2: {
-        const double y = Y[i];
-        dC[i] = pos[i] - (y * pot[3L * i] - pot[3L * i + 1]) / Z;
-        break;
-    }
-    default: {
-        const double y = Y[i];
-        dC[i] = pos[i] - (y * pot[2L * i + 1] - pot[2L * i]) / Z;
-        break;
-    }
+    double dy[2];
+    combine_point(Y, pos, pot, zbuf[0], i, cform, dy);
+    if (cform < 2) {
+        dC[2L * i] = dy[0];
+        dC[2L * i + 1] = dy[1];
+    } else {
+        dC[i] = dy[0];
     }
 }
 
 // Optimiser update, FP64, exactly the reference's elementwise loops (tsne.cpp:478-514), with the
 // block partial sums of the new Y for zeroMean.
+// One point's update with gradient dy[D]; ys: its new coordinates.
+__device__ __forceinline__ void update_point(double *__restrict__ Y, double *__restrict__ uY, double *__restrict__ gains,
+                                             const double *dy, long i, int D, double momentum, double lr, double msn,
+                                             int plain_descent, double *ys) {
+    if (plain_descent) {
+        for (int d = 0; d < D; d++) {
+            Y[i * D + d] = Y[i * D + d] - dy[d];
+            ys[d] = Y[i * D + d];
+        }
+        return;
+    }
+    double u[4], step = 0;
+    for (int d = 0; d < D; d++) {
+        const long e = i * D + d;
+        const double sd = dy[d] == .0 ? .0 : (dy[d] < .0 ? -1.0 : 1.0);
+        const double su = uY[e] == .0 ? .0 : (uY[e] < .0 ? -1.0 : 1.0);
+        double gn = sd != su ? gains[e] + .2 : gains[e] * .8;
+        if (gn < .01) gn = .01;
+        gains[e] = gn;
+        u[d] = momentum * uY[e] - lr * gn * dy[d];
+        step += u[d] * u[d];
+    }
+    if (msn > 0) {
+        step = sqrt(step);
+        if (step > msn)
+            for (int d = 0; d < D; d++) u[d] *= (msn / step);
+    }
+    for (int d = 0; d < D; d++) {
+        const long e = i * D + d;
+        uY[e] = u[d];
+        Y[e] = Y[e] + u[d];
+        ys[d] = Y[e];
+    }
+}
+
 __global__ __launch_bounds__(kThreads) void k_update_f64(double *__restrict__ Y, double *__restrict__ uY,
                                                          double *__restrict__ gains, const double *__restrict__ dY,
                                                          int N, int D, double momentum, double lr, double msn,
@@ -2507,35 +2699,9 @@ __global__ __launch_bounds__(kThreads) void k_update_f64(double *__restrict__ Y,
     const int i = blockIdx.x * kThreads + threadIdx.x;
     double ys[4] = {0, 0, 0, 0};  // D <= 4
     if (i < N) {
-        if (plain_descent) {
-            for (int d = 0; d < D; d++) {
-                Y[(long)i * D + d] = Y[(long)i * D + d] - dY[(long)i * D + d];
-                ys[d] = Y[(long)i * D + d];
-            }
-        } else {
-            double u[4], step = 0;
-            for (int d = 0; d < D; d++) {
-                const long e = (long)i * D + d;
-                const double sd = dY[e] == .0 ? .0 : (dY[e] < .0 ? -1.0 : 1.0);
-                const double su = uY[e] == .0 ? .0 : (uY[e] < .0 ? -1.0 : 1.0);
-                double gn = sd != su ? gains[e] + .2 : gains[e] * .8;
-                if (gn < .01) gn = .01;
-                gains[e] = gn;
-                u[d] = momentum * uY[e] - lr * gn * dY[e];
-                step += u[d] * u[d];
-            }
-            if (msn > 0) {
-                step = sqrt(step);
-                if (step > msn)
-                    for (int d = 0; d < D; d++) u[d] *= (msn / step);
-            }
-            for (int d = 0; d < D; d++) {
-                const long e = (long)i * D + d;
-                uY[e] = u[d];
-                Y[e] = Y[e] + u[d];
-                ys[d] = Y[e];
-            }
-        }
+        double dy[4];
+        for (int d = 0; d < D; d++) dy[d] = dY[(long)i * D + d];
+        update_point(Y, uY, gains, dy, i, D, momentum, lr, msn, plain_descent, ys);
     }
     __shared__ double sh[kThreads / kWave];
     for (int d = 0; d < D; d++) {
@@ -2544,12 +2710,30 @@ __global__ __launch_bounds__(kThreads) void k_update_f64(double *__restrict__ Y,
     }
 }
 
-// Split interleaved Y (FP64) into xs, ys (tsne.cpp:1042-1044).
-__global__ void k_split_f64(const double *__restrict__ Y, int N, double *__restrict__ xs, double *__restrict__ ys) {
+// k_combine_f64 and k_update_f64 in one pass over the points (D from cform).
+template <int D>
+__global__ __launch_bounds__(kThreads) void k_combine_update_f64(double *__restrict__ Y,
+                                                                 const double *__restrict__ pos,
+                                                                 const double *__restrict__ pot,
+                                                                 const double *__restrict__ zbuf, int N, int cform,
+                                                                 double *__restrict__ dC, double *__restrict__ uY,
+                                                                 double *__restrict__ gains, double momentum,
+                                                                 double lr, double msn, int plain_descent,
+                                                                 double *__restrict__ part) {
     const int i = blockIdx.x * kThreads + threadIdx.x;
+    double ys[4] = {0, 0, 0, 0};
     if (i < N) {
-        xs[i] = Y[2L * i];
-        ys[i] = Y[2L * i + 1];
+        double dy[2];
+        combine_point(Y, pos, pot, zbuf[0], i, cform, dy);
+#pragma unroll
+        for (int d = 0; d < D; d++) dC[(long)i * D + d] = dy[d];
+        update_point(Y, uY, gains, dy, i, D, momentum, lr, msn, plain_descent, ys);
+    }
+    __shared__ double sh[kThreads / kWave];
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+        const double s = block_sum(ys[d], sh);
+        if (threadIdx.x == 0) part[blockIdx.x * D + d] = s;
     }
 }
 
