@@ -3,12 +3,14 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/fitsne_abi.h"
@@ -188,6 +190,11 @@ struct fitsne_ctx {
     std::map<int, DBuf> tw32, tw64;
     // min/max handoff from the last step
     double *h_mm = nullptr;      // pinned [4]
+    char *stage = nullptr;       // pinned, at most kStage bytes: stage_copy's two halves (first behind h_mm)
+    char *stage_dev = nullptr;   // the same as the device addresses it
+    size_t stage_cap = 0;
+    hipEvent_t stage_ev[2] = {nullptr, nullptr};
+    DBuf ybuf;                   // the caller's Y, dC or a part of P as doubles
     double *h_mm_dev = nullptr;  // h_mm as the device addresses it
     hipEvent_t mm_event = nullptr;
     bool mm_pending = false, mm_valid = false;
@@ -315,6 +322,167 @@ static int sw_for(long long nnz, int N) {
 static int att_lanes(long long nnz, int N) {
     const double avg = N > 0 ? (double)nnz / N : 0;
     return avg >= 64 ? 16 : 8;
+}
+
+// ---------------------------------------------------------------- copies between host and device
+// The runtime's copies from and to pageable memory are slow around 1 MB (0.4 ms against 28 us from pinned
+// memory) and where the destination's pages are new (4 to 6 GB/s: one thread takes the page faults).  So copies go through a pinned buffer of the context, in pieces, the DMA of one
+// beside the memcpy of the other, and large ones have several threads for the memcpy (fresh pages:
+// 4.8 GB/s with one thread, 21 with eight; DMA 57).
+
+// Threads that copy their share of a piece beside the caller's; they last for one stage_copy.
+class CopyTeam {
+  public:
+    explicit CopyTeam(int helpers) {
+        try {
+            for (int i = 0; i < helpers; i++) th_.emplace_back([this, i] { work(i + 1); });
+        } catch (...) {  // no more threads: copy with those that started
+        }
+    }
+    ~CopyTeam() {
+        stop_ = true;
+        gen_.fetch_add(1, std::memory_order_release);
+        for (auto &t : th_) t.join();
+    }
+    void copy(char *dst, const char *src, size_t len) {
+        dst_ = dst;
+        src_ = src;
+        len_ = len;
+        parts_ = (int)th_.size() + 1;
+        left_.store((int)th_.size(), std::memory_order_relaxed);
+        gen_.fetch_add(1, std::memory_order_release);
+        part(0);
+        spin([this] { return left_.load(std::memory_order_acquire) == 0; });
+    }
+
+  private:
+    template <typename F>
+    static void spin(F done) {
+        for (int n = 0; !done(); n++)
+            if (n > 200) std::this_thread::yield();
+    }
+    void part(int i) {
+        const size_t share = (len_ / parts_ + 4095) & ~(size_t)4095, at = std::min(len_, share * i);
+        const size_t end = i + 1 == parts_ ? len_ : std::min(len_, at + share);
+        memcpy(dst_ + at, src_ + at, end - at);
+    }
+    void work(int i) {
+        for (int seen = 0;;) {
+            spin([&] { return gen_.load(std::memory_order_acquire) != seen; });
+            seen++;
+            if (stop_) return;
+            part(i);
+            left_.fetch_sub(1, std::memory_order_release);
+        }
+    }
+    std::vector<std::thread> th_;
+    std::atomic<int> gen_{0}, left_{0};
+    bool stop_ = false;
+    char *dst_ = nullptr;
+    const char *src_ = nullptr;
+    size_t len_ = 0;
+    int parts_ = 1;
+};
+
+constexpr size_t kStage = 4u << 20;
+constexpr size_t kStageFirst = 64 << 10;  // the context's first pinned allocation: h_mm in 256 bytes, then the stage
+static char *first_stage(const fitsne_ctx *c) { return reinterpret_cast<char *>(c->h_mm) + 256; }
+
+// At least `need` (<= kStage) bytes of pinned buffer; nothing may be in flight in it.
+static int stage_room(fitsne_ctx *c, size_t need) {
+    if (need <= c->stage_cap) return FITSNE_OK;
+    if (c->stage && c->stage != first_stage(c)) (void)hipHostFree(c->stage);
+    c->stage = nullptr;
+    c->stage_cap = 0;
+    size_t want = kStageFirst;
+    while (want < need) want *= 2;
+    if (hipHostMalloc((void **)&c->stage, want, hipHostMallocDefault) != hipSuccess ||
+        hipHostGetDevicePointer((void **)&c->stage_dev, c->stage, 0) != hipSuccess) {
+        if (c->stage) (void)hipHostFree(c->stage);
+        c->stage = nullptr;
+        return fail(FITSNE_E_ALLOC, "pinned allocation of " + std::to_string(want) + " bytes failed");
+    }
+    c->stage_cap = want;
+    return FITSNE_OK;
+}
+
+// Up to here the kernels read and write the caller's rows in the pinned buffer themselves (a DMA of its own costs
+// 10 us).
+constexpr size_t kStageDirect = 1 << 20;
+
+// bytes from device memory dev to host (out) or back, on c->stream behind what is queued there; done when it
+// returns.  Pieces: a quarter of the copy, from 256 KB (below which the DMA's latency shows) to half the buffer.
+// Helpers: one per 4 MB (starting one costs 20 us), at most seven.
+static int stage_copy(fitsne_ctx *c, char *host, char *dev, size_t bytes, bool out) {
+    if (!bytes) return FITSNE_OK;
+    const size_t piece = std::min(std::max((bytes / 4 + 4095) & ~(size_t)4095, (size_t)256 << 10), kStage / 2);
+    const size_t need = std::min(bytes, 2 * piece), n = (bytes + piece - 1) / piece;
+    TRY(stage_room(c, need));
+    auto half = [&](size_t k) { return c->stage + (k & 1) * piece; };
+    auto len = [&](size_t k) { return std::min(piece, bytes - k * piece); };
+    auto dma = [&](size_t k) {
+        return out ? hipMemcpyAsync(half(k), dev + k * piece, len(k), hipMemcpyDeviceToHost, c->stream)
+                   : hipMemcpyAsync(dev + k * piece, half(k), len(k), hipMemcpyHostToDevice, c->stream);
+    };
+    if (out) HIPTRY(dma(0));
+    CopyTeam team((int)std::min<size_t>({bytes >> 22, 7, std::max(1u, std::thread::hardware_concurrency()) - 1}));
+    for (size_t k = 0; k < n; k++) {
+        if (out) {
+            HIPTRY(hipStreamSynchronize(c->stream));
+            if (k + 1 < n) HIPTRY(dma(k + 1));
+            team.copy(host + k * piece, half(k), len(k));
+        } else {
+            hipEvent_t &ev = c->stage_ev[k & 1];
+            if (!ev) HIPTRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+            if (k >= 2) HIPTRY(hipEventSynchronize(ev));
+            team.copy(half(k), host + k * piece, len(k));
+            HIPTRY(dma(k));
+            if (k + 2 < n) HIPTRY(hipEventRecord(ev, c->stream));
+        }
+    }
+    if (!out) HIPTRY(hipStreamSynchronize(c->stream));
+    return FITSNE_OK;
+}
+
+static int copy_out(fitsne_ctx *c, void *dst, const void *src, size_t bytes) {
+    return stage_copy(c, static_cast<char *>(dst), static_cast<char *>(const_cast<void *>(src)), bytes, true);
+}
+// (Up to 512 KB the runtime's own copy to the device is as fast: 480 KB in 24 us.)
+static int copy_in(fitsne_ctx *c, void *dst, const void *src, size_t bytes) {
+    if (bytes <= (512 << 10)) {
+        HIPTRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+        HIPTRY(hipStreamSynchronize(c->stream));
+        return FITSNE_OK;
+    }
+    return stage_copy(c, static_cast<char *>(const_cast<void *>(src)), static_cast<char *>(dst), bytes, false);
+}
+
+// An error with this text if any of the n device doubles is infinite or NaN.
+static int need_finite(fitsne_ctx *c, const double *x, long n, const char *text) {
+    volatile int *flag = reinterpret_cast<volatile int *>(c->h_mm + 3);
+    *flag = 0;
+    launch(c, "nonfinite", k_nonfinite, dim3(std::min(blocks_for(n), 2048)), dim3(kThreads), 0, x, n,
+           reinterpret_cast<int *>(c->h_mm_dev + 3));
+    HIPTRY(hipGetLastError());
+    HIPTRY(hipStreamSynchronize(c->stream));
+    return *flag ? fail(FITSNE_E_ARG, text) : FITSNE_OK;
+}
+
+// Y or dC (N x D) in the caller's order and type.
+static int rows_to_host(fitsne_ctx *c, const DBuf &b, double *dst) {
+    const size_t n = (size_t)c->N * c->D, bytes = sizeof(double) * n;
+    if (c->precision != FITSNE_FP32) return copy_out(c, dst, b.p, bytes);
+    const bool direct = bytes <= kStageDirect;
+    if (direct) TRY(stage_room(c, bytes));
+    else TRY(ensure(c->ybuf, bytes));
+    launch(c, "rows_out", k_rows_out<float>, dim3(blocks_for((long)n)), dim3(kThreads), 0, b.as<const float>(),
+           c->permuted ? c->inv_d.as<const int>() : (const int *)nullptr, (long)n, c->D,
+           direct ? reinterpret_cast<double *>(c->stage_dev) : c->ybuf.as<double>());
+    HIPTRY(hipGetLastError());
+    if (!direct) return copy_out(c, dst, c->ybuf.p, bytes);
+    HIPTRY(hipStreamSynchronize(c->stream));
+    memcpy(dst, c->stage, bytes);
+    return FITSNE_OK;
 }
 
 // ---------------------------------------------------------------- min / max of the resident Y
@@ -1782,13 +1950,16 @@ extern "C" int fitsne_ctx_create(fitsne_ctx **out, int device, int precision, in
         hipEventCreateWithFlags(&c->kern_ev, kEvFlags) != hipSuccess ||
         hipEventCreateWithFlags(&c->kl_go, kEvFlags) != hipSuccess ||
         hipEventCreateWithFlags(&c->kl_ev, kEvFlags) != hipSuccess ||
-        hipHostMalloc((void **)&c->h_mm, sizeof(double) * 4, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void **)&c->h_mm, kStageFirst, hipHostMallocDefault) != hipSuccess ||
         hipHostGetDevicePointer((void **)&c->h_mm_dev, c->h_mm, 0) != hipSuccess ||
         hipEventCreateWithFlags(&c->mm_event, kEvFlags) != hipSuccess) {
         delete c;
         return fail(FITSNE_E_HIP, "stream/event/pinned allocation failed");
     }
     c->own_stream = c->stream;
+    c->stage = first_stage(c);
+    c->stage_dev = reinterpret_cast<char *>(c->h_mm_dev) + 256;
+    c->stage_cap = kStageFirst - 256;
     *out = c;
     return FITSNE_OK;
 }
@@ -1810,7 +1981,8 @@ extern "C" int fitsne_ctx_destroy(fitsne_ctx *c) {
                    &c->sy_row, &c->sy_col, &c->sy_val, &c->sy_erow, &c->sy_keys, &c->sy_keys2, &c->sy_vals,
                    &c->sy_vals2, &c->sy_partner, &c->sy_cnt, &c->sy_start, &c->sy_okeys, &c->sy_okeys2, &c->sy_tmp,
                    &c->sy_scol, &c->sy_sval, &c->bh_cell, &c->bh_leafpt, &c->bh_neg, &c->bh_Q, &c->bh_root, &c->bh_key,
-                   &c->bh_idx, &c->bh_pos, &c->bh_span, &c->bh_list, &c->bh_order, &c->bh_tmp, &c->bh_ab, &c->kline};
+                   &c->bh_idx, &c->bh_pos, &c->bh_span, &c->bh_list, &c->bh_order, &c->bh_tmp, &c->bh_ab, &c->kline,
+                   &c->ybuf};
     for (DBuf *b : all) release(*b);
     for (auto &kv : c->tw32) release(kv.second);
     for (auto &kv : c->tw64) release(kv.second);
@@ -1829,7 +2001,10 @@ extern "C" int fitsne_ctx_destroy(fitsne_ctx *c) {
     if (c->bh_ev) (void)hipEventDestroy(c->bh_ev);
     if (c->astream) (void)hipStreamDestroy(c->astream);
     if (c->kstream) (void)hipStreamDestroy(c->kstream);
+    if (c->stage && c->stage != first_stage(c)) (void)hipHostFree(c->stage);
     if (c->h_mm) (void)hipHostFree(c->h_mm);
+    for (hipEvent_t e : c->stage_ev)
+        if (e) (void)hipEventDestroy(e);
     if (c->bh_pin) (void)hipHostFree(c->bh_pin);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
     delete c;
@@ -1850,25 +2025,34 @@ static int set_P_impl(fitsne_ctx *c, int N, const TI *row_P, const TC *col_P, co
         if ((long long)row_P[i + 1] < (long long)row_P[i]) return fail(FITSNE_E_ARG, "row_P must be non-decreasing");
     std::vector<int64_t> r(N + 1);
     for (int i = 0; i <= N; i++) r[i] = (int64_t)row_P[i];
-    std::vector<uint32_t> cc((size_t)nnz);
-    for (long long k = 0; k < nnz; k++) {
-        const long long j = (long long)col_P[k];
-        if (j < 0 || j >= N) return fail(FITSNE_E_ARG, "col_P entry out of range");
-        cc[k] = (uint32_t)j;
-    }
+    static_assert(sizeof(TC) == sizeof(uint32_t), "the caller's columns are copied as they are");
+    bool out_of_range = false;
+    for (long long k = 0; k < nnz; k++) out_of_range |= (uint32_t)col_P[k] >= (uint32_t)N;  // (negative ones too)
+    if (out_of_range) return fail(FITSNE_E_ARG, "col_P entry out of range");
     TRY(sync_ctx(c));
     TRY(ensure(c->rowP, sizeof(int64_t) * (N + 1)));
     TRY(ensure(c->colP, sizeof(uint32_t) * (size_t)std::max<long long>(nnz, 1)));
-    HIPTRY(hipMemcpy(c->rowP.p, r.data(), sizeof(int64_t) * (N + 1), hipMemcpyHostToDevice));
-    if (nnz) HIPTRY(hipMemcpy(c->colP.p, cc.data(), sizeof(uint32_t) * nnz, hipMemcpyHostToDevice));
+    TRY(copy_in(c, c->rowP.p, r.data(), sizeof(int64_t) * (N + 1)));
+    TRY(copy_in(c, c->colP.p, col_P, sizeof(uint32_t) * nnz));
     if (c->precision == FITSNE_FP32) {
-        std::vector<float> v((size_t)nnz);
-        for (long long k = 0; k < nnz; k++) v[k] = (float)val_P[k];
         TRY(ensure(c->val, sizeof(float) * (size_t)std::max<long long>(nnz, 1)));
-        if (nnz) HIPTRY(hipMemcpy(c->val.p, v.data(), sizeof(float) * nnz, hipMemcpyHostToDevice));
+        // a small P is converted here, a large one on the device (a call with 252,000 entries 209 us, with 277,200
+        // 215; 18 million 8.5 ms, converted here 41)
+        std::vector<float> v(nnz <= (1 << 18) ? (size_t)nnz : 0);
+        for (size_t k = 0; k < v.size(); k++) v[k] = (float)val_P[k];
+        if (!v.empty()) TRY(copy_in(c, c->val.p, v.data(), sizeof(float) * v.size()));
+        constexpr long long kChunk = 4 << 20;  // doubles on the device at a time
+        if (v.empty()) TRY(ensure(c->ybuf, sizeof(double) * (size_t)std::min(std::max<long long>(nnz, 1), kChunk)));
+        for (long long k = v.size(); k < nnz; k += kChunk) {
+            const long m = (long)std::min(nnz - k, kChunk);
+            TRY(copy_in(c, c->ybuf.p, val_P + k, sizeof(double) * m));
+            launch(c, "to_float", k_to_float, dim3(blocks_for(m)), dim3(kThreads), 0, c->ybuf.as<const double>(), m,
+                   c->val.as<float>() + k);
+        }
+        TRY(sync_ctx(c));
     } else {
         TRY(ensure(c->val, sizeof(double) * (size_t)std::max<long long>(nnz, 1)));
-        if (nnz) HIPTRY(hipMemcpy(c->val.p, val_P, sizeof(double) * nnz, hipMemcpyHostToDevice));
+        TRY(copy_in(c, c->val.p, val_P, sizeof(double) * nnz));
     }
     if (N != c->N) c->mm_valid = c->mm_pending = false;
     c->N = N;
@@ -1945,7 +2129,7 @@ extern "C" int fitsne_set_P_dense(fitsne_ctx *c, int N, const double *P) {
     TRY(sync_ctx(c));
     const size_t nn = (size_t)N * N;
     TRY(ensure(c->val, sizeof(double) * nn));
-    HIPTRY(hipMemcpy(c->val.p, P, sizeof(double) * nn, hipMemcpyHostToDevice));
+    TRY(copy_in(c, c->val.p, P, sizeof(double) * nn));
     dense_P_set(c, N);
     return FITSNE_OK;
 }
@@ -1969,18 +2153,17 @@ extern "C" int fitsne_exact_affinities(fitsne_ctx *c, const double *X, int N, in
         plist.push_back(perplexity);  // the kernel takes the fixed width when perplexity <= 0
     }
     const size_t nd = (size_t)N * D, nn = (size_t)N * N;
-    for (size_t i = 0; i < nd; i++)
-        if (!std::isfinite(X[i])) return fail(FITSNE_E_ARG, "X contains non-finite values");
     HIPTRY(hipSetDevice(c->device));
     TRY(sync_ctx(c));
     TRY(ensure(c->knnX, sizeof(double) * nd));
+    TRY(copy_in(c, c->knnX.p, X, sizeof(double) * nd));
+    TRY(need_finite(c, c->knnX.as<const double>(), (long)nd, "X contains non-finite values"));
     TRY(ensure(c->knnXT, sizeof(double) * nd));
     TRY(ensure(c->w, sizeof(double) * nn));
     TRY(ensure(c->val, sizeof(double) * nn));
     TRY(ensure(c->xs, sizeof(double) * (size_t)N));
     TRY(ensure(c->klpart, sizeof(double) * kDenseSumBlocks));
     TRY(ensure(c->zbuf, sizeof(double) * 4));
-    HIPTRY(hipMemcpy(c->knnX.p, X, sizeof(double) * nd, hipMemcpyHostToDevice));
     launch(c, "transpose64", k_transpose_f64, dim3((N + 31) / 32, (D + 31) / 32), dim3(256), 0,
            c->knnX.as<const double>(), (long)N, D, c->knnXT.as<double>());
     launch(c, "sqdist64", k_sqdist_f64, dim3(blocks_for(N), (N + kSqRows - 1) / kSqRows), dim3(kThreads), 0,
@@ -2008,9 +2191,9 @@ extern "C" int fitsne_exact_affinities(fitsne_ctx *c, const double *X, int N, in
     HIPTRY(hipGetLastError());
     double total = 0.0;
     HIPTRY(hipMemcpyAsync(c->h_mm + 3, c->zbuf.p, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    if (P_out) HIPTRY(hipMemcpyAsync(P_out, c->val.p, sizeof(double) * nn, hipMemcpyDeviceToHost, c->stream));
     TRY(sync_ctx(c));
     total = c->h_mm[3];
+    if (P_out) TRY(copy_out(c, P_out, c->val.p, sizeof(double) * nn));
     release(c->w);  // the N x N distance matrix is not needed after the calibration
     dense_P_set(c, N);
     if (sum_P) *sum_P = total;
@@ -2034,7 +2217,7 @@ static int reorder_points(fitsne_ctx *c) {
     drop_graph(c);
     c->mm_parts_valid = false;
     std::vector<float> y((size_t)N * D);
-    HIPTRY(hipMemcpy(y.data(), c->Y.p, sizeof(float) * y.size(), hipMemcpyDeviceToHost));
+    TRY(copy_out(c, y.data(), c->Y.p, sizeof(float) * y.size()));
     float lo[2] = {INFINITY, INFINITY}, hi[2] = {-INFINITY, -INFINITY};
     for (int i = 0; i < N; i++)
         for (int d = 0; d < D; d++) {
@@ -2042,8 +2225,11 @@ static int reorder_points(fitsne_ctx *c) {
             hi[d] = std::max(hi[d], y[(size_t)i * D + d]);
         }
     const int G = D == 2 ? 512 : 1 << 18;
-    const int nkeys = D == 2 ? G * G : G;
-    std::vector<int> key(N), cnt(nkeys + 1, 0);
+    // keys of 18 bits, sorted by two stable counting passes of 9 (one pass over 2^18 counters costs more than
+    // all the rest for a small embedding)
+    constexpr int kBits = 9, kBuckets = 1 << kBits;
+    std::vector<int> key(N), rel(N), irel(N), lowp(N);
+    int cnt[2][kBuckets + 1] = {};
     for (int i = 0; i < N; i++) {
         uint32_t q[2] = {0, 0};
         for (int d = 0; d < D; d++) {
@@ -2053,11 +2239,13 @@ static int reorder_points(fitsne_ctx *c) {
             q[d] = (uint32_t)std::min(std::max(v, 0), G - 1);
         }
         key[i] = D == 2 ? (int)morton2(q[0], q[1]) : (int)q[0];
-        cnt[key[i] + 1]++;
+        cnt[0][(key[i] & (kBuckets - 1)) + 1]++;
+        cnt[1][(key[i] >> kBits) + 1]++;
     }
-    for (int k = 0; k < nkeys; k++) cnt[k + 1] += cnt[k];
-    std::vector<int> rel(N), irel(N);
-    for (int i = 0; i < N; i++) rel[cnt[key[i]]++] = i;  // stable
+    for (auto &t : cnt)
+        for (int k = 0; k < kBuckets; k++) t[k + 1] += t[k];
+    for (int i = 0; i < N; i++) lowp[cnt[0][key[i] & (kBuckets - 1)]++] = i;
+    for (int j = 0; j < N; j++) rel[cnt[1][key[lowp[j]] >> kBits]++] = lowp[j];
     for (int r = 0; r < N; r++) irel[rel[r]] = r;
     std::vector<int64_t> rown(N + 1);
     rown[0] = 0;
@@ -2069,9 +2257,9 @@ static int reorder_points(fitsne_ctx *c) {
     DBuf rowN;
     TRY(ensure(rowN, sizeof(int64_t) * (N + 1)));
     int *d_rel = c->tmp.as<int>(), *d_irel = c->tmp.as<int>() + N;
-    HIPTRY(hipMemcpy(d_rel, rel.data(), sizeof(int) * N, hipMemcpyHostToDevice));
-    HIPTRY(hipMemcpy(d_irel, irel.data(), sizeof(int) * N, hipMemcpyHostToDevice));
-    HIPTRY(hipMemcpy(rowN.p, rown.data(), sizeof(int64_t) * (N + 1), hipMemcpyHostToDevice));
+    TRY(copy_in(c, d_rel, rel.data(), sizeof(int) * N));
+    TRY(copy_in(c, d_irel, irel.data(), sizeof(int) * N));
+    TRY(copy_in(c, rowN.p, rown.data(), sizeof(int64_t) * (N + 1)));
     launch(c, "permute_csr", k_permute_csr<float>, dim3(blocks_for((long)N * kWave)), dim3(kThreads), 0,
            c->rowP.as<const int64_t>(), c->colP.as<const uint32_t>(), c->val.as<const float>(),
            rowN.as<const int64_t>(), (const int *)d_rel, (const int *)d_irel, N, c->colP2.as<uint32_t>(),
@@ -2099,7 +2287,7 @@ static int reorder_points(fitsne_ctx *c) {
     for (int r = 0; r < N; r++) c->inv[c->perm[r]] = r;
     c->rowP_host.swap(rown);
     TRY(ensure(c->inv_d, sizeof(int) * (size_t)N));
-    HIPTRY(hipMemcpy(c->inv_d.p, c->inv.data(), sizeof(int) * N, hipMemcpyHostToDevice));
+    TRY(copy_in(c, c->inv_d.p, c->inv.data(), sizeof(int) * N));
     c->permuted = true;
     c->win_ok = false;
     c->mm_valid = c->mm_pending = false;
@@ -2140,31 +2328,33 @@ extern "C" int fitsne_set_Y(fitsne_ctx *c, const double *Y) {
     if (!c || !Y) return fail(FITSNE_E_ARG, "null argument");
     if (c->N <= 0) return fail(FITSNE_E_ARG, "set P before Y");
     const size_t n = (size_t)c->N * c->D;
-    for (size_t e = 0; e < n; e++)
-        if (!std::isfinite(Y[e])) return fail(FITSNE_E_ARG, "Y contains non-finite values");
     HIPTRY(hipSetDevice(c->device));
     TRY(sync_ctx(c));
-    c->ctr_lazy = false;  // Y is replaced: a pending centring is void
-    const int D = c->D;
-    if (c->precision == FITSNE_FP32) {
-        std::vector<float> y(n), z(n, 0.f), one(n, 1.f);
-        for (size_t r = 0; r < (size_t)c->N; r++)
-            for (int d = 0; d < D; d++) y[r * D + d] = (float)Y[(size_t)c->perm[r] * D + d];
-        TRY(ensure(c->Y, sizeof(float) * n));
-        TRY(ensure(c->uY, sizeof(float) * n));
-        TRY(ensure(c->gains, sizeof(float) * n));
-        HIPTRY(hipMemcpy(c->Y.p, y.data(), sizeof(float) * n, hipMemcpyHostToDevice));
-        HIPTRY(hipMemcpy(c->uY.p, z.data(), sizeof(float) * n, hipMemcpyHostToDevice));
-        HIPTRY(hipMemcpy(c->gains.p, one.data(), sizeof(float) * n, hipMemcpyHostToDevice));
+    const double *src;
+    if (sizeof(double) * n <= kStageDirect) {
+        TRY(stage_room(c, sizeof(double) * n));
+        memcpy(c->stage, Y, sizeof(double) * n);
+        src = reinterpret_cast<const double *>(c->stage_dev);
     } else {
-        std::vector<double> z(n, 0.0), one(n, 1.0);
-        TRY(ensure(c->Y, sizeof(double) * n));
-        TRY(ensure(c->uY, sizeof(double) * n));
-        TRY(ensure(c->gains, sizeof(double) * n));
-        HIPTRY(hipMemcpy(c->Y.p, Y, sizeof(double) * n, hipMemcpyHostToDevice));
-        HIPTRY(hipMemcpy(c->uY.p, z.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-        HIPTRY(hipMemcpy(c->gains.p, one.data(), sizeof(double) * n, hipMemcpyHostToDevice));
+        TRY(ensure(c->ybuf, sizeof(double) * n));
+        TRY(copy_in(c, c->ybuf.p, Y, sizeof(double) * n));
+        src = c->ybuf.as<const double>();
     }
+    TRY(need_finite(c, src, (long)n, "Y contains non-finite values"));
+    c->ctr_lazy = false;  // Y is replaced: a pending centring is void
+    const int nblk = blocks_for((long)n), fblk = std::min(nblk, 2048);
+    auto load = [&](auto zero) {
+        using TV = decltype(zero);
+        TRY(ensure(c->Y, sizeof(TV) * n));
+        TRY(ensure(c->uY, sizeof(TV) * n));
+        TRY(ensure(c->gains, sizeof(TV) * n));
+        launch(c, "rows_in", k_rows_in<TV>, dim3(nblk), dim3(kThreads), 0, src,
+               c->permuted ? c->inv_d.as<const int>() : (const int *)nullptr, (long)n, c->D, c->Y.as<TV>());
+        launch(c, "fill", k_fill<TV>, dim3(fblk), dim3(kThreads), 0, c->uY.as<TV>(), (long)n, zero);
+        launch(c, "fill", k_fill<TV>, dim3(fblk), dim3(kThreads), 0, c->gains.as<TV>(), (long)n, (TV)1);
+        return sync_ctx(c);
+    };
+    TRY(c->precision == FITSNE_FP32 ? load(0.f) : load(0.0));
     c->mm_valid = c->mm_pending = false;
     c->have_grad = false;
     c->kcache = false;
@@ -2179,18 +2369,7 @@ extern "C" int fitsne_get_Y(fitsne_ctx *c, double *Y) {
     HIPTRY(hipSetDevice(c->device));
     TRY(check_graph(c));
     TRY(materialize(c));
-    TRY(sync_ctx(c));
-    const size_t n = (size_t)c->N * c->D;
-    if (c->precision == FITSNE_FP32) {
-        std::vector<float> y(n);
-        HIPTRY(hipMemcpy(y.data(), c->Y.p, sizeof(float) * n, hipMemcpyDeviceToHost));
-        const int D = c->D;
-        for (size_t r = 0; r < (size_t)c->N; r++)
-            for (int d = 0; d < D; d++) Y[(size_t)c->perm[r] * D + d] = y[r * D + d];
-    } else {
-        HIPTRY(hipMemcpy(Y, c->Y.p, sizeof(double) * n, hipMemcpyDeviceToHost));
-    }
-    return FITSNE_OK;
+    return rows_to_host(c, c->Y, Y);
 }
 
 extern "C" int fitsne_gradient(fitsne_ctx *c, double *dC, double *sum_Q) {
@@ -2198,19 +2377,7 @@ extern "C" int fitsne_gradient(fitsne_ctx *c, double *dC, double *sum_Q) {
     TRY(check_graph(c));
     TRY(run_pipeline(c, 0, nullptr));
     TRY(read_sumq(c, sum_Q));
-    if (dC) {
-        const size_t n = (size_t)c->N * c->D;
-        if (c->precision == FITSNE_FP32) {
-            std::vector<float> d(n);
-            HIPTRY(hipMemcpy(d.data(), c->dC.p, sizeof(float) * n, hipMemcpyDeviceToHost));
-            const int D = c->D;
-            for (size_t r = 0; r < (size_t)c->N; r++)
-                for (int e = 0; e < D; e++) dC[(size_t)c->perm[r] * D + e] = d[r * D + e];
-        } else {
-            HIPTRY(hipMemcpy(dC, c->dC.p, sizeof(double) * n, hipMemcpyDeviceToHost));
-        }
-    }
-    return FITSNE_OK;
+    return dC ? rows_to_host(c, c->dC, dC) : FITSNE_OK;
 }
 
 // ============================================================================ captured steps
@@ -3367,15 +3534,16 @@ extern "C" int fitsne_distances2similarities_batch(const double *D, double *P, i
     TRY(ensure(c->xs, sizeof(double) * n_points));
     TRY(ensure(c->ys, sizeof(double) * n_points));
     TRY(ensure(c->box, sizeof(int) * n_points));
-    HIPTRY(hipMemcpy(c->w.p, D, sizeof(double) * nk, hipMemcpyHostToDevice));
-    if (beta0) HIPTRY(hipMemcpy(c->ys.p, beta0, sizeof(double) * n_points, hipMemcpyHostToDevice));
+    TRY(copy_in(c, c->w.p, D, sizeof(double) * nk));
+    if (beta0) TRY(copy_in(c, c->ys.p, beta0, sizeof(double) * n_points));
     const long threads = (long)n_points * kWave;
     launch(c, "d2s", k_d2s, dim3(blocks_for(threads)), dim3(kThreads), 0, c->w.as<const double>(), c->V.as<double>(),
            n_points, K, perplexity, sigma, ifSquared, beta0 ? c->ys.as<const double>() : (const double *)nullptr,
            c->xs.as<double>(), c->box.as<int>(), 0, 0);
-    HIPTRY(hipMemcpyAsync(P, c->V.p, sizeof(double) * nk, hipMemcpyDeviceToHost, c->stream));
-    HIPTRY(hipMemcpyAsync(beta, c->xs.p, sizeof(double) * n_points, hipMemcpyDeviceToHost, c->stream));
-    if (iters) HIPTRY(hipMemcpyAsync(iters, c->box.p, sizeof(int) * n_points, hipMemcpyDeviceToHost, c->stream));
+    HIPTRY(hipGetLastError());
+    TRY(copy_out(c, P, c->V.p, sizeof(double) * nk));
+    TRY(copy_out(c, beta, c->xs.p, sizeof(double) * n_points));
+    if (iters) TRY(copy_out(c, iters, c->box.p, sizeof(int) * n_points));
     return sync_ctx(c);
 }
 
@@ -3388,8 +3556,9 @@ extern "C" int fitsne_symmetrize(const uint32_t *row_P, const uint32_t *col_P, c
         if (row_P[i + 1] < row_P[i]) return fail(FITSNE_E_ARG, "row_P must be non-decreasing");
     const long nnz = (long)row_P[N];
     if (nnz > (long)(INT32_MAX / 2)) return fail(FITSNE_E_UNSUPPORTED, "more than 2^30 entries");
-    for (long k = 0; k < nnz; k++)
-        if (col_P[k] >= (uint32_t)N) return fail(FITSNE_E_ARG, "col_P entry out of range");
+    bool out_of_range = false;
+    for (long k = 0; k < nnz; k++) out_of_range |= col_P[k] >= (uint32_t)N;
+    if (out_of_range) return fail(FITSNE_E_ARG, "col_P entry out of range");
     const int cbits = bits_for((unsigned long long)N - 1), rbits = bits_for((unsigned long long)N);
     const int ebits = bits_for((unsigned long long)std::max<long>(nnz - 1, 0));
     std::lock_guard<std::mutex> lk(g_mirror_mu);
@@ -3417,9 +3586,9 @@ extern "C" int fitsne_symmetrize(const uint32_t *row_P, const uint32_t *col_P, c
     TRY(ensure(c->sy_okeys2, sizeof(uint64_t) * 2 * ne));
     TRY(ensure(c->sy_scol, sizeof(uint32_t) * 2 * ne));
     TRY(ensure(c->sy_sval, sizeof(double) * 2 * ne));
-    HIPTRY(hipMemcpyAsync(c->sy_row.p, row_P, sizeof(uint32_t) * (N + 1), hipMemcpyHostToDevice, c->stream));
-    HIPTRY(hipMemcpyAsync(c->sy_col.p, col_P, sizeof(uint32_t) * ne, hipMemcpyHostToDevice, c->stream));
-    HIPTRY(hipMemcpyAsync(c->sy_val.p, val_P, sizeof(double) * ne, hipMemcpyHostToDevice, c->stream));
+    TRY(copy_in(c, c->sy_row.p, row_P, sizeof(uint32_t) * (N + 1)));
+    TRY(copy_in(c, c->sy_col.p, col_P, sizeof(uint32_t) * ne));
+    TRY(copy_in(c, c->sy_val.p, val_P, sizeof(double) * ne));
     HIPTRY(hipMemsetAsync(c->sy_cnt.p, 0, sizeof(int) * N, c->stream));
     const int gblk = std::min(blocks_for(nnz), 8192);
     launch(c, "sym_rows", k_entry_rows<uint32_t>, dim3(blocks_for((long)N * kWave)), dim3(kThreads), 0,
@@ -3450,13 +3619,10 @@ extern "C" int fitsne_symmetrize(const uint32_t *row_P, const uint32_t *col_P, c
            c->sy_col.as<const uint32_t>(), c->sy_val.as<const double>(), c->sy_partner.as<const int64_t>(),
            c->sy_scol.as<uint32_t>(), c->sy_sval.as<double>());
     HIPTRY(hipGetLastError());
-    std::vector<int> start((size_t)N + 1);
-    HIPTRY(hipMemcpyAsync(start.data(), c->sy_start.p, sizeof(int) * (N + 1), hipMemcpyDeviceToHost, c->stream));
-    TRY(sync_ctx(c));
-    const long M = start[N];
-    for (int i = 0; i <= N; i++) sym_row_P[i] = (uint32_t)start[i];
-    HIPTRY(hipMemcpy(sym_col_P, c->sy_scol.p, sizeof(uint32_t) * (size_t)M, hipMemcpyDeviceToHost));
-    HIPTRY(hipMemcpy(sym_val_P, c->sy_sval.p, sizeof(double) * (size_t)M, hipMemcpyDeviceToHost));
+    TRY(copy_out(c, sym_row_P, c->sy_start.p, sizeof(int) * ((size_t)N + 1)));
+    const long M = (long)sym_row_P[N];
+    TRY(copy_out(c, sym_col_P, c->sy_scol.p, sizeof(uint32_t) * (size_t)M));
+    TRY(copy_out(c, sym_val_P, c->sy_sval.p, sizeof(double) * (size_t)M));
     if (sym_nnz) *sym_nnz = M;
     return FITSNE_OK;
 }
@@ -3580,7 +3746,8 @@ static int knn_filtered(fitsne_ctx *c, const double *X, int N, int D, int K, int
     double *part = m.ptr<double>(oPart), *mean = m.ptr<double>(oMean);
     int *redo = m.ptr<int>(oR), *nr = redo + N, *di = m.ptr<int>(oI);
     double *dd = m.ptr<double>(oD);
-    HIPTRY(hipMemcpyAsync(m.ptr<double>(oX), X, sizeof(double) * nd, hipMemcpyHostToDevice, c->stream));
+    TRY(copy_in(c, m.ptr<double>(oX), X, sizeof(double) * nd));
+    TRY(need_finite(c, d.X, (long)nd, "X contains non-finite values"));
     launch(c, "fill", k_fill<int>, dim3(1), dim3(kWave), 0, nr, 1L, 0);
     launch(c, "fill", k_fill<int>, dim3(std::min(blocks_for(N), 1024)), dim3(kThreads), 0, d.cnt, (long)N, 0);
     launch(c, "knn_colsum", k_knn_colsum, dim3(cblk), dim3(256), 0, d.X, N, D, part);
@@ -3614,8 +3781,8 @@ static int knn_filtered(fitsne_ctx *c, const double *X, int N, int D, int K, int
     if (n < 0 || n > N) return fail(FITSNE_E_HIP, "inconsistent recompute count");
     KnnSlab xt;
     if (n > 0) TRY(knn_fp64(c, d.X, xt.b, N, D, K, di, dd, redo, n));
-    HIPTRY(hipMemcpyAsync(idx, di, sizeof(int) * nk, hipMemcpyDeviceToHost, c->stream));
-    HIPTRY(hipMemcpyAsync(dist, dd, sizeof(double) * nk, hipMemcpyDeviceToHost, c->stream));
+    TRY(copy_out(c, idx, di, sizeof(int) * nk));
+    TRY(copy_out(c, dist, dd, sizeof(double) * nk));
     TRY(sync_ctx(c));
     if (nredo) *nredo = n;
     return FITSNE_OK;
@@ -3628,21 +3795,16 @@ static int knn_args(const double *X, int N, int D, int K, const int32_t *idx, co
     return FITSNE_OK;
 }
 
-static int knn_finite(const double *X, size_t nd) {
-    for (size_t i = 0; i < nd; i++)
-        if (!std::isfinite(X[i])) return fail(FITSNE_E_ARG, "X contains non-finite values");
-    return FITSNE_OK;
-}
-
 // X up, the FP64 kernel over all queries, neighbours down.
 static int knn_plain(fitsne_ctx *c, const double *X, int N, int D, int K, int32_t *idx, double *dist) {
     TRY(ensure(c->knnX, sizeof(double) * (size_t)N * D));
     TRY(ensure(c->knnI, sizeof(int) * (size_t)N * K));
     TRY(ensure(c->knnD, sizeof(double) * (size_t)N * K));
-    HIPTRY(hipMemcpy(c->knnX.p, X, sizeof(double) * (size_t)N * D, hipMemcpyHostToDevice));
+    TRY(copy_in(c, c->knnX.p, X, sizeof(double) * (size_t)N * D));
+    TRY(need_finite(c, c->knnX.as<const double>(), (long)N * D, "X contains non-finite values"));
     TRY(knn_fp64(c, c->knnX.as<const double>(), c->knnXT, N, D, K, c->knnI.as<int>(), c->knnD.as<double>(), nullptr, N));
-    HIPTRY(hipMemcpyAsync(idx, c->knnI.p, sizeof(int) * (size_t)N * K, hipMemcpyDeviceToHost, c->stream));
-    HIPTRY(hipMemcpyAsync(dist, c->knnD.p, sizeof(double) * (size_t)N * K, hipMemcpyDeviceToHost, c->stream));
+    TRY(copy_out(c, idx, c->knnI.p, sizeof(int) * (size_t)N * K));
+    TRY(copy_out(c, dist, c->knnD.p, sizeof(double) * (size_t)N * K));
     return sync_ctx(c);
 }
 
@@ -3656,7 +3818,6 @@ constexpr long kKnnFilterWork = 150000;
 
 extern "C" int fitsne_knn_exact(const double *X, int N, int D, int K, int32_t *idx, double *dist) {
     TRY(knn_args(X, N, D, K, idx, dist));
-    TRY(knn_finite(X, (size_t)N * D));
     std::lock_guard<std::mutex> lk(g_mirror_mu);
     fitsne_ctx *c;
     TRY(mirror_ctx(&c, 1, 3, 1.0, 1, 1.0));
@@ -3671,7 +3832,6 @@ extern "C" int fitsne_knn_mfma(const double *X, int N, int D, int K, int32_t *id
     TRY(knn_args(X, N, D, K, idx, dist));
     if (D > kKmMaxD) return fail(FITSNE_E_UNSUPPORTED, "the MFMA kNN takes D <= 128 (use fitsne_knn_exact)");
     if (K > kKmMaxK) return fail(FITSNE_E_UNSUPPORTED, "the MFMA kNN takes K <= 256 (use fitsne_knn_exact)");
-    TRY(knn_finite(X, (size_t)N * D));
     std::lock_guard<std::mutex> lk(g_mirror_mu);
     fitsne_ctx *c;
     TRY(mirror_ctx(&c, 1, 3, 1.0, 1, 1.0));
