@@ -653,12 +653,46 @@ static auto pick_spread_f32(int p) -> decltype(&k_spread_f32<3, D>) {
     }
 }
 template <int D>
+static auto pick_spread_wave(int p) -> decltype(&k_spread_wave<3, D>) {
+    switch (p) {
+    case 2: return k_spread_wave<2, D>;
+    case 3: return k_spread_wave<3, D>;
+    case 4: return k_spread_wave<4, D>;
+    default: return k_spread_wave<5, D>;
+    }
+}
+template <int D>
 static auto pick_spread_f32_v(int p) -> decltype(&k_spread_f32_v<3, D>) {
     switch (p) {
     case 2: return k_spread_f32_v<2, D>;
     case 3: return k_spread_f32_v<3, D>;
     case 4: return k_spread_f32_v<4, D>;
     default: return k_spread_f32_v<5, D>;
+    }
+}
+static auto pick_spread_kern(int p) -> decltype(&k_spread_kern<3, kKernTot>) {
+    switch (p) {
+    case 2: return k_spread_kern<2, kKernTot>;
+    case 3: return k_spread_kern<3, kKernTot>;
+    case 4: return k_spread_kern<4, kKernTot>;
+    default: return k_spread_kern<5, kKernTot>;
+    }
+}
+static size_t spread_wave_lds(int p) {
+    switch (p) {
+    case 2: return sizeof(SpreadWaveLds<2, 2>);
+    case 3: return sizeof(SpreadWaveLds<3, 2>);
+    case 4: return sizeof(SpreadWaveLds<4, 2>);
+    default: return sizeof(SpreadWaveLds<5, 2>);
+    }
+}
+template <int D>
+static auto pick_spread_wave_v(int p) -> decltype(&k_spread_wave_v<3, D>) {
+    switch (p) {
+    case 2: return k_spread_wave_v<2, D>;
+    case 3: return k_spread_wave_v<3, D>;
+    case 4: return k_spread_wave_v<4, D>;
+    default: return k_spread_wave_v<5, D>;
     }
 }
 template <int D>
@@ -972,20 +1006,13 @@ static int launch_f32_stages(fitsne_ctx *c, const cx<float> *tw, const StageDims
                    c->K1.as<float>(), c->KS.as<float>(), c->KT.as<float>());
         }
     };
-    const bool kside = D == 2 && kern && side && c->overlap;
-    if (kside) {
-        // the spectra read the record (by value with hv) and the twiddles: wait for the stream only when
-        // it wrote either in this step
-        if (!hv || c->tw_fresh) {
-            HIPTRY(hipEventRecord(c->geo_ev, c->stream));
-            HIPTRY(hipStreamWaitEvent(c->astream, c->geo_ev, 0));
-        }
-        hipStream_t main = c->stream;
-        c->stream = c->astream;
-        kernel_spectra();
-        c->stream = main;
-        HIPTRY(hipEventRecord(c->kern_ev, c->astream));
-    }
+    const bool waves = N < kSpreadWaveN;
+    const bool fused = D == 2 && kern && hv && waves;  // passes of a small embedding's step share launches
+    const bool kside = D == 2 && kern && side && c->overlap && !fused;
+    // the spectra read the record (by value with hv) and the twiddles: wait for the stream only when it wrote
+    // either in this step
+    const bool kwait = kside && (!hv || c->tw_fresh);
+    if (kwait) HIPTRY(hipEventRecord(c->geo_ev, c->stream));
     // 1D: the kernel line (its spectra depend only on the geometry record and the twiddles) on the third
     // stream, after the work queued so far on the grid stages' stream (the twiddle table, the last
     // convolution's read of kline)
@@ -1003,20 +1030,42 @@ static int launch_f32_stages(fitsne_ctx *c, const cx<float> *tw, const StageDims
         HIPTRY(hipEventRecord(c->kl_ev, c->kstream));
     }
     c->tw_fresh = false;
-    const int pts = c->spread_pts;
-    if (hv) {
-        launch(c, "spread_f32", pick_spread_f32_v<D>(p), dim3((N + pts - 1) / pts), dim3(kSpreadThreads), 0,
+    const int pts = waves ? 2 * kWave : c->spread_pts;
+    const dim3 sgrid((N + pts - 1) / pts), sblk(waves ? kWave : kSpreadThreads);
+    if (fused) {
+        const size_t Mp = (size_t)sd.Mp, lines = sizeof(cx<float>) * (lspan<true>((int)Mp) + Mp);
+        const int per = 2 * kSpreadThreads;
+        launch(c, "spread_kern", pick_spread_kern(p), dim3(sd.gr_rows + (N + per - 1) / per), dim3(kSpreadThreads),
+               std::max(lines, spread_wave_lds(p) * (kSpreadThreads / kWave)), c->Y.as<const float>(), N, *hv,
+               c->dgeo.as<DevGeo>(), c->fixgrid.as<unsigned long long>(), ctr, sd.gr_rows, tw, kind_q, kind_1, c->df,
+               c->Trow.as<cx<float>>());
+    } else if (hv)
+        launch(c, "spread_f32", waves ? pick_spread_wave_v<D>(p) : pick_spread_f32_v<D>(p), sgrid, sblk, 0,
                c->Y.as<const float>(), N, pts, *hv, c->dgeo.as<DevGeo>(), c->fixgrid.as<unsigned long long>(), ctr);
-    } else {
-        launch(c, "spread_f32", pick_spread_f32<D>(p), dim3((N + pts - 1) / pts), dim3(kSpreadThreads), 0,
+    else
+        launch(c, "spread_f32", waves ? pick_spread_wave<D>(p) : pick_spread_f32<D>(p), sgrid, sblk, 0,
                c->Y.as<const float>(), N, pts, dg, c->fixgrid.as<unsigned long long>(), ctr);
+    if (kside) {  // after the spread, whose launch the grid stages wait for
+        if (kwait) HIPTRY(hipStreamWaitEvent(c->astream, c->geo_ev, 0));
+        hipStream_t main = c->stream;
+        c->stream = c->astream;
+        kernel_spectra();
+        c->stream = main;
+        HIPTRY(hipEventRecord(c->kern_ev, c->astream));
     }
     if constexpr (D == 2) {
         const size_t Mp = (size_t)sd.Mp;
-        if (kern && !kside) kernel_spectra();
-        launch(c, "rows_fwd", k_rows_fwd<float, kRowThreads, kRowTot, true>, dim3(sd.gr_rows), dim3(kRowThreads),
-               sizeof(cx<float>) * (lspan<true>(2 * (int)Mp) + Mp), dg, tw, (const float *)nullptr, 4, 4, c->spec.as<cx<float>>(),
-               c->fixgrid.as<unsigned long long>());
+        if (kern && !kside && !fused) kernel_spectra();
+        if (fused)
+            launch(c, "rows_kern", k_rows_kern<kRowThreads, kRowTot, kKernTot>, dim3(sd.gr_rows + sd.gr_cols),
+                   dim3(kRowThreads), sizeof(cx<float>) * (lspan<true>(2 * (int)Mp) + Mp), dg, tw,
+                   c->spec.as<cx<float>>(), c->fixgrid.as<unsigned long long>(), sd.gr_rows,
+                   c->Trow.as<const cx<float>>(), c->KQ.as<float>(), c->K1.as<float>(), c->KS.as<float>(),
+                   c->KT.as<float>());
+        else
+            launch(c, "rows_fwd", k_rows_fwd<float, kRowThreads, kRowTot, true>, dim3(sd.gr_rows), dim3(kRowThreads),
+                   sizeof(cx<float>) * (lspan<true>(2 * (int)Mp) + Mp), dg, tw, (const float *)nullptr, 4, 4,
+                   c->spec.as<cx<float>>(), c->fixgrid.as<unsigned long long>());
         if (kside) {
             // kern_ev follows the attractive kernel on the side stream, so this one wait also joins it:
             // each cross-stream wait costs about 10 us of queue latency, even on a finished event
@@ -1141,7 +1190,8 @@ static int pipeline_f32(fitsne_ctx *c, int mode, const fitsne_step_params *sp) {
     const DevGeo *live;
     TRY(live_record(c, &live));
     // 2D: the attractive term on the second stream (after everything queued so far), beside the grid
-    // stages; the interpolation waits for it.
+    // stages; the interpolation waits for it.  A small embedding's stays on the main stream, where it runs
+    // while the host plans the grid.
     // The second stream is made on first use: contexts that only run captured or batched steps never
     // create it, so their streams alone share the device's hardware queues (a second stream per context
     // measured a third fewer batched iterations).
@@ -1167,7 +1217,7 @@ static int pipeline_f32(fitsne_ctx *c, int mode, const fitsne_step_params *sp) {
         TRY((launch_attractive<float, D>(c, (float)c->exag, c->pos.as<float>(), live, false, ctr)));
         c->swap_main = c->stream;
         c->stream = c->astream;
-    } else if (c->overlap) {
+    } else if (c->overlap && c->N >= kSpreadWaveN) {
         if (!c->astream) HIPTRY(hipStreamCreateWithFlags(&c->astream, hipStreamNonBlocking));
         HIPTRY(hipEventRecord(c->fork_ev, c->stream));
         HIPTRY(hipStreamWaitEvent(c->astream, c->fork_ev, 0));
@@ -1246,6 +1296,7 @@ constexpr float kSpreadGain = 0.97f;
 template <int D>
 static int tune_spread(fitsne_ctx *c) {
     const int N = c->N;
+    if (N < kSpreadWaveN) return FITSNE_OK;  // one form whatever the workgroup
     double mn, mx;
     TRY(current_minmax<float>(c, &mn, &mx));
     Geo g;

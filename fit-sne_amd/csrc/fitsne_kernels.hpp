@@ -1000,12 +1000,97 @@ __device__ __forceinline__ int point_charges(const float (&y)[D], const Geo &g, 
     return box;
 }
 
+// The points i and i + 1 (i even, this lane's place in the wavefront's 128) of the spread: charges summed
+// over the runs of one box, each run's sum given to flush(on, box, values).  Each lane takes two consecutive
+// points, a and b, so a wavefront covers 128 points and its scan and flush serve twice as many points.  A
+// lane's running sum is that of b's box: a joins it when both share a box; otherwise a joins the left
+// neighbour's sum when it continues that lane's b box, and is flushed on its own in the rare remaining case
+// (a box holding a alone between two others).  Runs of lanes with the same b box are summed by the segmented
+// scan, and each run's last lane flushes.
+template <int P, int D, typename F>
+__device__ __forceinline__ void spread_pairs(const float *__restrict__ Y, int N, long i, const Geo &g,
+                                             const double *__restrict__ ctr, F flush) {
+    constexpr int NV = (D == 2 ? P * P : P), NQ = (D == 2 ? 4 : 3);
+    const int lane = threadIdx.x % kWave;
+    float ya[D], yb[D];
+    const bool oka = i < N, okb = i + 1 < N;
+    if (okb) {
+        if constexpr (D == 2) {
+            const float4 v = reinterpret_cast<const float4 *>(Y)[i >> 1];
+            ya[0] = v.x;
+            ya[1] = v.y;
+            yb[0] = v.z;
+            yb[1] = v.w;
+        } else {
+            const float2 v = reinterpret_cast<const float2 *>(Y)[i >> 1];
+            ya[0] = v.x;
+            yb[0] = v.y;
+        }
+    } else if (oka) {
+        load_pt<float, D>(Y, i, ya);
+    }
+    if (ctr) {  // pending centring (uniform branch)
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            ya[d] = oka ? centred(ya[d], ctr[d]) : 0.f;
+            yb[d] = okb ? centred(yb[d], ctr[d]) : 0.f;
+        }
+    }
+    float val[NV][NQ];
+#pragma unroll
+    for (int v = 0; v < NV; v++)
+#pragma unroll
+        for (int q = 0; q < NQ; q++) val[v][q] = 0.f;
+    // boxes (lanes past N: distinct negative keys, never a real box or run)
+    int ka = -1 - 2 * lane, kb = -2 - 2 * lane;
+    if (oka) ka = point_charges<P, D>(ya, g, val);
+    if (okb) {
+        double tb;
+        kb = box_coord<D>((double)yb[0], g, tb);
+        if constexpr (D == 2) kb += box_coord<D>((double)yb[1], g, tb) * g.nb;
+    }
+    const int kb_prev = __shfl_up(kb, 1, kWave), ka_next = __shfl_down(ka, 1, kWave),
+              kb_next = __shfl_down(kb, 1, kWave);
+    const bool pure = ka == kb;                                          // a is in b's box
+    const bool give = !pure && lane > 0 && ka == kb_prev;                // a continues the left lane's box
+    const bool take = lane < kWave - 1 && ka_next == kb && ka_next != kb_next;  // the right lane's a is ours
+    if (__ballot(oka && !pure && !give)) flush(oka && !pure && !give, ka, val);
+    // a's charges: kept (pure), moved one lane to the left (give / take), or already flushed
+#pragma unroll
+    for (int v = 0; v < NV; v++)
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            const float right = __int_as_float(
+                __builtin_amdgcn_update_dpp(0, __float_as_int(val[v][q]), 0x130, 0xf, 0xf, false));  // wave_shl:1
+            const float own = pure ? val[v][q] : 0.f;
+            val[v][q] = take ? own + right : own;
+        }
+    if (okb) {
+        float vb[NV][NQ];
+        (void)point_charges<P, D>(yb, g, vb);
+#pragma unroll
+        for (int v = 0; v < NV; v++)
+#pragma unroll
+            for (int q = 0; q < NQ; q++) val[v][q] += vb[v][q];
+    }
+    // runs of equal b boxes among consecutive lanes: a segmented inclusive scan over the wave (DPP row
+    // shifts and row broadcasts, in the VALU) leaves each run's sum in its last lane.  The wave's
+    // points and their order are fixed, so the float sums are bitwise repeatable.
+    const bool head = lane == 0 || kb != kb_prev;
+    const unsigned long long heads = __ballot(head);
+    const int run = __popcll(heads & ((2ull << lane) - 1ull));  // 1-based run of this lane
+    seg_scan_step<0x111, 0xf, NV, NQ>(val, run);  // row_shr:1
+    seg_scan_step<0x112, 0xf, NV, NQ>(val, run);  // row_shr:2
+    seg_scan_step<0x114, 0xf, NV, NQ>(val, run);  // row_shr:4
+    seg_scan_step<0x118, 0xf, NV, NQ>(val, run);  // row_shr:8
+    seg_scan_step<0x142, 0xa, NV, NQ>(val, run);  // row_bcast:15 into rows 1 and 3
+    seg_scan_step<0x143, 0xc, NV, NQ>(val, run);  // row_bcast:31 into rows 2 and 3
+    const bool tail = lane == kWave - 1 || kb != kb_next;
+    flush(tail && kb >= 0, kb, val);
+}
+
 // Workgroup `bid` of the spread (points [bid pts, (bid + 1) pts)); the body of k_spread_f32 and of its
-// batched form.  Each lane takes two consecutive points, a and b, so a wavefront covers 128 points and
-// its scan and flush serve twice as many points.  A lane's running sum is that of b's box: a joins it
-// when both share a box; otherwise a joins the left neighbour's sum when it continues that lane's b
-// box, and is flushed on its own in the rare remaining case (a box holding a alone between two others).
-// Runs of lanes with the same b box are summed by the segmented scan, and each run's last lane flushes.
+// batched form.
 template <int P, int D>
 __device__ __forceinline__ void spread_block(const float *__restrict__ Y, int N, int pts, const DevGeo *__restrict__ dg,
                                              unsigned long long *__restrict__ grid, int bid, SpreadLds<P, D> &L,
@@ -1016,7 +1101,7 @@ __device__ __forceinline__ void spread_block(const float *__restrict__ Y, int N,
     int *tkey = L.tkey;
     auto &tval = L.tval;
     const Geo &g = dg->g;
-    const int t = threadIdx.x, lane = t % kWave;
+    const int t = threadIdx.x;
     for (int o = t; o < NS; o += kSpreadThreads) tkey[o] = -1;
     for (int o = t; o < NS * NV * NQ; o += kSpreadThreads) (&tval[0][0])[o] = 0ull;
     __syncthreads();
@@ -1062,84 +1147,8 @@ __device__ __forceinline__ void spread_block(const float *__restrict__ Y, int N,
             }
         }
     };
-    for (int chunk = 0; chunk < pts / (2 * kSpreadThreads); chunk++) {
-        const long i = (long)bid * pts + (long)chunk * 2 * kSpreadThreads + 2 * (long)t;  // point a; b = i + 1
-        float ya[D], yb[D];
-        const bool oka = i < N, okb = i + 1 < N;
-        if (okb) {
-            if constexpr (D == 2) {
-                const float4 v = reinterpret_cast<const float4 *>(Y)[i >> 1];
-                ya[0] = v.x;
-                ya[1] = v.y;
-                yb[0] = v.z;
-                yb[1] = v.w;
-            } else {
-                const float2 v = reinterpret_cast<const float2 *>(Y)[i >> 1];
-                ya[0] = v.x;
-                yb[0] = v.y;
-            }
-        } else if (oka) {
-            load_pt<float, D>(Y, i, ya);
-        }
-        if (ctr) {  // pending centring (uniform branch)
-#pragma unroll
-            for (int d = 0; d < D; d++) {
-                ya[d] = oka ? centred(ya[d], ctr[d]) : 0.f;
-                yb[d] = okb ? centred(yb[d], ctr[d]) : 0.f;
-            }
-        }
-        float val[NV][NQ];
-#pragma unroll
-        for (int v = 0; v < NV; v++)
-#pragma unroll
-            for (int q = 0; q < NQ; q++) val[v][q] = 0.f;
-        // boxes (lanes past N: distinct negative keys, never a real box or run)
-        int ka = -1 - 2 * lane, kb = -2 - 2 * lane;
-        if (oka) ka = point_charges<P, D>(ya, g, val);
-        if (okb) {
-            double tb;
-            kb = box_coord<D>((double)yb[0], g, tb);
-            if constexpr (D == 2) kb += box_coord<D>((double)yb[1], g, tb) * g.nb;
-        }
-        const int kb_prev = __shfl_up(kb, 1, kWave), ka_next = __shfl_down(ka, 1, kWave),
-                  kb_next = __shfl_down(kb, 1, kWave);
-        const bool pure = ka == kb;                                          // a is in b's box
-        const bool give = !pure && lane > 0 && ka == kb_prev;                // a continues the left lane's box
-        const bool take = lane < kWave - 1 && ka_next == kb && ka_next != kb_next;  // the right lane's a is ours
-        if (__ballot(oka && !pure && !give)) flush(oka && !pure && !give, ka, val);
-        // a's charges: kept (pure), moved one lane to the left (give / take), or already flushed
-#pragma unroll
-        for (int v = 0; v < NV; v++)
-#pragma unroll
-            for (int q = 0; q < NQ; q++) {
-                const float right = __int_as_float(
-                    __builtin_amdgcn_update_dpp(0, __float_as_int(val[v][q]), 0x130, 0xf, 0xf, false));  // wave_shl:1
-                const float own = pure ? val[v][q] : 0.f;
-                val[v][q] = take ? own + right : own;
-            }
-        if (okb) {
-            float vb[NV][NQ];
-            (void)point_charges<P, D>(yb, g, vb);
-#pragma unroll
-            for (int v = 0; v < NV; v++)
-#pragma unroll
-                for (int q = 0; q < NQ; q++) val[v][q] += vb[v][q];
-        }
-        // runs of equal b boxes among consecutive lanes: a segmented inclusive scan over the wave (DPP row
-        // shifts and row broadcasts, in the VALU) leaves each run's sum in its last lane.  The wave's
-        // points and their order are fixed, so the float sums are bitwise repeatable.
-        const bool head = lane == 0 || kb != kb_prev;
-        const unsigned long long heads = __ballot(head);
-        const int run = __popcll(heads & ((2ull << lane) - 1ull));  // 1-based run of this lane
-        seg_scan_step<0x111, 0xf, NV, NQ>(val, run);  // row_shr:1
-        seg_scan_step<0x112, 0xf, NV, NQ>(val, run);  // row_shr:2
-        seg_scan_step<0x114, 0xf, NV, NQ>(val, run);  // row_shr:4
-        seg_scan_step<0x118, 0xf, NV, NQ>(val, run);  // row_shr:8
-        seg_scan_step<0x142, 0xa, NV, NQ>(val, run);  // row_bcast:15 into rows 1 and 3
-        seg_scan_step<0x143, 0xc, NV, NQ>(val, run);  // row_bcast:31 into rows 2 and 3
-        const bool tail = lane == kWave - 1 || kb != kb_next;
-        flush(tail && kb >= 0, kb, val);
-    }
+    for (int chunk = 0; chunk < pts / (2 * kSpreadThreads); chunk++)
+        spread_pairs<P, D>(Y, N, (long)bid * pts + (long)chunk * 2 * kSpreadThreads + 2 * (long)t, g, ctr, flush);
     __syncthreads();
     // table -> grid
     for (int o = t; o < NS * NV * NQ; o += kSpreadThreads) {
@@ -1177,6 +1186,79 @@ __global__ __launch_bounds__(kSpreadThreads) __attribute__((amdgpu_waves_per_eu(
     if (blockIdx.x == 0 && threadIdx.x == 0) *out = v;
     if (!v.live) return;
     spread_block<P, D>(Y, N, pts, &v, grid, blockIdx.x, L, ctr);
+}
+
+// LDS of one k_spread_wave wavefront: the sums of its runs of one flush, a row of values each (odd stride).
+template <int P, int D>
+struct SpreadWaveLds {
+    static constexpr int NV = (D == 2 ? P * P : P), NQ = (D == 2 ? 4 : 3), ROW = (NV * NQ) | 1;
+    float val[kWave][ROW];
+    int box[kWave];
+};
+
+// Below this many points the spread goes straight into the grid, a wavefront to a workgroup (spread_wave), else over the
+// workgroups' tables.  A table pays where workgroups are many and their boxes few; a small embedding gives
+// either too few workgroups (2 of 1024 points at N = 2,000) or more boxes than the table has slots, whose every probe
+// walks the whole table.  Launch to end, 2D, 3 nodes, table of 1024 and of 512 points, and this: N = 2,000
+// 74, 42, 18 us; 70,000 (5,625 boxes) 19, 13, 12 and (6,400 boxes) 35, 19, 15; 140,000 18, 14, 14 and 34, 17, 16;
+// 300,000 20, 16, 22 and 41, 18, 23; a million 29, 29, 62.  1D: 2,000 9.6, 7.5, 7.5; 70,000 8.9, 7.0, 5.9.
+constexpr int kSpreadWaveN = 150000;
+
+// The 128 points of wavefront `bid`, straight into the grid: each flush puts the runs' sums into LDS, and the lanes
+// add them value by value, so that the 4 NV values of a run are a few neighbouring pieces of the grid in one
+// instruction.  The runs and their order are those of spread_block, and so the grid is the same to the bit.
+template <int P, int D>
+__device__ __forceinline__ void spread_wave(const float *__restrict__ Y, int N, const DevGeo *__restrict__ dg,
+                                            unsigned long long *__restrict__ grid, int bid, SpreadWaveLds<P, D> &L,
+                                            const double *__restrict__ ctr) {
+    constexpr int NV = SpreadWaveLds<P, D>::NV, NQ = SpreadWaveLds<P, D>::NQ, NE = NV * NQ;
+    const Geo &g = dg->g;
+    const int lane = threadIdx.x % kWave;
+    spread_pairs<P, D>(Y, N, (long)bid * 2 * kWave + 2 * lane, g, ctr,
+                       [&](bool on, int box, const float (&val)[NV][NQ]) {
+        const unsigned long long who = __ballot(on);
+        const int n = __popcll(who), at = __popcll(who & ((1ull << lane) - 1ull));
+        if (on) {
+            L.box[at] = box;
+#pragma unroll
+            for (int v = 0; v < NV; v++)
+#pragma unroll
+                for (int q = 0; q < NQ; q++) L.val[at][v * NQ + q] = val[v][q];
+        }
+        __threadfence_block();  // the wavefront's own LDS writes, read by its other lanes
+        __builtin_amdgcn_wave_barrier();
+        for (int e = lane; e < n * NE; e += kWave) {
+            const int r = e / NE, k = e - r * NE, v = k / NQ, q = k - v * NQ, b = L.box[r];
+            const int by = D == 2 ? b / g.nb : 0, bx = b - by * g.nb;
+            const long node = D == 2 ? (long)(bx * P + v / P) * g.n1d + by * P + v % P : (long)b * P + v;
+            const double x = (double)L.val[r][k] * g.fix;
+            atomicAdd(&grid[node * 4 + q], (unsigned long long)(g.fix_fast ? fix_rn(x) : fix_rn_any(x)));
+        }
+        __threadfence_block();
+        __builtin_amdgcn_wave_barrier();
+    });
+}
+
+// k_spread_f32 and k_spread_f32_v by spread_wave, one wavefront to a workgroup.
+template <int P, int D>
+__global__ __launch_bounds__(kWave) void k_spread_wave(const float *__restrict__ Y, int N, int,
+                                                       const DevGeo *__restrict__ dg,
+                                                       unsigned long long *__restrict__ grid,
+                                                       const double *__restrict__ ctr) {
+    __shared__ SpreadWaveLds<P, D> L;
+    if (!dg->live) return;
+    spread_wave<P, D>(Y, N, dg, grid, blockIdx.x, L, ctr);
+}
+
+template <int P, int D>
+__global__ __launch_bounds__(kWave) void k_spread_wave_v(const float *__restrict__ Y, int N, int, const DevGeo v,
+                                                         DevGeo *__restrict__ out,
+                                                         unsigned long long *__restrict__ grid,
+                                                         const double *__restrict__ ctr) {
+    __shared__ SpreadWaveLds<P, D> L;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *out = v;
+    if (!v.live) return;
+    spread_wave<P, D>(Y, N, &v, grid, blockIdx.x, L, ctr);
 }
 
 // int64 grid -> float4 (A, c, b_x, b_y) and clear, for the 1D path (the 2D row FFT does this itself).
@@ -1236,7 +1318,8 @@ __device__ __forceinline__ void kern_rows_line(const DevGeo *__restrict__ dg, cx
 
 template <typename T, int NTHR, int MAXTOT, bool PAD>
 __device__ __forceinline__ void kern_rows_body(const DevGeo *__restrict__ dg, const cx<T> *__restrict__ tw,
-                                               int kind_q, int kind_1, double df, cx<T> *__restrict__ Trow) {
+                                               int kind_q, int kind_1, double df, cx<T> *__restrict__ Trow, int bid,
+                                               int nblk) {
     if (!dg->live || !dg->kspec_stale) return;
     const Geo &g = dg->g;
     extern __shared__ unsigned char smem_raw[];
@@ -1244,7 +1327,7 @@ __device__ __forceinline__ void kern_rows_body(const DevGeo *__restrict__ dg, co
     const int Mp = g.Mp, n1d = g.n1d;
     const cx<T> *twl = stage_twiddles(buf + lspan<PAD>(Mp), tw, Mp);
     const int npad = 8 * ((n1d + 7) / 8);
-    for (int slot = blockIdx.x; slot < npad; slot += gridDim.x) {
+    for (int slot = bid; slot < npad; slot += nblk) {
         const int a = xcd_slot_row(slot, n1d);
         if (a >= n1d) continue;
         kern_rows_line<T, NTHR, MAXTOT, PAD>(dg, buf, twl, kind_q, kind_1, df, Trow, a);
@@ -1254,7 +1337,7 @@ __device__ __forceinline__ void kern_rows_body(const DevGeo *__restrict__ dg, co
 template <typename T, int NTHR, int MAXTOT, bool PAD = false>
 __global__ __launch_bounds__(NTHR) void k_kern_rows(const DevGeo *__restrict__ dg, const cx<T> *__restrict__ tw,
                                                     int kind_q, int kind_1, double df, cx<T> *__restrict__ Trow) {
-    kern_rows_body<T, NTHR, MAXTOT, PAD>(dg, tw, kind_q, kind_1, df, Trow);
+    kern_rows_body<T, NTHR, MAXTOT, PAD>(dg, tw, kind_q, kind_1, df, Trow, blockIdx.x, gridDim.x);
 }
 
 // The same with a host-planned geometry record passed by value, so that the pass need not wait for the
@@ -1262,7 +1345,7 @@ __global__ __launch_bounds__(NTHR) void k_kern_rows(const DevGeo *__restrict__ d
 template <typename T, int NTHR, int MAXTOT, bool PAD = false>
 __global__ __launch_bounds__(NTHR) void k_kern_rows_v(const DevGeo v, const cx<T> *__restrict__ tw, int kind_q,
                                                       int kind_1, double df, cx<T> *__restrict__ Trow) {
-    kern_rows_body<T, NTHR, MAXTOT, PAD>(&v, tw, kind_q, kind_1, df, Trow);
+    kern_rows_body<T, NTHR, MAXTOT, PAD>(&v, tw, kind_q, kind_1, df, Trow, blockIdx.x, gridDim.x);
 }
 
 // buf[q] = f(q) for q < total, the loads of a thread issued eight at a time before their LDS writes, so
@@ -1350,7 +1433,8 @@ __device__ __forceinline__ void kern_cols_line(const DevGeo *__restrict__ dg, cx
 template <typename T, int NTHR, int MAXTOT, bool PAD>
 __device__ __forceinline__ void kern_cols_body(const DevGeo *__restrict__ dg, const cx<T> *__restrict__ tw,
                                                const cx<T> *__restrict__ Trow, int need_s, T *__restrict__ KQ,
-                                               T *__restrict__ K1, T *__restrict__ KS, T *__restrict__ KT) {
+                                               T *__restrict__ K1, T *__restrict__ KS, T *__restrict__ KT, int bid,
+                                               int nblk) {
     if (!dg->live || !dg->kspec_stale) return;
     const Geo &g = dg->g;
     extern __shared__ unsigned char smem_raw[];
@@ -1358,7 +1442,7 @@ __device__ __forceinline__ void kern_cols_body(const DevGeo *__restrict__ dg, co
     const int Mp = g.Mp, H = g.H;
     const cx<T> *twl = stage_twiddles(buf + lspan<PAD>(Mp), tw, Mp);
     const int npad = 8 * ((H + 7) / 8);
-    for (int slot = blockIdx.x; slot < npad; slot += gridDim.x) {
+    for (int slot = bid; slot < npad; slot += nblk) {
         const int k = xcd_slot_row(slot, H);
         if (k >= H) continue;
         kern_cols_line<T, NTHR, MAXTOT, PAD>(dg, buf, twl, Trow, need_s, KQ, K1, KS, KT, k);
@@ -1370,7 +1454,7 @@ __global__ __launch_bounds__(NTHR) void k_kern_cols(const DevGeo *__restrict__ d
                                                     const cx<T> *__restrict__ Trow, int need_s,
                                                     T *__restrict__ KQ, T *__restrict__ K1, T *__restrict__ KS,
                                                     T *__restrict__ KT) {
-    kern_cols_body<T, NTHR, MAXTOT, PAD>(dg, tw, Trow, need_s, KQ, K1, KS, KT);
+    kern_cols_body<T, NTHR, MAXTOT, PAD>(dg, tw, Trow, need_s, KQ, K1, KS, KT, blockIdx.x, gridDim.x);
 }
 
 template <typename T, int NTHR, int MAXTOT, bool PAD = false>
@@ -1378,7 +1462,7 @@ __global__ __launch_bounds__(NTHR) void k_kern_cols_v(const DevGeo v, const cx<T
                                                       const cx<T> *__restrict__ Trow, int need_s,
                                                       T *__restrict__ KQ, T *__restrict__ K1, T *__restrict__ KS,
                                                       T *__restrict__ KT) {
-    kern_cols_body<T, NTHR, MAXTOT, PAD>(&v, tw, Trow, need_s, KQ, K1, KS, KT);
+    kern_cols_body<T, NTHR, MAXTOT, PAD>(&v, tw, Trow, need_s, KQ, K1, KS, KT, blockIdx.x, gridDim.x);
 }
 
 // Row FFT, forward.  grid: [n1d][n1d][sin] real (u = x node, v = y node); terms 2l, 2l+1 packed as
@@ -1430,11 +1514,11 @@ __device__ __forceinline__ void rows_fwd_line(const DevGeo *__restrict__ dg, cx<
     __syncthreads();
 }
 
-template <typename T, int NTHR, int MAXTOT, bool PAD = false>
-__global__ __launch_bounds__(NTHR) void k_rows_fwd(const DevGeo *__restrict__ dg, const cx<T> *__restrict__ tw,
-                                                   const T *__restrict__ grid, int sin, int nterms,
-                                                   cx<T> *__restrict__ spec,
-                                                   unsigned long long *__restrict__ fixgrid) {
+template <typename T, int NTHR, int MAXTOT, bool PAD>
+__device__ __forceinline__ void rows_fwd_body(const DevGeo *__restrict__ dg, const cx<T> *__restrict__ tw,
+                                              const T *__restrict__ grid, int sin, int nterms,
+                                              cx<T> *__restrict__ spec, unsigned long long *__restrict__ fixgrid,
+                                              int bid, int nblk) {
     if (!dg->live) return;
     const Geo &g = dg->g;
     extern __shared__ unsigned char smem_raw[];
@@ -1443,11 +1527,60 @@ __global__ __launch_bounds__(NTHR) void k_rows_fwd(const DevGeo *__restrict__ dg
     const int lines = (nterms + 1) / 2;
     const cx<T> *twl = stage_twiddles(buf + lspan<PAD>(lines * Mp), tw, Mp);
     const int npad = 8 * ((n1d + 7) / 8);
-    for (int slot = blockIdx.x; slot < npad; slot += gridDim.x) {
+    for (int slot = bid; slot < npad; slot += nblk) {
         const int u = xcd_slot_row(slot, n1d);
         if (u >= n1d) continue;
         rows_fwd_line<T, NTHR, MAXTOT, PAD>(dg, buf, twl, grid, sin, nterms, spec, fixgrid, u);
     }
+}
+
+template <typename T, int NTHR, int MAXTOT, bool PAD = false>
+__global__ __launch_bounds__(NTHR) void k_rows_fwd(const DevGeo *__restrict__ dg, const cx<T> *__restrict__ tw,
+                                                   const T *__restrict__ grid, int sin, int nterms,
+                                                   cx<T> *__restrict__ spec,
+                                                   unsigned long long *__restrict__ fixgrid) {
+    rows_fwd_body<T, NTHR, MAXTOT, PAD>(dg, tw, grid, sin, nterms, spec, fixgrid, blockIdx.x, gridDim.x);
+}
+
+// ---- a small embedding's step (2D, below kSpreadWaveN points): its passes are bound by latency, not by work, so passes that
+// do not depend on each other share a launch and the step stays on one stream (each wait for another stream costs
+// about 10 us).  With the attractive term and the spectra on the second stream 20 steps of 2,000 points took
+// 2.46 ms with their set-up and ten of 70,000 1.36 ms, so 1.95 and 1.25.
+
+// The spectra's row pass (the first `nrows` workgroups, a multiple of 8) and the spread (four spread_waves to a
+// workgroup), with the host-planned record by value; the first workgroup stores it to `out`.
+template <int P, int MAXTOT>
+__global__ __launch_bounds__(kSpreadThreads) void k_spread_kern(const float *__restrict__ Y, int N, const DevGeo v,
+                                                                DevGeo *__restrict__ out,
+                                                                unsigned long long *__restrict__ grid,
+                                                                const double *__restrict__ ctr, int nrows,
+                                                                const cx<float> *__restrict__ tw, int kind_q,
+                                                                int kind_1, double df, cx<float> *__restrict__ Trow) {
+    extern __shared__ unsigned char smem_raw[];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *out = v;
+    if (!v.live) return;
+    if ((int)blockIdx.x < nrows) {
+        kern_rows_body<float, kSpreadThreads, MAXTOT, true>(&v, tw, kind_q, kind_1, df, Trow, blockIdx.x, nrows);
+        return;
+    }
+    const int w = threadIdx.x / kWave;
+    auto *L = reinterpret_cast<SpreadWaveLds<P, 2> *>(smem_raw);
+    spread_wave<P, 2>(Y, N, &v, grid, ((int)blockIdx.x - nrows) * (kSpreadThreads / kWave) + w, L[w], ctr);
+}
+
+// The spectra's column pass (behind the first `nrows` workgroups, a multiple of 8) and the forward row pass.
+template <int NTHR, int MAXTOT, int MAXKERN>
+__global__ __launch_bounds__(NTHR) void k_rows_kern(const DevGeo *__restrict__ dg, const cx<float> *__restrict__ tw,
+                                                    cx<float> *__restrict__ spec,
+                                                    unsigned long long *__restrict__ fixgrid, int nrows,
+                                                    const cx<float> *__restrict__ Trow, float *__restrict__ KQ,
+                                                    float *__restrict__ K1, float *__restrict__ KS,
+                                                    float *__restrict__ KT) {
+    if ((int)blockIdx.x < nrows)
+        rows_fwd_body<float, NTHR, MAXTOT, true>(dg, tw, nullptr, 4, 4, spec, fixgrid, blockIdx.x, nrows);
+    else
+        kern_cols_body<float, NTHR, MAXKERN, true>(dg, tw, Trow, 1, KQ, K1, KS, KT, (int)blockIdx.x - nrows,
+                                                   (int)gridDim.x - nrows);
 }
 
 // Column pass, FP32 form.  For column frequency k: DFT over u of A, c, b_x, b_y; then with K_q, K_1
