@@ -118,7 +118,8 @@ __device__ __forceinline__ double exact_qpow(double q, double df) {
 // computed on row N - 1 and discarded.  The next column's Y and P values are loaded into a second
 // register buffer while the current column is computed, so the loads of consecutive columns overlap
 // (the P loads are unconditional: every index is in bounds, the self pair is masked afterwards).
-// DF1 = (df == 1).
+// DF1 = (df == 1).  Without GRAD only the columns past the row count, twice (q is symmetric): zrow sums to the
+// same Z (N = 8,001: 60 us, over the triangle 33; bound by the division).
 // Grid: ceil(N / kExRows) workgroups of kThreads.
 template <int D, bool DF1, bool GRAD>
 __global__ __launch_bounds__(kThreads) void k_exact_rows(const double *__restrict__ P, const double *__restrict__ Y,
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(kThreads) void k_exact_rows(const double *__restric
     auto column = [&](int mm, const double (&ym)[D], const double (&pv)[kExRows]) {
 #pragma unroll
         for (int r = 0; r < kExRows; r++) {
-            const bool self = mm == n0 + r;
+            const bool self = GRAD ? mm == n0 + r : mm <= n0 + r;
             double diff[D], d2 = 0.0;
             {
 #pragma clang fp contract(off)
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(kThreads) void k_exact_rows(const double *__restric
             }
         }
     };
-    int m = threadIdx.x;
+    int m = (GRAD ? 0 : n0) + threadIdx.x;
     fetch(m, yA, pA);
     for (; m < N; m += 2 * kThreads) {
         fetch(m + kThreads, yB, pB);
@@ -214,7 +215,7 @@ __global__ __launch_bounds__(kThreads) void k_exact_rows(const double *__restric
         if (n < N && (GRAD || k == 2 * D)) {
             double t = 0.0;
             for (int i = 0; i < kThreads / kWave; i++) t += red[i][threadIdx.x];
-            if (k == 2 * D) zrow[n] = t;
+            if (k == 2 * D) zrow[n] = GRAD ? t : 2.0 * t;
             else if (k < D) att[(long)n * D + k] = t;
             else rep[(long)n * D + k - D] = t;
         }
@@ -231,10 +232,31 @@ __global__ __launch_bounds__(kThreads) void k_exact_combine(const double *__rest
         dC[e] = att[e] - rep[e] / Z;
 }
 
+// *flag = 1 if P[n][m] != P[m][n] for some pair.  Workgroup (I, J), J >= I, compares the tiles (I, J) and (J, I).
+// Grid: (T, T) with T = ceil(N / kSymTile), 256 threads = 32 x 8.
+__global__ __launch_bounds__(256) void k_exact_asym(const double *__restrict__ P, int N, int *__restrict__ flag) {
+    const int I = blockIdx.y, J = blockIdx.x;
+    if (J < I) return;
+    __shared__ double b[kSymTile][kSymTile + 1];
+    const int tx = threadIdx.x % kSymTile, ty = threadIdx.x / kSymTile;
+    const long r0 = (long)I * kSymTile, c0 = (long)J * kSymTile;
+    for (int r = ty; r < kSymTile; r += 256 / kSymTile)
+        b[r][tx] = c0 + r < N && r0 + tx < N ? P[(c0 + r) * N + r0 + tx] : 0.0;
+    __syncthreads();
+    bool differs = false;
+    for (int r = ty; r < kSymTile; r += 256 / kSymTile)
+        if (r0 + r < N && c0 + tx < N) differs |= !(P[(r0 + r) * N + c0 + tx] == b[tx][r]);  // (NaN differs too)
+    if (__ballot(differs) && threadIdx.x % kWave == 0) *flag = 1;
+}
+
 // KL of evaluateError (tsne.cpp:1286-1326) over rows n0 .. n0 + kExRows - 1: Q = q^df / sum_Q off the
 // diagonal, DBL_MIN / sum_Q on it, sum_Q = DBL_MIN + sum_{n != m} q^df (zsum[0] holds the sum);
-// C += P log((P + FLT_MIN) / (Q + FLT_MIN)) over all N^2 entries.  Block partials into part.
-template <int D, bool DF1>
+// C += P log((P + FLT_MIN) / (Q + FLT_MIN)) over all N^2 entries.  Block partials into part.  SYM: P equals
+// its transpose, and each pair is taken once, for twice its term.  Bound by the divisions and the logarithm, so
+// the quotients become one (two with the power): with w = sum_Q / q^df, (P + FLT_MIN) / (1 / w + FLT_MIN) =
+// (P + FLT_MIN) w / (1 + FLT_MIN w); w is cut at 1e200, where the 1 has long left the sum.  (N = 8,001: all
+// entries with three divisions 313 us, with one 276, SYM 139.)
+template <int D, bool DF1, bool SYM>
 __global__ __launch_bounds__(kThreads) void k_exact_kl(const double *__restrict__ P, const double *__restrict__ Y,
                                                        int N, double df, const double *__restrict__ zsum,
                                                        double *__restrict__ part) {
@@ -271,13 +293,17 @@ __global__ __launch_bounds__(kThreads) void k_exact_kl(const double *__restrict_
                     d2 += t * t;
                 }
             }
-            const double Q = (mm == n0 + r ? DBL_MIN : exact_qpow<DF1>(exact_q<DF1>(d2, df), df)) / sQ;
+            double w;
+            if constexpr (DF1) w = (1.0 + d2) * sQ;
+            else w = sQ / exact_qpow<DF1>(exact_q<DF1>(d2, df), df);
+            w = w > 1e200 ? 1e200 : w;
             const double p = pv[r];
-            const double c = p * log((p + fm) / (Q + fm));
-            acc += n0 + r < N ? c : 0.0;
+            const double c = p * log((p + fm) * w / (1.0 + fm * w));
+            const bool on = n0 + r < N && (SYM ? mm > n0 + r : mm != n0 + r);
+            acc += on ? c : 0.0;
         }
     };
-    int m = threadIdx.x;
+    int m = (SYM ? n0 : 0) + threadIdx.x;
     fetch(m, yA, pA);
     for (; m < N; m += 2 * kThreads) {
         fetch(m + kThreads, yB, pB);
@@ -285,6 +311,12 @@ __global__ __launch_bounds__(kThreads) void k_exact_kl(const double *__restrict_
         if (m + kThreads >= N) break;
         fetch(m + 2 * kThreads, yA, pA);
         column(m + kThreads, yB, pB);
+    }
+    if (SYM) acc *= 2.0;
+    if ((int)threadIdx.x < kExRows && n0 + (int)threadIdx.x < N) {  // the diagonal
+        const long n = n0 + threadIdx.x;
+        const double p = P[n * N + n];
+        acc += p * log((p + fm) / (DBL_MIN / sQ + fm));
     }
     __shared__ double sh[kThreads / kWave];
     acc = block_sum(acc, sh);

@@ -195,6 +195,7 @@ struct fitsne_ctx {
     size_t stage_cap = 0;
     hipEvent_t stage_ev[2] = {nullptr, nullptr};
     DBuf ybuf;                   // the caller's Y, dC or a part of P as doubles
+    bool P_sym = false;          // the dense P equals its transpose
     double *h_mm_dev = nullptr;  // h_mm as the device addresses it
     hipEvent_t mm_event = nullptr;
     bool mm_pending = false, mm_valid = false;
@@ -457,15 +458,24 @@ static int copy_in(fitsne_ctx *c, void *dst, const void *src, size_t bytes) {
     return stage_copy(c, static_cast<char *>(const_cast<void *>(src)), static_cast<char *>(dst), bytes, false);
 }
 
-// An error with this text if any of the n device doubles is infinite or NaN.
-static int need_finite(fitsne_ctx *c, const double *x, long n, const char *text) {
-    volatile int *flag = reinterpret_cast<volatile int *>(c->h_mm + 3);
-    *flag = 0;
-    launch(c, "nonfinite", k_nonfinite, dim3(std::min(blocks_for(n), 2048)), dim3(kThreads), 0, x, n,
-           reinterpret_cast<int *>(c->h_mm_dev + 3));
+// A flag that a kernel sets in pinned slot 3: cleared (nothing on the stream may write the slot), and read when the
+// stream is done.
+static void clear_flag(fitsne_ctx *c) { *reinterpret_cast<volatile int *>(c->h_mm + 3) = 0; }
+static int read_flag(fitsne_ctx *c, bool *set) {
     HIPTRY(hipGetLastError());
     HIPTRY(hipStreamSynchronize(c->stream));
-    return *flag ? fail(FITSNE_E_ARG, text) : FITSNE_OK;
+    *set = *reinterpret_cast<volatile int *>(c->h_mm + 3) != 0;
+    return FITSNE_OK;
+}
+
+// An error with this text if any of the n device doubles is infinite or NaN.
+static int need_finite(fitsne_ctx *c, const double *x, long n, const char *text) {
+    clear_flag(c);
+    launch(c, "nonfinite", k_nonfinite, dim3(std::min(blocks_for(n), 2048)), dim3(kThreads), 0, x, n,
+           reinterpret_cast<int *>(c->h_mm_dev + 3));
+    bool bad;
+    TRY(read_flag(c, &bad));
+    return bad ? fail(FITSNE_E_ARG, text) : FITSNE_OK;
 }
 
 // Y or dC (N x D) in the caller's order and type.
@@ -1632,7 +1642,9 @@ static int kl_exact_d(fitsne_ctx *c) {
            c->Y.as<const double>(), N, c->df, (double *)nullptr, (double *)nullptr, c->zrow.as<double>());
     launch(c, "kl_zsum", k_sum_final, dim3(1), dim3(kThreads), 0, c->zrow.as<const double>(), N, 0.0,
            c->mean.as<double>() + 2);
-    launch(c, "exact_kl", c->df == 1.0 ? k_exact_kl<D, true> : k_exact_kl<D, false>, dim3(nblk), dim3(kThreads), 0, c->val.as<const double>(),
+    auto kl = c->df == 1.0 ? (c->P_sym ? k_exact_kl<D, true, true> : k_exact_kl<D, true, false>)
+                           : (c->P_sym ? k_exact_kl<D, false, true> : k_exact_kl<D, false, false>);
+    launch(c, "exact_kl", kl, dim3(nblk), dim3(kThreads), 0, c->val.as<const double>(),
            c->Y.as<const double>(), N, c->df, c->mean.as<const double>() + 2, c->klpart.as<double>());
     launch(c, "kl_sum", k_sum_final, dim3(1), dim3(kThreads), 0, c->klpart.as<const double>(), nblk, 0.0,
            c->mean.as<double>());
@@ -2179,9 +2191,17 @@ extern "C" int fitsne_set_P_dense(fitsne_ctx *c, int N, const double *P) {
     HIPTRY(hipSetDevice(c->device));
     TRY(sync_ctx(c));
     const size_t nn = (size_t)N * N;
+    c->P_sym = false;
     TRY(ensure(c->val, sizeof(double) * nn));
     TRY(copy_in(c, c->val.p, P, sizeof(double) * nn));
+    clear_flag(c);
+    const int T = (N + kSymTile - 1) / kSymTile;
+    launch(c, "exact_asym", k_exact_asym, dim3(T, T), dim3(256), 0, c->val.as<const double>(), N,
+           reinterpret_cast<int *>(c->h_mm_dev + 3));
+    bool asym;
+    TRY(read_flag(c, &asym));
     dense_P_set(c, N);
+    c->P_sym = !asym;
     return FITSNE_OK;
 }
 
@@ -2209,6 +2229,7 @@ extern "C" int fitsne_exact_affinities(fitsne_ctx *c, const double *X, int N, in
     TRY(ensure(c->knnX, sizeof(double) * nd));
     TRY(copy_in(c, c->knnX.p, X, sizeof(double) * nd));
     TRY(need_finite(c, c->knnX.as<const double>(), (long)nd, "X contains non-finite values"));
+    c->P_sym = false;
     TRY(ensure(c->knnXT, sizeof(double) * nd));
     TRY(ensure(c->w, sizeof(double) * nn));
     TRY(ensure(c->val, sizeof(double) * nn));
@@ -2247,6 +2268,7 @@ extern "C" int fitsne_exact_affinities(fitsne_ctx *c, const double *X, int N, in
     if (P_out) TRY(copy_out(c, P_out, c->val.p, sizeof(double) * nn));
     release(c->w);  // the N x N distance matrix is not needed after the calibration
     dense_P_set(c, N);
+    c->P_sym = true;  // k_exact_sym
     if (sum_P) *sum_P = total;
     return FITSNE_OK;
 }
