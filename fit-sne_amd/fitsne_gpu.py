@@ -240,7 +240,7 @@ def knn_exact(X, K):
 
 
 def knn_mfma(X, K):
-    """The same neighbours as knn_exact for large N (FP32 MFMA candidates, FP64 re-rank): (idx, dist,
+    """The same neighbours as knn_exact for large N (f16 MFMA candidates, FP64 re-rank): (idx, dist,
     number of queries recomputed by the FP64 kernel)."""
     X = np.ascontiguousarray(X, dtype=np.float64)
     N, D = X.shape
