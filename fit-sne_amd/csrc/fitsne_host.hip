@@ -3895,8 +3895,11 @@ extern "C" int fitsne_knn_exact(const double *X, int N, int D, int K, int32_t *i
     fitsne_ctx *c;
     TRY(mirror_ctx(&c, 1, 3, 1.0, 1, 1.0));
     HIPTRY(hipSetDevice(c->device));
-    if (N >= kKnnFilterMinN && D <= kKmMaxD && K <= kKmMaxK && (long)N * (D + 40) >= kKnnFilterWork)
-        return knn_filtered(c, X, N, D, K, idx, dist, nullptr);
+    if (N >= kKnnFilterMinN && D <= kKmMaxD && K <= kKmMaxK && (long)N * (D + 40) >= kKnnFilterWork) {
+        const int rc = knn_filtered(c, X, N, D, K, idx, dist, nullptr);
+        if (rc != FITSNE_E_ALLOC) return rc;
+        (void)hipGetLastError();  // no room for the candidate lists: the FP64 kernel needs none
+    }
     return knn_plain(c, X, N, D, K, idx, dist);
 }
 
