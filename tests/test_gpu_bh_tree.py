@@ -109,3 +109,13 @@ def test_steps_follow_the_host_loop(scale):
         np.testing.assert_array_equal(g, gr)
         assert z == zr
     c.close()
+
+
+@pytest.mark.parametrize("scale", [1e126, 1e128, 1e160])
+@pytest.mark.parametrize("N", [17, 1100])
+def test_far_apart(N, scale):
+    """Q so small that Z lies below the range the parallel sum folds, or is zero (then dC is not a number)."""
+    rng = np.random.default_rng(N)
+    print(f"[gpu] bh far apart N={N} scale={scale}", flush=True)
+    with np.errstate(all="ignore"):
+        compare(rng.normal(size=(N, 2)) * scale, 0.5)
