@@ -1019,10 +1019,19 @@ static int launch_f32_stages(fitsne_ctx *c, const cx<float> *tw, const StageDims
     const bool waves = N < kSpreadWaveN;
     const bool fused = D == 2 && kern && hv && waves;  // passes of a small embedding's step share launches
     const bool kside = D == 2 && kern && side && c->overlap && !fused;
-    // the spectra read the record (by value with hv) and the twiddles: wait for the stream only when it wrote
-    // either in this step
-    const bool kwait = kside && (!hv || c->tw_fresh);
-    if (kwait) HIPTRY(hipEventRecord(c->geo_ev, c->stream));
+    if (kside) {  // before the spread (behind its launch: N = 300,000 171 to 177 us a step, so 171 to 172)
+        // the spectra read the record (by value with hv) and the twiddles: wait for the stream only when
+        // it wrote either in this step
+        if (!hv || c->tw_fresh) {
+            HIPTRY(hipEventRecord(c->geo_ev, c->stream));
+            HIPTRY(hipStreamWaitEvent(c->astream, c->geo_ev, 0));
+        }
+        hipStream_t main = c->stream;
+        c->stream = c->astream;
+        kernel_spectra();
+        c->stream = main;
+        HIPTRY(hipEventRecord(c->kern_ev, c->astream));
+    }
     // 1D: the kernel line (its spectra depend only on the geometry record and the twiddles) on the third
     // stream, after the work queued so far on the grid stages' stream (the twiddle table, the last
     // convolution's read of kline)
@@ -1055,14 +1064,6 @@ static int launch_f32_stages(fitsne_ctx *c, const cx<float> *tw, const StageDims
     else
         launch(c, "spread_f32", waves ? pick_spread_wave<D>(p) : pick_spread_f32<D>(p), sgrid, sblk, 0,
                c->Y.as<const float>(), N, pts, dg, c->fixgrid.as<unsigned long long>(), ctr);
-    if (kside) {  // after the spread, whose launch the grid stages wait for
-        if (kwait) HIPTRY(hipStreamWaitEvent(c->astream, c->geo_ev, 0));
-        hipStream_t main = c->stream;
-        c->stream = c->astream;
-        kernel_spectra();
-        c->stream = main;
-        HIPTRY(hipEventRecord(c->kern_ev, c->astream));
-    }
     if constexpr (D == 2) {
         const size_t Mp = (size_t)sd.Mp;
         if (kern && !kside && !fused) kernel_spectra();
