@@ -662,13 +662,12 @@ static auto pick_spread_f32(int p) -> decltype(&k_spread_f32<3, D>) {
     default: return k_spread_f32<5, D>;
     }
 }
-template <int D>
-static auto pick_spread_wave(int p) -> decltype(&k_spread_wave<3, D>) {
+static auto pick_spread_wave(int p) -> decltype(&k_spread_wave<3>) {
     switch (p) {
-    case 2: return k_spread_wave<2, D>;
-    case 3: return k_spread_wave<3, D>;
-    case 4: return k_spread_wave<4, D>;
-    default: return k_spread_wave<5, D>;
+    case 2: return k_spread_wave<2>;
+    case 3: return k_spread_wave<3>;
+    case 4: return k_spread_wave<4>;
+    default: return k_spread_wave<5>;
     }
 }
 template <int D>
@@ -690,19 +689,18 @@ static auto pick_spread_kern(int p) -> decltype(&k_spread_kern<3, kKernTot>) {
 }
 static size_t spread_wave_lds(int p) {
     switch (p) {
-    case 2: return sizeof(SpreadWaveLds<2, 2>);
-    case 3: return sizeof(SpreadWaveLds<3, 2>);
-    case 4: return sizeof(SpreadWaveLds<4, 2>);
-    default: return sizeof(SpreadWaveLds<5, 2>);
+    case 2: return sizeof(SpreadWaveLds<2>);
+    case 3: return sizeof(SpreadWaveLds<3>);
+    case 4: return sizeof(SpreadWaveLds<4>);
+    default: return sizeof(SpreadWaveLds<5>);
     }
 }
-template <int D>
-static auto pick_spread_wave_v(int p) -> decltype(&k_spread_wave_v<3, D>) {
+static auto pick_spread_wave_v(int p) -> decltype(&k_spread_wave_v<3>) {
     switch (p) {
-    case 2: return k_spread_wave_v<2, D>;
-    case 3: return k_spread_wave_v<3, D>;
-    case 4: return k_spread_wave_v<4, D>;
-    default: return k_spread_wave_v<5, D>;
+    case 2: return k_spread_wave_v<2>;
+    case 3: return k_spread_wave_v<3>;
+    case 4: return k_spread_wave_v<4>;
+    default: return k_spread_wave_v<5>;
     }
 }
 template <int D>
@@ -1016,8 +1014,8 @@ static int launch_f32_stages(fitsne_ctx *c, const cx<float> *tw, const StageDims
                    c->K1.as<float>(), c->KS.as<float>(), c->KT.as<float>());
         }
     };
-    const bool waves = N < kSpreadWaveN;
-    const bool fused = D == 2 && kern && hv && waves;  // passes of a small embedding's step share launches
+    const bool waves = spread_waves(D, p, N);
+    const bool fused = waves && kern && hv;  // passes of a small embedding's step share launches
     const bool kside = D == 2 && kern && side && c->overlap && !fused;
     if (kside) {  // before the spread (behind its launch: N = 300,000 171 to 177 us a step, so 171 to 172)
         // the spectra read the record (by value with hv) and the twiddles: wait for the stream only when
@@ -1051,19 +1049,27 @@ static int launch_f32_stages(fitsne_ctx *c, const cx<float> *tw, const StageDims
     c->tw_fresh = false;
     const int pts = waves ? 2 * kWave : c->spread_pts;
     const dim3 sgrid((N + pts - 1) / pts), sblk(waves ? kWave : kSpreadThreads);
-    if (fused) {
-        const size_t Mp = (size_t)sd.Mp, lines = sizeof(cx<float>) * (lspan<true>((int)Mp) + Mp);
-        const int per = 2 * kSpreadThreads;
-        launch(c, "spread_kern", pick_spread_kern(p), dim3(sd.gr_rows + (N + per - 1) / per), dim3(kSpreadThreads),
-               std::max(lines, spread_wave_lds(p) * (kSpreadThreads / kWave)), c->Y.as<const float>(), N, *hv,
-               c->dgeo.as<DevGeo>(), c->fixgrid.as<unsigned long long>(), ctr, sd.gr_rows, tw, kind_q, kind_1, c->df,
-               c->Trow.as<cx<float>>());
-    } else if (hv)
-        launch(c, "spread_f32", waves ? pick_spread_wave_v<D>(p) : pick_spread_f32_v<D>(p), sgrid, sblk, 0,
-               c->Y.as<const float>(), N, pts, *hv, c->dgeo.as<DevGeo>(), c->fixgrid.as<unsigned long long>(), ctr);
-    else
-        launch(c, "spread_f32", waves ? pick_spread_wave<D>(p) : pick_spread_f32<D>(p), sgrid, sblk, 0,
-               c->Y.as<const float>(), N, pts, dg, c->fixgrid.as<unsigned long long>(), ctr);
+    if constexpr (D == 2) {
+        if (fused) {
+            const size_t Mp = (size_t)sd.Mp, lines = sizeof(cx<float>) * (lspan<true>((int)Mp) + Mp);
+            const int per = 2 * kSpreadThreads;
+            launch(c, "spread_kern", pick_spread_kern(p), dim3(sd.gr_rows + (N + per - 1) / per), dim3(kSpreadThreads),
+                   std::max(lines, spread_wave_lds(p) * (kSpreadThreads / kWave)), c->Y.as<const float>(), N, *hv,
+                   c->dgeo.as<DevGeo>(), c->fixgrid.as<unsigned long long>(), ctr, sd.gr_rows, tw, kind_q, kind_1,
+                   c->df, c->Trow.as<cx<float>>());
+        } else if (waves && hv)
+            launch(c, "spread_f32", pick_spread_wave_v(p), sgrid, sblk, 0, c->Y.as<const float>(), N, pts, *hv,
+                   c->dgeo.as<DevGeo>(), c->fixgrid.as<unsigned long long>(), ctr);
+        else if (waves)
+            launch(c, "spread_f32", pick_spread_wave(p), sgrid, sblk, 0, c->Y.as<const float>(), N, pts, dg,
+                   c->fixgrid.as<unsigned long long>(), ctr);
+    }
+    if (!waves && hv)
+        launch(c, "spread_f32", pick_spread_f32_v<D>(p), sgrid, sblk, 0, c->Y.as<const float>(), N, pts, *hv,
+               c->dgeo.as<DevGeo>(), c->fixgrid.as<unsigned long long>(), ctr);
+    else if (!waves)
+        launch(c, "spread_f32", pick_spread_f32<D>(p), sgrid, sblk, 0, c->Y.as<const float>(), N, pts, dg,
+               c->fixgrid.as<unsigned long long>(), ctr);
     if constexpr (D == 2) {
         const size_t Mp = (size_t)sd.Mp;
         if (kern && !kside && !fused) kernel_spectra();
@@ -1228,7 +1234,7 @@ static int pipeline_f32(fitsne_ctx *c, int mode, const fitsne_step_params *sp) {
         TRY((launch_attractive<float, D>(c, (float)c->exag, c->pos.as<float>(), live, false, ctr)));
         c->swap_main = c->stream;
         c->stream = c->astream;
-    } else if (c->overlap && c->N >= kSpreadWaveN) {
+    } else if (c->overlap && !spread_waves(D, c->p, c->N)) {
         if (!c->astream) HIPTRY(hipStreamCreateWithFlags(&c->astream, hipStreamNonBlocking));
         HIPTRY(hipEventRecord(c->fork_ev, c->stream));
         HIPTRY(hipStreamWaitEvent(c->astream, c->fork_ev, 0));
@@ -1307,7 +1313,7 @@ constexpr float kSpreadGain = 0.97f;
 template <int D>
 static int tune_spread(fitsne_ctx *c) {
     const int N = c->N;
-    if (N < kSpreadWaveN) return FITSNE_OK;  // one form whatever the workgroup
+    if (spread_waves(D, c->p, N)) return FITSNE_OK;  // one form whatever the workgroup
     double mn, mx;
     TRY(current_minmax<float>(c, &mn, &mx));
     Geo g;

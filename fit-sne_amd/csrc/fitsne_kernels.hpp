@@ -1189,32 +1189,39 @@ __global__ __launch_bounds__(kSpreadThreads) __attribute__((amdgpu_waves_per_eu(
 }
 
 // LDS of one k_spread_wave wavefront: the sums of its runs of one flush, a row of values each (odd stride).
-template <int P, int D>
+template <int P>
 struct SpreadWaveLds {
-    static constexpr int NV = (D == 2 ? P * P : P), NQ = (D == 2 ? 4 : 3), ROW = (NV * NQ) | 1;
+    static constexpr int NV = P * P, NQ = 4, ROW = (NV * NQ) | 1;
     float val[kWave][ROW];
     int box[kWave];
 };
 
-// Below this many points the spread goes straight into the grid, a wavefront to a workgroup (spread_wave), else over the
-// workgroups' tables.  A table pays where workgroups are many and their boxes few; a small embedding gives
+// Below these many points the 2D spread goes straight into the grid, a wavefront to a workgroup (spread_wave), else
+// over the workgroups' tables.  A table pays where workgroups are many and their boxes few; a small embedding gives
 // either too few workgroups (2 of 1024 points at N = 2,000) or more boxes than the table has slots, whose every probe
-// walks the whole table.  Launch to end, 2D, 3 nodes, table of 1024 and of 512 points, and this: N = 2,000
-// 74, 42, 18 us; 70,000 (5,625 boxes) 19, 13, 12 and (6,400 boxes) 35, 19, 15; 140,000 18, 14, 14 and 34, 17, 16;
-// 300,000 20, 16, 22 and 41, 18, 23; a million 29, 29, 62.  1D: 2,000 9.6, 7.5, 7.5; 70,000 8.9, 7.0, 5.9.
-constexpr int kSpreadWaveN = 150000;
+// walks the whole table.  Straight, every run of points costs 4 P^2 atomics, and once the points are out of order
+// (a run from a random start: after a few dozen steps) a run is one or two points, and where most points share few
+// boxes the atomics meet.  So the line lies where whole runs of 750 steps from a random start take the same (us a
+// step, 60 entries per row, table with its streams / straight on one stream): 3 nodes N = 5,000 97 / 72, 20,000 118
+// / 86, 30,000 119 / 100, 40,000 117 / 111, 50,000 114 / 125, 70,000 129 / 156 (captured 30,000 145 / 135, 40,000 147 /
+// 150, 70,000 157 / 197); 2 nodes 40,000 95 / 83, 70,000 103 / 106.  With 4 and 5 nodes the values of a box fill the
+// table's slots sooner: 70,000 303 / 165 and 472 / 237, 140,000 460 / 270 and 816 / 414 (points still in their sorted
+// order 188 / 204 and 194 / 281).  In 1D straight is no faster from 10,000 points on (70,000 88 / 102, captured 92 /
+// 109) and within 3% below: always the table.
+constexpr int kSpreadWaveN = 40000, kSpreadWaveNWide = 150000;  // up to 3 nodes per box and side, and more
+constexpr bool spread_waves(int D, int p, int N) { return D == 2 && N < (p <= 3 ? kSpreadWaveN : kSpreadWaveNWide); }
 
 // The 128 points of wavefront `bid`, straight into the grid: each flush puts the runs' sums into LDS, and the lanes
 // add them value by value, so that the 4 NV values of a run are a few neighbouring pieces of the grid in one
 // instruction.  The runs and their order are those of spread_block, and so the grid is the same to the bit.
-template <int P, int D>
+template <int P>
 __device__ __forceinline__ void spread_wave(const float *__restrict__ Y, int N, const DevGeo *__restrict__ dg,
-                                            unsigned long long *__restrict__ grid, int bid, SpreadWaveLds<P, D> &L,
+                                            unsigned long long *__restrict__ grid, int bid, SpreadWaveLds<P> &L,
                                             const double *__restrict__ ctr) {
-    constexpr int NV = SpreadWaveLds<P, D>::NV, NQ = SpreadWaveLds<P, D>::NQ, NE = NV * NQ;
+    constexpr int NV = SpreadWaveLds<P>::NV, NQ = SpreadWaveLds<P>::NQ, NE = NV * NQ;
     const Geo &g = dg->g;
     const int lane = threadIdx.x % kWave;
-    spread_pairs<P, D>(Y, N, (long)bid * 2 * kWave + 2 * lane, g, ctr,
+    spread_pairs<P, 2>(Y, N, (long)bid * 2 * kWave + 2 * lane, g, ctr,
                        [&](bool on, int box, const float (&val)[NV][NQ]) {
         const unsigned long long who = __ballot(on);
         const int n = __popcll(who), at = __popcll(who & ((1ull << lane) - 1ull));
@@ -1229,8 +1236,8 @@ __device__ __forceinline__ void spread_wave(const float *__restrict__ Y, int N, 
         __builtin_amdgcn_wave_barrier();
         for (int e = lane; e < n * NE; e += kWave) {
             const int r = e / NE, k = e - r * NE, v = k / NQ, q = k - v * NQ, b = L.box[r];
-            const int by = D == 2 ? b / g.nb : 0, bx = b - by * g.nb;
-            const long node = D == 2 ? (long)(bx * P + v / P) * g.n1d + by * P + v % P : (long)b * P + v;
+            const int by = b / g.nb, bx = b - by * g.nb;
+            const long node = (long)(bx * P + v / P) * g.n1d + by * P + v % P;
             const double x = (double)L.val[r][k] * g.fix;
             atomicAdd(&grid[node * 4 + q], (unsigned long long)(g.fix_fast ? fix_rn(x) : fix_rn_any(x)));
         }
@@ -1240,25 +1247,25 @@ __device__ __forceinline__ void spread_wave(const float *__restrict__ Y, int N, 
 }
 
 // k_spread_f32 and k_spread_f32_v by spread_wave, one wavefront to a workgroup.
-template <int P, int D>
+template <int P>
 __global__ __launch_bounds__(kWave) void k_spread_wave(const float *__restrict__ Y, int N, int,
                                                        const DevGeo *__restrict__ dg,
                                                        unsigned long long *__restrict__ grid,
                                                        const double *__restrict__ ctr) {
-    __shared__ SpreadWaveLds<P, D> L;
+    __shared__ SpreadWaveLds<P> L;
     if (!dg->live) return;
-    spread_wave<P, D>(Y, N, dg, grid, blockIdx.x, L, ctr);
+    spread_wave<P>(Y, N, dg, grid, blockIdx.x, L, ctr);
 }
 
-template <int P, int D>
+template <int P>
 __global__ __launch_bounds__(kWave) void k_spread_wave_v(const float *__restrict__ Y, int N, int, const DevGeo v,
                                                          DevGeo *__restrict__ out,
                                                          unsigned long long *__restrict__ grid,
                                                          const double *__restrict__ ctr) {
-    __shared__ SpreadWaveLds<P, D> L;
+    __shared__ SpreadWaveLds<P> L;
     if (blockIdx.x == 0 && threadIdx.x == 0) *out = v;
     if (!v.live) return;
-    spread_wave<P, D>(Y, N, &v, grid, blockIdx.x, L, ctr);
+    spread_wave<P>(Y, N, &v, grid, blockIdx.x, L, ctr);
 }
 
 // int64 grid -> float4 (A, c, b_x, b_y) and clear, for the 1D path (the 2D row FFT does this itself).
@@ -1542,10 +1549,11 @@ __global__ __launch_bounds__(NTHR) void k_rows_fwd(const DevGeo *__restrict__ dg
     rows_fwd_body<T, NTHR, MAXTOT, PAD>(dg, tw, grid, sin, nterms, spec, fixgrid, blockIdx.x, gridDim.x);
 }
 
-// ---- a small embedding's step (2D, below kSpreadWaveN points): its passes are bound by latency, not by work, so passes that
+// ---- a small embedding's step (2D, where spread_waves): its passes are bound by latency, not by work, so passes that
 // do not depend on each other share a launch and the step stays on one stream (each wait for another stream costs
-// about 10 us).  With the attractive term and the spectra on the second stream 20 steps of 2,000 points took
-// 2.46 ms with their set-up and ten of 70,000 1.36 ms, so 1.95 and 1.25.
+// about 10 us).  With the spread straight into the grid but the attractive term and the spectra on the second stream:
+// N = 5,000 92 us a step against 72, 40,000 126 against 111, and with 250 entries per row 111 against 94; 4 nodes, 140,000 points
+// and 240 entries per row, where the term is longest, 302 against 311.
 
 // The spectra's row pass (the first `nrows` workgroups, a multiple of 8) and the spread (four spread_waves to a
 // workgroup), with the host-planned record by value; the first workgroup stores it to `out`.
@@ -1564,8 +1572,8 @@ __global__ __launch_bounds__(kSpreadThreads) void k_spread_kern(const float *__r
         return;
     }
     const int w = threadIdx.x / kWave;
-    auto *L = reinterpret_cast<SpreadWaveLds<P, 2> *>(smem_raw);
-    spread_wave<P, 2>(Y, N, &v, grid, ((int)blockIdx.x - nrows) * (kSpreadThreads / kWave) + w, L[w], ctr);
+    auto *L = reinterpret_cast<SpreadWaveLds<P> *>(smem_raw);
+    spread_wave<P>(Y, N, &v, grid, ((int)blockIdx.x - nrows) * (kSpreadThreads / kWave) + w, L[w], ctr);
 }
 
 // The spectra's column pass (behind the first `nrows` workgroups, a multiple of 8) and the forward row pass.

@@ -17,7 +17,7 @@ def context(P, Y, D=2, p=3):
     return c
 
 
-@pytest.mark.parametrize("N,p", [(150_001, 3), (150_001, 4)])
+@pytest.mark.parametrize("N,p", [(40_001, 3), (150_001, 3), (150_001, 4)])
 def test_streams_leave_results_bitwise_unchanged(N, p):
     """Overlap on and off, across a wider Y (a longer FFT line, so that the spectra's buffers grow) and back."""
     print(f"[gpu] step forms: overlap N={N} p={p}", flush=True)
@@ -42,3 +42,53 @@ def test_streams_leave_results_bitwise_unchanged(N, p):
     assert za == zb
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("D,N,p,small", [(2, 39_999, 3, True), (2, 40_000, 3, False), (2, 39_999, 2, True), (2, 70_000, 3, False),
+                                         (2, 40_000, 4, True), (2, 149_999, 5, True), (2, 150_000, 4, False),
+                                         (1, 2_000, 3, False)])
+def test_which_form_a_step_takes(D, N, p, small):
+    """The shared launches only where they were measured to be the faster form, and there the same grid: the step
+    equals a batch member's (which always spreads over tables) bit for bit."""
+    print(f"[gpu] step forms: D={D} N={N} p={p}", flush=True)
+    P, Y = random_csr(N, 6, seed=N), blobs(N, D, 6, seed=p, span=40.0, sd=2.0)
+    a = context(P, Y, D, p)
+    a.set_timing(True)
+    a.step(0.5, 200.0, 5.0)
+    names = [str(k) for k in a.kernel_stats()]
+    a.set_timing(False)
+    assert any("spread_kern" in k for k in names) == small, names
+    for _ in range(2):
+        a.step(0.5, 200.0, 5.0)
+    if D == 2:
+        m = context(P, Y, D, p)
+        b = fg.Batch([m])
+        for _ in range(3):
+            b.step([(0.5, 200.0, 5.0)])
+        np.testing.assert_array_equal(a.get_Y(), m.get_Y())
+        b.close()
+        m.close()
+    a.close()
+
+
+@pytest.mark.parametrize("N,p", [(41_000, 3), (150_001, 4)])
+def test_spread_workgroup_size_does_not_change_a_2d_step(N, p):
+    """Points per workgroup of the table spread, at sizes that take it, host-planned and captured."""
+    print(f"[gpu] step forms: spread points N={N} p={p}", flush=True)
+    P, Y = random_csr(N, 6, seed=N), blobs(N, 2, 6, seed=p, span=40.0, sd=2.0)
+    want = None
+    for pts in (1024, 512, 2048, 4096):
+        for graph in (False, True):
+            c = context(P, Y, 2, p)
+            c.set_spread_points(pts)
+            g, z = c.gradient()
+            if graph:
+                c.set_graph(True)
+            for _ in range(3):
+                c.step(0.5, 200.0, 5.0)
+            got = (g, z, c.get_Y())
+            c.close()
+            want = want or got
+            np.testing.assert_array_equal(got[0], want[0])
+            assert got[1] == want[1]
+            np.testing.assert_array_equal(got[2], want[2])
