@@ -1306,14 +1306,14 @@ static int launch_step_dev(fitsne_ctx *c) {
 // points); only the time differs: small problems want more, smaller workgroups, large ones fewer table
 // flushes.  A larger candidate is kept only when it is more than 3% faster alone: inside the step the
 // spread fills the CUs the attractive kernel frees, which smaller workgroups do better (at N = 2M in 1D,
-// 1024 points measured 4% slower per step than 512, though alone the two are within noise).
+// 1024 points measured 4% slower per step than 512, though alone the two are within noise).  A small 2D context
+// does not use it alone (spread_waves), but as a member of a batch.
 constexpr int kSpreadPtsCand[] = {512, 1024, 2048, 4096};
 constexpr float kSpreadGain = 0.97f;
 
 template <int D>
 static int tune_spread(fitsne_ctx *c) {
     const int N = c->N;
-    if (spread_waves(D, c->p, N)) return FITSNE_OK;  // one form whatever the workgroup
     double mn, mx;
     TRY(current_minmax<float>(c, &mn, &mx));
     Geo g;

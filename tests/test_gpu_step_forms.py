@@ -92,3 +92,23 @@ def test_spread_workgroup_size_does_not_change_a_2d_step(N, p):
             np.testing.assert_array_equal(got[0], want[0])
             assert got[1] == want[1]
             np.testing.assert_array_equal(got[2], want[2])
+
+
+def test_batch_members_get_their_own_spread_size():
+    """Creating a batch tunes every member's table spread, also of those that would not use one alone: 2,000 points
+    are two workgroups of 1024 points (the default) or four of 512."""
+    sizes = [2000, 2001, 2500]
+    print(f"[gpu] step forms: batch tuning {sizes}", flush=True)
+    data = [(random_csr(N, 6, seed=N), blobs(N, 2, 4, seed=N, span=30.0, sd=2.0)) for N in sizes]
+    single, members = [context(P, Y) for P, Y in data], [context(P, Y) for P, Y in data]
+    b = fg.Batch(members)
+    assert [c.tuned()[0] for c in members] == [512] * len(sizes)
+    for _ in range(3):
+        b.step([(0.5, 100.0, 5.0)] * len(sizes))
+        for c in single:
+            c.step(0.5, 100.0, 5.0)
+    for c, m in zip(single, members):
+        np.testing.assert_array_equal(c.get_Y(), m.get_Y())
+    b.close()
+    for c in single + members:
+        c.close()
