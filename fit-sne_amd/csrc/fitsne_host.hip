@@ -326,10 +326,12 @@ static int att_lanes(long long nnz, int N) {
 }
 
 // ---------------------------------------------------------------- copies between host and device
-// The runtime's copies from and to pageable memory are slow around 1 MB (0.4 ms against 28 us from pinned
-// memory) and where the destination's pages are new (4 to 6 GB/s: one thread takes the page faults).  So copies go through a pinned buffer of the context, in pieces, the DMA of one
-// beside the memcpy of the other, and large ones have several threads for the memcpy (fresh pages:
-// 4.8 GB/s with one thread, 21 with eight; DMA 57).
+// The runtime's copies from pageable memory are slow for about the first 90 of every hardware queue (the CPU
+// writes them at 2.4 GB/s: 200 KB 88 us, 404 KB 170, from pinned memory 14 and 20; a new context's P of 103,622
+// entries 392 us), those to it where the destination's pages are new (4 to 6 GB/s: one thread takes the page
+// faults).  So copies go through a pinned buffer of the context, in pieces, the DMA of one beside the memcpy of the
+// other, and large ones have several threads for the memcpy (fresh pages: 4.8 GB/s with one thread, 21 with
+// eight; DMA 57).
 
 // Threads that copy their share of a piece beside the caller's; they last for one stage_copy.
 class CopyTeam {
@@ -386,7 +388,8 @@ class CopyTeam {
 };
 
 constexpr size_t kStage = 4u << 20;
-constexpr size_t kStageFirst = 64 << 10;  // the context's first pinned allocation: h_mm in 256 bytes, then the stage
+// The context's first pinned allocation: h_mm in 256 bytes, then the stage (it costs 12 us, of 16 KB as of 4 MB).
+constexpr size_t kStageFirst = (512 << 10) + 256;
 static char *first_stage(const fitsne_ctx *c) { return reinterpret_cast<char *>(c->h_mm) + 256; }
 
 // At least `need` (<= kStage) bytes of pinned buffer; nothing may be in flight in it.
@@ -395,7 +398,7 @@ static int stage_room(fitsne_ctx *c, size_t need) {
     if (c->stage && c->stage != first_stage(c)) (void)hipHostFree(c->stage);
     c->stage = nullptr;
     c->stage_cap = 0;
-    size_t want = kStageFirst;
+    size_t want = kStageFirst - 256;
     while (want < need) want *= 2;
     if (hipHostMalloc((void **)&c->stage, want, hipHostMallocDefault) != hipSuccess ||
         hipHostGetDevicePointer((void **)&c->stage_dev, c->stage, 0) != hipSuccess) {
@@ -412,11 +415,12 @@ static int stage_room(fitsne_ctx *c, size_t need) {
 constexpr size_t kStageDirect = 1 << 20;
 
 // bytes from device memory dev to host (out) or back, on c->stream behind what is queued there; done when it
-// returns.  Pieces: a quarter of the copy, from 256 KB (below which the DMA's latency shows) to half the buffer.
+// returns.  Pieces: a quarter of the copy, from 512 KB (uploads of 404 and 829 KB in pieces of 256 KB 20 to 25 us longer: a
+// DMA of its own each) to half the buffer.
 // Helpers: one per 4 MB (starting one costs 20 us), at most seven.
 static int stage_copy(fitsne_ctx *c, char *host, char *dev, size_t bytes, bool out) {
     if (!bytes) return FITSNE_OK;
-    const size_t piece = std::min(std::max((bytes / 4 + 4095) & ~(size_t)4095, (size_t)256 << 10), kStage / 2);
+    const size_t piece = std::min(std::max((bytes / 4 + 4095) & ~(size_t)4095, (size_t)512 << 10), kStage / 2);
     const size_t need = std::min(bytes, 2 * piece), n = (bytes + piece - 1) / piece;
     TRY(stage_room(c, need));
     auto half = [&](size_t k) { return c->stage + (k & 1) * piece; };
@@ -426,7 +430,7 @@ static int stage_copy(fitsne_ctx *c, char *host, char *dev, size_t bytes, bool o
                    : hipMemcpyAsync(dev + k * piece, half(k), len(k), hipMemcpyHostToDevice, c->stream);
     };
     if (out) HIPTRY(dma(0));
-    CopyTeam team((int)std::min<size_t>({bytes >> 22, 7, std::max(1u, std::thread::hardware_concurrency()) - 1}));
+    CopyTeam team(bytes >> 22 ? (int)std::min<size_t>({bytes >> 22, 7, std::max(1u, std::thread::hardware_concurrency()) - 1}) : 0);
     for (size_t k = 0; k < n; k++) {
         if (out) {
             HIPTRY(hipStreamSynchronize(c->stream));
@@ -448,13 +452,7 @@ static int stage_copy(fitsne_ctx *c, char *host, char *dev, size_t bytes, bool o
 static int copy_out(fitsne_ctx *c, void *dst, const void *src, size_t bytes) {
     return stage_copy(c, static_cast<char *>(dst), static_cast<char *>(const_cast<void *>(src)), bytes, true);
 }
-// (Up to 512 KB the runtime's own copy to the device is as fast: 480 KB in 24 us.)
 static int copy_in(fitsne_ctx *c, void *dst, const void *src, size_t bytes) {
-    if (bytes <= (512 << 10)) {
-        HIPTRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
-        HIPTRY(hipStreamSynchronize(c->stream));
-        return FITSNE_OK;
-    }
     return stage_copy(c, static_cast<char *>(const_cast<void *>(src)), static_cast<char *>(dst), bytes, false);
 }
 

@@ -76,3 +76,28 @@ def test_knn_refuses_non_finite(N, D, K):
     d = np.sqrt(((X[idx[-1]] - X[-1]) ** 2).sum(axis=1))
     np.testing.assert_allclose(dist[-1], d, rtol=1e-12)
     assert np.all(np.diff(dist[-1]) >= 0) and len(set(idx[-1])) == K
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("nnz", [16383, 16385, 65535, 65537, 131071, 131073, 131137])
+def test_small_P(nnz, prec):
+    """P whose columns (4 bytes) and values (4 or 8) end about the first buffer's halves and end: the
+    attractive term of every entry, by the gradient against the oracle."""
+    print(f"[gpu] copies P nnz={nnz} {prec}", flush=True)
+    import orc
+
+    N = 2000
+    rng = np.random.default_rng(nnz)
+    row = np.r_[0, np.sort(rng.integers(0, nnz + 1, N - 1)), nnz].astype(np.uint32)
+    col = rng.integers(0, N, nnz).astype(np.uint32)
+    val = rng.random(nnz)
+    val /= val.sum()
+    Y = fixed_order(rng.normal(size=(N, 2)) * 12.0).astype(np.float32).astype(np.float64)
+    c = fg.Context(no_dims=2, precision=fg.FP64_PLAIN if prec == "fp64" else fg.FP32)
+    c.set_P(row, col, val)
+    c.set_Y(Y)
+    g, _ = c.gradient()
+    c.close()
+    want, _ = orc.gradient((row, col, val), Y)
+    r = np.linalg.norm(g - want) / np.linalg.norm(want)
+    assert r <= (1e-9 if prec == "fp64" else 1e-4), r
