@@ -57,3 +57,30 @@ def test_far_points(symmetric):
     Y[7], Y[8] = 1e140, -1e90
     got, want = kl(P, Y, 1.0), orc.exact_kl(P, Y)
     assert abs(got - want) <= 1e-12 * abs(want)
+
+
+@pytest.mark.parametrize("symmetric", [True, False])
+@pytest.mark.parametrize("df,N,D", [(1.0, 2047, 2), (1.0, 2048, 2), (0.7, 2049, 1), (1.0, 2079, 3), (0.7, 2081, 4)])
+def test_kl_from_the_comparison_on(N, D, df, symmetric):
+    """About 2,048 points: from there on P is compared with its transpose."""
+    test_kl(N, D, df, symmetric)
+
+
+@pytest.mark.parametrize("at", [(2099, 0), (2099, 2098), (31, 32), (0, 2099)])
+def test_one_asymmetric_entry_of_many(at):
+    print(f"[gpu] exact KL, entry {at} differs", flush=True)
+    P = dense_P(2100, 1, True)
+    P[at] = P[at] * 1.5 + 1e-4
+    Y = np.random.default_rng(2).normal(0, 5, size=(2100, 2))
+    got, want = kl(P, Y, 1.0), orc.exact_kl(P, Y)
+    assert abs(got - want) <= 1e-12 * abs(want)
+
+
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_far_points_over_the_triangle(symmetric):
+    print("[gpu] exact KL, far points, triangle", flush=True)
+    P = dense_P(2100, 3, symmetric)
+    Y = np.random.default_rng(4).normal(0, 5, size=(2100, 2))
+    Y[7], Y[8] = 1e140, -1e90
+    got, want = kl(P, Y, 1.0), orc.exact_kl(P, Y)
+    assert abs(got - want) <= 1e-12 * abs(want)
