@@ -1446,10 +1446,16 @@ static int plain_conv(fitsne_ctx *c, const Geo &g, const cx<double> *tw, const d
     return FITSNE_OK;
 }
 
-// The attractive term runs on the second stream beside the grid stages, the 2D kernel spectra on the third (unless
-// overlap is off).  It starts before the host has the last step's bounds, which the grid stages wait for.  (N =
-// 200,003, 84 entries per row: 346 us per step with the reading of Y, 396 with the term behind the bounds and
-// the spectra, 1644 one stage after the other with an atomic per point, node and term.)
+// From kSide64Nnz entries of P on the attractive term runs on the second stream beside the grid stages, the 2D kernel
+// spectra on the third (unless overlap is off).  It starts before the host has the last step's bounds, which the
+// grid stages wait for.  (N = 200,003, 84 entries per row: 346 us per step with the reading of Y, 396 with the term
+// behind the bounds and the spectra, 1644 one stage after the other with an atomic per point, node and term.)
+// Below, the waits between streams cost more than the overlap gives: a step / a gradient with its wait on three
+// streams and on one, 2D, N = 2,000 with 30 entries per row 118 / 132 us and 102 / 97, 10,000 with 90 119 / 136 and
+// 104 / 100, 20,000 with 220 128 / 142 and 129 / 125, 50,000 with 90 142 / 151 and 142 / 137, with 260 168 / 180 and
+// 183 / 178; 1D, 50,000 with 250 181 / 190 and 180 / 182; and a context's first step makes the streams (30 us each,
+// the process's first 360).
+constexpr long long kSide64Nnz = 6000000;
 template <int D>
 static int pipeline_f64(fitsne_ctx *c, int mode, const fitsne_step_params *sp) {
     const int N = c->N, p = c->p;
@@ -1461,7 +1467,7 @@ static int pipeline_f64(fitsne_ctx *c, int mode, const fitsne_step_params *sp) {
         hipStream_t s;
         ~Restore() { c->stream = s; }
     } restore{c, main};
-    const bool side = c->overlap;
+    const bool side = c->overlap && c->nnz >= kSide64Nnz;
     if (side) {
         if (!c->astream) HIPTRY(hipStreamCreateWithFlags(&c->astream, hipStreamNonBlocking));
         if (D == 2 && !c->kstream) HIPTRY(hipStreamCreateWithFlags(&c->kstream, hipStreamNonBlocking));

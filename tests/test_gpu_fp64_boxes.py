@@ -67,3 +67,29 @@ def test_boxes(name, D):
         mni = 131 if D == 2 else 600  # (1D: an FFT of at most 4096)
         Y = rng.normal(0, 8, size=(3000, D))
     compare(Y, 1.0, mni=mni)
+
+
+@pytest.mark.parametrize("per", [61, 6])
+@pytest.mark.parametrize("D", [1, 2])
+def test_streams(D, per):
+    """Both sides of the six million entries from which the step runs on three streams: the gradient against the
+    oracle, and three steps with overlap on against those with it off (atomics add in any order)."""
+    N = 100_001
+    print(f"[gpu] fp64 streams D={D} per={per}", flush=True)
+    P = random_csr(N, per, seed=per, symmetric=False)
+    Y = blobs(N, D, 8, seed=D, span=30.0, sd=2.0)
+    out = []
+    for overlap in (True, False):
+        c = fg.Context(no_dims=D, precision=fg.FP64_PLAIN)
+        c.set_overlap(overlap)
+        c.set_P(*P)
+        c.set_Y(Y)
+        g, z = c.gradient()
+        for _ in range(3):
+            c.step(0.5, 200.0, 5.0)
+        out.append((g, z, c.get_Y()))
+        c.close()
+    want, zw = orc.gradient(P, Y)
+    for g, z, y in out:
+        assert rel(g, want) <= TOL and abs(z - zw) <= TOL * abs(zw)
+        assert rel(y, out[0][2]) <= TOL
