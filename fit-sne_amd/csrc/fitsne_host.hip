@@ -1541,7 +1541,8 @@ static int pipeline_f64(fitsne_ctx *c, int mode, const fitsne_step_params *sp) {
     TRY(ensure(c->bstart, sizeof(int) * ((size_t)nbox + 1)));
     int *used = c->bstart.as<int>(), *start = used + 1;
     const double *Y = c->Y.as<const double>();
-    launch(c, "box64", k_box_f64<D>, dim3(nblk), dim3(kThreads), 0, Y, N, g, box, rank, c->bcount.as<int>(), used, w,
+    const int bblk = std::max(nblk, std::min(blocks_for(nodes * nt), 2048));  // few points may have a large grid to clear
+    launch(c, "box64", k_box_f64<D>, dim3(bblk), dim3(kThreads), 0, Y, N, g, box, rank, c->bcount.as<int>(), used, w,
            nodes * nt);
     launch(c, "box_starts", k_box_starts, dim3(blocks_for(nbox)), dim3(kThreads), 0, c->bcount.as<int>(), nbox, used,
            start);
