@@ -2111,9 +2111,10 @@ static int set_P_impl(fitsne_ctx *c, int N, const TI *row_P, const TC *col_P, co
     TRY(copy_in(c, c->colP.p, col_P, sizeof(uint32_t) * nnz));
     if (c->precision == FITSNE_FP32) {
         TRY(ensure(c->val, sizeof(float) * (size_t)std::max<long long>(nnz, 1)));
-        // a small P is converted here, a large one on the device (a call with 252,000 entries 209 us, with 277,200
-        // 215; 18 million 8.5 ms, converted here 41)
-        std::vector<float> v(nnz <= (1 << 18) ? (size_t)nnz : 0);
+        // a small P is converted here, a large one on the device, from doubles that need a buffer of their own (582,000
+        // entries in a new context, here 395 us, on the device 1200, in a used one 399 and 469; 1.1 million on the
+        // device 735; 18 million 8.5 ms, here 41)
+        std::vector<float> v(nnz <= (1 << 20) ? (size_t)nnz : 0);
         for (size_t k = 0; k < v.size(); k++) v[k] = (float)val_P[k];
         if (!v.empty()) TRY(copy_in(c, c->val.p, v.data(), sizeof(float) * v.size()));
         constexpr long long kChunk = 4 << 20;  // doubles on the device at a time

@@ -79,10 +79,10 @@ def test_knn_refuses_non_finite(N, D, K):
 
 
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
-@pytest.mark.parametrize("nnz", [16383, 16385, 65535, 65537, 131071, 131073, 131137])
+@pytest.mark.parametrize("nnz", [16383, 16385, 65535, 65537, 131071, 131073, 131137, 1 << 20, (1 << 20) + 1])
 def test_small_P(nnz, prec):
-    """P whose columns (4 bytes) and values (4 or 8) end about the first buffer's halves and end: the
-    attractive term of every entry, by the gradient against the oracle."""
+    """P whose columns (4 bytes) and values (4 or 8) end about the first buffer's halves and end, and about the
+    2^20 entries up to which the host converts them: the attractive term of every entry, by the gradient against the oracle."""
     print(f"[gpu] copies P nnz={nnz} {prec}", flush=True)
     import orc
 
