@@ -1729,14 +1729,14 @@ static int bh_tree_on_host(fitsne_ctx *c) {
 
 // The tree of the resident Y (fitsne_bh.hpp): on the GPU unless it needs the reference's insertions.  beside():
 // work for a side stream that needs only P and Y.  Side streams: the exact mean, the check of the keys against
-// it and beside() on one, the root's center of mass on the other; the walk waits for both.  The host
-// reads back twice: the node count, which sizes what follows, and the check, by when the rest is queued.
+// it and beside() on one, the root's center of mass on the other; the walk waits for both (with overlap off
+// everything runs in turn on the context's stream).  The host reads back twice: the node count, which sizes what follows, and the check, by when the rest is queued.
 template <int D, typename F>
 static int bh_tree_of_Y(fitsne_ctx *c, F &&beside) {
     const int N = c->N;
     const double *Y = c->Y.as<const double>();
-    if (!c->astream) HIPTRY(hipStreamCreateWithFlags(&c->astream, hipStreamNonBlocking));
-    if (!c->kstream) HIPTRY(hipStreamCreateWithFlags(&c->kstream, hipStreamNonBlocking));
+    if (c->overlap && !c->astream) HIPTRY(hipStreamCreateWithFlags(&c->astream, hipStreamNonBlocking));
+    if (c->overlap && !c->kstream) HIPTRY(hipStreamCreateWithFlags(&c->kstream, hipStreamNonBlocking));
     if (!c->bh_ev) HIPTRY(hipEventCreateWithFlags(&c->bh_ev, hipEventDisableTiming));  // the host reads a copy after it
     if (c->bh_ab_n != N) {
         TRY(ensure(c->bh_ab, sizeof(double2) * ((size_t)N + 1)));
@@ -1777,13 +1777,14 @@ static int bh_tree_of_Y(fitsne_ctx *c, F &&beside) {
         hipStream_t s;
         ~Restore() { c->stream = s; }
     } restore{c, main};
+    const hipStream_t s1 = c->overlap ? c->astream : main, s2 = c->overlap ? c->kstream : main;
     HIPTRY(hipEventRecord(c->fork_ev, main));
-    HIPTRY(hipStreamWaitEvent(c->astream, c->fork_ev, 0));
-    HIPTRY(hipStreamWaitEvent(c->kstream, c->fork_ev, 0));
-    c->stream = c->astream;
+    HIPTRY(hipStreamWaitEvent(s1, c->fork_ev, 0));
+    HIPTRY(hipStreamWaitEvent(s2, c->fork_ev, 0));
+    c->stream = s1;
     launch(c, "bh_com_root", k_bh_com_root<D>, dim3(1), dim3(kWave), 0, Y, N, c->bh_ab.as<const double2>(), rcom);
-    HIPTRY(hipEventRecord(c->join_ev, c->astream));
-    c->stream = c->kstream;
+    HIPTRY(hipEventRecord(c->join_ev, s1));
+    c->stream = s2;
     launch(c, "bh_clear", k_bh_clear, dim3(1), dim3(1), 0, differs);
     launch(c, "bh_mean", k_bh_mean<D>, dim3(1), dim3(256), 0, Y, N, mean);
     c->stream = main;
@@ -1799,15 +1800,15 @@ static int bh_tree_of_Y(fitsne_ctx *c, F &&beside) {
            (const uint64_t *)key2, (const uint32_t *)sidx, (const unsigned char *)lost, N, lcp, cnt, info);
     // the check on the side stream, once the leaves' depths are there
     HIPTRY(hipEventRecord(c->kl_go, main));
-    HIPTRY(hipStreamWaitEvent(c->kstream, c->kl_go, 0));
-    c->stream = c->kstream;
+    HIPTRY(hipStreamWaitEvent(s2, c->kl_go, 0));
+    c->stream = s2;
     launch(c, "bh_check", k_bh_check<D>, dim3(blocks_for(N)), dim3(kThreads), 0, Y, N, (const double *)mean,
            (const double *)ext, (const uint64_t *)skey, (const uint64_t *)key2, (const uint32_t *)sidx, (const int *)lcp,
            exact, differs);
-    HIPTRY(hipMemcpyAsync((void *)&h->differs, differs, sizeof(int), hipMemcpyDeviceToHost, c->kstream));
-    HIPTRY(hipEventRecord(c->bh_ev, c->kstream));
+    HIPTRY(hipMemcpyAsync((void *)&h->differs, differs, sizeof(int), hipMemcpyDeviceToHost, s2));
+    HIPTRY(hipEventRecord(c->bh_ev, s2));
     const int rc = beside();
-    HIPTRY(hipEventRecord(c->kl_ev, c->kstream));
+    HIPTRY(hipEventRecord(c->kl_ev, s2));
     TRY(rc);
     c->stream = main;
     HIPTRY(rocprim::exclusive_scan(c->bh_tmp.p, t2, cnt, off, 0, (size_t)N + 1, rocprim::plus<int>(), main));

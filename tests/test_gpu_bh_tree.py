@@ -3,6 +3,8 @@ equal bit for bit at the edges of the build: the fewest points, chains of one th
 (64 to a chunk, 2048 the longest of the second list), the root's chunks (2048), the Z sum's runs (1024 and 16384);
 close pairs (deep trees), a far centre, tiny extents, and what goes to the host's insertions (duplicates, pairs
 closer than the keys resolve)."""
+import time
+
 import numpy as np
 import pytest
 
@@ -119,3 +121,29 @@ def test_far_apart(N, scale):
     print(f"[gpu] bh far apart N={N} scale={scale}", flush=True)
     with np.errstate(all="ignore"):
         compare(rng.normal(size=(N, 2)) * scale, 0.5)
+
+
+@pytest.mark.parametrize("D", [2, 3])
+def test_overlap_off(D):
+    """One kernel after another: the same bits, and kernel times that add up to no more than the call."""
+    N = 60_000
+    print(f"[gpu] bh overlap off D={D}", flush=True)
+    Y = np.random.default_rng(D).normal(size=(N, D)) * 20
+    P, out = small_P(N, 1), []
+    for overlap in (True, False):
+        c = fg.Context(no_dims=D, precision=fg.FP64_BH)
+        c.set_overlap(overlap)
+        c.set_P(*P)
+        c.set_Y(Y)
+        c.gradient()
+        c.set_timing(True)
+        t = time.perf_counter()
+        g, z = c.gradient()
+        t = (time.perf_counter() - t) * 1e3
+        if not overlap:
+            ms = sum(m for _, m in c.kernel_stats().values())
+            assert ms <= t, (ms, t)
+        out.append((g, z))
+        c.close()
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    assert out[0][1] == out[1][1]
