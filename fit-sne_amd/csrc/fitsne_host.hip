@@ -182,6 +182,7 @@ struct fitsne_ctx {
     DBuf bh_root, bh_key, bh_idx, bh_pos, bh_span, bh_list, bh_order, bh_tmp, bh_ab;
     int bh_ab_n = 0;
     hipEvent_t bh_ev = nullptr;
+    int bh_skip = 0, bh_back = 0;  // tree builds still to go to the host directly; how many after the last failed one
     bool bh_sorted = false;  // the current tree came from the GPU: bh_idx holds the points in key order
     // symmetrisation of a CSR P (mirror tier)
     DBuf sy_row, sy_col, sy_val, sy_erow, sy_keys, sy_keys2, sy_vals, sy_vals2, sy_partner, sy_cnt, sy_start,
@@ -1709,7 +1710,7 @@ static int bh_tree_on_host(fitsne_ctx *c) {
     const size_t ybytes = sizeof(double) * (size_t)N * D;
     TRY(bh_pinned(c, ybytes));
     HIPTRY(hipMemcpyAsync(c->bh_pin, c->Y.p, ybytes, hipMemcpyDeviceToHost, c->stream));
-    TRY(sync_ctx(c));
+    HIPTRY(hipStreamSynchronize(c->stream));
     c->bh_y.resize((size_t)N * D);
     std::memcpy(c->bh_y.data(), c->bh_pin, ybytes);
     BhTree<D> &t = bh_tree_for<D>(c);
@@ -1731,9 +1732,23 @@ static int bh_tree_on_host(fitsne_ctx *c) {
 // work for a side stream that needs only P and Y.  Side streams: the exact mean, the check of the keys against
 // it and beside() on one, the root's center of mass on the other; the walk waits for both (with overlap off
 // everything runs in turn on the context's stream).  The host reads back twice: the node count, which sizes what follows, and the check, by when the rest is queued.
+// Few points are inserted on the host at once: the build's dozen launches and two waits take as long (a gradient / a
+// step, on the GPU and on the host: 2D 300 points 271 / 215 and 143 / 144 us, 700 294 / 223 and 187 / 217, 1,500 346 / 258
+// and 300 / 378; 3D 200 250 / 192 and 185 / 177, 500 282 / 209 and 291 / 264; 1D 700 300 / 224 and 146 / 186).  And where
+// the last build ended on the host (coinciding points as a rule, which stay so for a while), the next 1, 3, 7 and
+// then 15 at a time go there directly (10,000 points of which 1,000 differ: 1020 us with the attempt, 655 without).
+constexpr int kBhBackMost = 15;
+template <int D>
+constexpr int kBhHostN = D == 3 ? 256 : 700;
+
 template <int D, typename F>
 static int bh_tree_of_Y(fitsne_ctx *c, F &&beside) {
     const int N = c->N;
+    if (N < kBhHostN<D> || c->bh_skip > 0) {
+        if (c->bh_skip > 0) c->bh_skip--;
+        TRY(beside());
+        return bh_tree_on_host<D>(c);
+    }
     const double *Y = c->Y.as<const double>();
     if (c->overlap && !c->astream) HIPTRY(hipStreamCreateWithFlags(&c->astream, hipStreamNonBlocking));
     if (c->overlap && !c->kstream) HIPTRY(hipStreamCreateWithFlags(&c->kstream, hipStreamNonBlocking));
@@ -1768,8 +1783,9 @@ static int bh_tree_of_Y(fitsne_ctx *c, F &&beside) {
         BhInfo info;
         int nodes, differs;
     };
-    TRY(bh_pinned(c, sizeof(Back)));
-    auto *h = static_cast<volatile Back *>(c->bh_pin);
+    // (not in bh_pin: the host's insertions may start before the check's answer is there)
+    static_assert(128 + sizeof(Back) <= 256, "behind h_mm's four doubles, before the stage");
+    auto *h = reinterpret_cast<volatile Back *>(reinterpret_cast<char *>(c->h_mm) + 128);
     // a side stream's launches, behind the work queued so far
     hipStream_t main = c->stream;
     struct Restore {
@@ -1846,9 +1862,17 @@ static int bh_tree_of_Y(fitsne_ctx *c, F &&beside) {
         HIPTRY(hipEventSynchronize(c->bh_ev));  // the check's answer
         ok = !h->differs;
     }
+    if (!ok) {
+        c->bh_back = std::min(2 * c->bh_back + 1, kBhBackMost);
+        c->bh_skip = c->bh_back;
+        TRY(bh_tree_on_host<D>(c));  // beside what the side streams still run
+        HIPTRY(hipStreamWaitEvent(main, c->join_ev, 0));
+        HIPTRY(hipStreamWaitEvent(main, c->kl_ev, 0));
+        return FITSNE_OK;
+    }
+    c->bh_back = 0;
     HIPTRY(hipStreamWaitEvent(main, c->join_ev, 0));
     HIPTRY(hipStreamWaitEvent(main, c->kl_ev, 0));
-    if (!ok) return bh_tree_on_host<D>(c);
     launch(c, "bh_finish", k_bh_finish<D>, dim3(blocks_for(nodes)), dim3(kThreads), 0, c->bh_span.as<const BhSpan>(),
            nodes, (const BhRoot *)exact, (const double *)rcom, bh_cells<D>(c));
     HIPTRY(hipGetLastError());
@@ -2449,6 +2473,7 @@ extern "C" int fitsne_set_Y(fitsne_ctx *c, const double *Y) {
         return sync_ctx(c);
     };
     TRY(c->precision == FITSNE_FP32 ? load(0.f) : load(0.0));
+    c->bh_skip = c->bh_back = 0;
     c->mm_valid = c->mm_pending = false;
     c->have_grad = false;
     c->kcache = false;

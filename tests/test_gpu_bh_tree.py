@@ -147,3 +147,38 @@ def test_overlap_off(D):
         c.close()
     np.testing.assert_array_equal(out[0][0], out[1][0])
     assert out[0][1] == out[1][1]
+
+
+@pytest.mark.parametrize("N,D", [(699, 1), (699, 2), (700, 1), (700, 2), (701, 2), (255, 3), (256, 3), (257, 3)])
+def test_about_the_host_line(N, D):
+    print(f"[gpu] bh host line N={N} D={D}", flush=True)
+    compare(np.random.default_rng(N + D).normal(0, 5, size=(N, D)), 0.6)
+
+
+def test_builds_that_end_on_the_host():
+    """Coinciding points send this and the next trees to the host; a new Y starts anew, between calls of both kinds."""
+    N = 2000
+    print("[gpu] bh host builds", flush=True)
+    rng = np.random.default_rng(9)
+    Y = rng.normal(0, 5, size=(N, 2))
+    Yd = Y.copy()
+    Yd[100:300] = Yd[:200]
+    P = small_P(N, 2)
+    c = fg.Context(no_dims=2, precision=fg.FP64_BH)
+    c.set_P(*P)
+    for V, calls in ((Yd, 7), (Y, 3), (Yd, 2), (Y, 1)):
+        c.set_Y(V)
+        gr, zr = orc.bh_gradient(P, V, 0.5)
+        for _ in range(calls):
+            g, z = c.gradient()
+            np.testing.assert_array_equal(g, gr)
+            assert z == zr
+    c.set_Y(Yd)
+    for _ in range(24):  # the pairs part after the first step; the GPU's trees come back on their own
+        c.step(0.5, 100.0)
+    V = c.get_Y()
+    g, z = c.gradient()
+    gr, zr = orc.bh_gradient(P, V, 0.5)
+    np.testing.assert_array_equal(g, gr)
+    assert z == zr
+    c.close()
