@@ -3838,11 +3838,11 @@ template <int NCH>
 static void knn_passes(fitsne_ctx *c, const KnnPlan &p, const KnnDev &d) {
     const size_t lds = sizeof(f16x8) * 2 * kKmCt<NCH> * NCH * 2 * kWave;
     launch(c, "knn_query", k_knn_query, dim3(p.npad / 256), dim3(256), 0, (const double *)d.nrm, p.N, p.npad,
-           (const float *)nullptr, d.QA);
+           16 * NCH, (const float *)nullptr, (const KnnScale *)d.sc, d.QA);
     launch(c, "knn_tau", k_knn_tau<NCH>, dim3(p.qblocks), dim3(kKmThreads), lds, (const f16x8 *)d.XC,
            (const f16x4 *)d.QA, p.N, p.D, (const f16x8 *)d.XS, p.NS, p.stride, d.cut);
     launch(c, "knn_query", k_knn_query, dim3(p.npad / 256), dim3(256), 0, (const double *)d.nrm, p.N, p.npad,
-           (const float *)d.cut, d.QA);
+           16 * NCH, (const float *)d.cut, (const KnnScale *)d.sc, d.QA);
     launch(c, "knn_collect", k_knn_collect<NCH>, dim3(p.qblocks * p.parts), dim3(kKmThreads), lds,
            (const f16x8 *)d.XC, (const f16x4 *)d.QA, p.N, p.D, p.qblocks, p.per, p.cap, d.cand, d.cnt);
 }

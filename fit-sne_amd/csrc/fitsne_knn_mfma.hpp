@@ -46,6 +46,7 @@ constexpr int kKmQueue = 2048;                 // candidate pass: queued hits pe
 constexpr int kKmAug = 6;                      // the last coordinates of the last chunk: the norms
 constexpr int kKmMaxCh = 9;                    // chunks of 16 coordinates: D + 6 <= 144
 constexpr int kKmMaxD = 128, kKmMaxK = 256;
+constexpr double kKmNever = -60000.0;          // a constant that keeps every accumulator below 0 (they reach 2,048)
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -211,7 +212,7 @@ __global__ __launch_bounds__(256) void k_knn_prep(const double *__restrict__ X, 
         part[blockIdx.x] = m;
     }
     auto pieces = [&](int r, int c, int g, bool real, f16x8 &h, f16x8 &l) {
-        const f16x4 b = knn_split3(real ? -0.5 * sn[r] : -60000.0);
+        const f16x4 b = knn_split3(real ? -0.5 * sn[r] : kKmNever);
 #pragma unroll
         for (int j = 0; j < 8; j++) {
             const int k = 16 * c + 8 * g + j;
@@ -254,13 +255,20 @@ __global__ __launch_bounds__(256) void k_knn_prep(const double *__restrict__ X, 
         }
 }
 
-// The query's constant -|x|^2 / 2 - acc[q] as three halves (acc null: no threshold yet).  Queries past N
-// never pass.
-__global__ __launch_bounds__(256) void k_knn_query(const double *__restrict__ nrm, int N, int npad,
-                                                   const float *__restrict__ acc, f16x4 *__restrict__ QA) {
+// The query's constant -|x|^2 / 2 - cut[q] as three halves (cut null: no threshold yet).  Queries past N, and with
+// kKmNever as their constant also those that the exact pass must refuse in any case (the threshold lies within the
+// error bound of distance zero: many coinciding points, or a scale set by far outliers), never pass.
+__global__ __launch_bounds__(256) void k_knn_query(const double *__restrict__ nrm, int N, int npad, int kp,
+                                                   const float *__restrict__ cut, const KnnScale *__restrict__ sc,
+                                                   f16x4 *__restrict__ QA) {
     const int q = blockIdx.x * 256 + threadIdx.x;
     if (q >= npad) return;
-    QA[q] = knn_split3(q < N ? -0.5 * nrm[q] - (acc ? (double)acc[q] : 0.0) : -60000.0);
+    double c = kKmNever;
+    if (q < N) {
+        const double k = cut ? (double)cut[q] : 0.0;
+        if (!cut || knn_err(nrm[q], sc->nmax, fabs(k), kp) < -k) c = -0.5 * nrm[q] - k;
+    }
+    QA[q] = knn_split3(c);
 }
 
 // The sweep both passes share: the workgroup's queries q0 .. q0 + 255 of XQ (candidate tiles, the norm
@@ -426,7 +434,9 @@ __global__ __launch_bounds__(kKmThreads, NCH <= 7 ? 2 : 1) void k_knn_tau(const 
 // into cand[q][0 .. cap) as (~accumulator bits, j): ascending keys are ascending distances; count[q]
 // (zeroed by the caller) = how many there were.  Workgroup (query block, part of the points).  Hits are
 // queued in LDS and written out when the queue is half full: ranks within the queue by LDS atomics, then
-// one global atomic per query; what the queue cannot take goes out by itself.
+// one global atomic per query; what the queue cannot take goes out by itself, unless the query's list has overflowed
+// already (full: a bit each), as where many points lie at one distance just inside the threshold: N hits for every
+// query (5,000 points in 30 places: 4.7 ms a call with a global atomic for each, 1.9 so).
 template <int NCH>
 __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__restrict__ XC,
                                                             const f16x4 *__restrict__ QA, int N, int D, int qblocks,
@@ -436,16 +446,19 @@ __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__re
     __shared__ unsigned long long qkey[kKmQueue];
     __shared__ unsigned char qq_[kKmQueue];
     __shared__ int hist[kKmWg];
+    __shared__ unsigned full[kKmWg / 32];
     __shared__ int qn, qflag[2];
     static_assert(kKmWg <= 256, "a queued hit's query is one byte");
     const int w = threadIdx.x / kWave, l = threadIdx.x % kWave, tid = threadIdx.x;
     const int q0 = (blockIdx.x % qblocks) * kKmWg, part = blockIdx.x / qblocks;
     const int tiles = (N + 31) / 32;
     const int t0 = part * per, t1 = min(tiles, t0 + per);
+    if (!__syncthreads_or((float)QA[q0 + tid][0] > 0.5f * (float)kKmNever)) return;  // none of the queries can pass
     if (tid == 0) {
         qn = 0;
         qflag[0] = qflag[1] = 0;
     }
+    if (tid < kKmWg / 32) full[tid] = 0;
     auto flush = [&]() {  // whole workgroup
         __syncthreads();
         const int n = min(qn, kKmQueue);
@@ -461,6 +474,7 @@ __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__re
         const int mine = hist[tid];
         int base = 0;
         if (mine && q0 + tid < N) base = atomicAdd(&count[q0 + tid], mine);
+        if (base + mine > cap) atomicOr(&full[tid / 32], 1u << tid % 32);
         __syncthreads();
         hist[tid] = base;
         __syncthreads();
@@ -506,9 +520,10 @@ __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__re
                     if (pos < kKmQueue) {
                         qkey[pos] = key;
                         qq_[pos] = (unsigned char)qq;
-                    } else if (q0 + qq < N) {
+                    } else if (q0 + qq < N && !(*(volatile unsigned *)&full[qq / 32] >> qq % 32 & 1u)) {
                         const int p = atomicAdd(&count[q0 + qq], 1);
                         if (p < cap) cand[(long)(q0 + qq) * cap + p] = key;
+                        else atomicOr(&full[qq / 32], 1u << qq % 32);
                     }
                 }
                 at += __popcll(m);
@@ -526,7 +541,7 @@ __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__re
 // Exact pass: one workgroup of one wavefront per query.  Of its candidates, those whose accumulator is
 // within two error bounds of the K-th largest (nearest) are evaluated: FP64 squared distances
 // (coordinate order, no fused multiply-add, as the FP64 kernel), sorted by (distance, index); the first K
-// go to out_idx / out_dist (square root correctly rounded).  X is read as rows of Dp doubles.  A query
+// go to out_idx / out_dist (square root correctly rounded).  A query
 // whose list is short or overflowed, or whose K-th distance does not clear the threshold less the error
 // bound, is appended to redo[] instead.
 constexpr int kKmExact = 512;  // FP64 distances per query

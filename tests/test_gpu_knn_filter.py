@@ -75,3 +75,33 @@ def test_filter_matches_the_fp64_kernel(N, D, K):
     assert np.array_equal(i_f, i_e[:, :K])
     assert np.array_equal(d_f, d_e[:, :K])
     assert redo <= N // 100
+
+
+@pytest.mark.parametrize("name", ["cauchy", "half_equal", "most_equal", "ten_points", "one_far", "few_far", "lattice", "mass_and_rest", "thirty_places"])
+@pytest.mark.parametrize("N", [1300, 4100])
+def test_filter_where_queries_cannot_pass(name, N):
+    """Thresholds within the error bound of zero distance, for all queries, for some of every workgroup, for whole
+    workgroups: those go to the FP64 kernel, the others through the lists."""
+    rng = np.random.default_rng(N)
+    X = mixture(N, 12, N)
+    if name == "cauchy":
+        X = rng.standard_cauchy((N, 12))
+    elif name == "half_equal":
+        X[rng.random(N) < 0.5] = 1.0
+    elif name == "most_equal":
+        X[rng.random(N) < 0.97] = 1.0
+    elif name == "ten_points":
+        X = X[rng.integers(0, 10, N)]
+    elif name == "one_far":
+        X[5] *= 1e6
+    elif name == "few_far":
+        X[::100] *= 1e3
+    elif name == "lattice":
+        X = np.round(X[:, :3] / 3.0)
+    elif name == "thirty_places":  # all at one distance from each other: every list overflows
+        X = np.eye(30)[rng.integers(0, 30, N)]
+    else:
+        X[: N // 2] = X[0]  # whole workgroups of coinciding points, in front
+    print(f"[gpu] knn filter {name} N={N}", flush=True)
+    check(X, 40, fg.knn_mfma(X, 40)[:2])
+    check(X, 40, fg.knn_exact(X, 40))
