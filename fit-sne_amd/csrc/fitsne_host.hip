@@ -3795,8 +3795,10 @@ struct KnnSlab {
 };
 
 struct KnnPlan {
-    int N, D, K, nch, stride, NS, npad, nspad, cap, qblocks, parts, per;
+    int N, D, K, nch, stride, NS, npad, nspad, cap, qblocks, qper, parts, per;
 };
+
+constexpr int kKmQueries = 1 << 19;
 
 // The threshold sample's stride and the list length.  About 33 strides of all points lie nearer than the
 // cut (kKmRank of 64 classes: 64 (H64 - H38) sample points), give or take a fifth.  A list is short only if
@@ -3815,9 +3817,13 @@ static KnnPlan knn_plan(int N, int D, int K) {
     p.npad = (N + kKmWg - 1) / kKmWg * kKmWg;
     p.nspad = (p.NS + 31) / 32 * 32;
     p.qblocks = p.npad / kKmWg;
+    // candidates are collected for so many queries at a time, so that their lists take 3.2 to 9.7 GB at most whatever
+    // N (300,000 queries in three rounds of 2^17 took the same as in one)
+    const int most = kKmQueries / kKmWg, rounds = (p.qblocks + most - 1) / most;
+    p.qper = (p.qblocks + rounds - 1) / rounds;
     // enough workgroups for several rounds of the chip, each with at least 16 tiles to sweep
     const int tiles = (N + 31) / 32;
-    const int parts = std::max(1, std::min(tiles / 16, (2048 + p.qblocks - 1) / p.qblocks));
+    const int parts = std::max(1, std::min(tiles / 16, (2048 + p.qper - 1) / p.qper));
     p.per = ((tiles + parts - 1) / parts + 1) / 2 * 2;
     p.parts = (tiles + p.per - 1) / p.per;
     return p;
@@ -3835,16 +3841,30 @@ struct KnnDev {
 };
 
 template <int NCH>
-static void knn_passes(fitsne_ctx *c, const KnnPlan &p, const KnnDev &d) {
+static void knn_thresholds(fitsne_ctx *c, const KnnPlan &p, const KnnDev &d) {
     const size_t lds = sizeof(f16x8) * 2 * kKmCt<NCH> * NCH * 2 * kWave;
-    launch(c, "knn_query", k_knn_query, dim3(p.npad / 256), dim3(256), 0, (const double *)d.nrm, p.N, p.npad,
-           16 * NCH, (const float *)nullptr, (const KnnScale *)d.sc, d.QA);
+    launch(c, "knn_query", k_knn_query, dim3(p.npad / 256), dim3(256), 0, (const double *)d.nrm, p.N, p.npad, 16 * NCH,
+           (const float *)nullptr, (const KnnScale *)d.sc, d.QA);
     launch(c, "knn_tau", k_knn_tau<NCH>, dim3(p.qblocks), dim3(kKmThreads), lds, (const f16x8 *)d.XC,
-           (const f16x4 *)d.QA, p.N, p.D, (const f16x8 *)d.XS, p.NS, p.stride, d.cut);
-    launch(c, "knn_query", k_knn_query, dim3(p.npad / 256), dim3(256), 0, (const double *)d.nrm, p.N, p.npad,
-           16 * NCH, (const float *)d.cut, (const KnnScale *)d.sc, d.QA);
-    launch(c, "knn_collect", k_knn_collect<NCH>, dim3(p.qblocks * p.parts), dim3(kKmThreads), lds,
-           (const f16x8 *)d.XC, (const f16x4 *)d.QA, p.N, p.D, p.qblocks, p.per, p.cap, d.cand, d.cnt);
+           (const f16x4 *)d.QA, p.N, (const f16x8 *)d.XS, p.NS, p.stride, d.cut);
+    launch(c, "knn_query", k_knn_query, dim3(p.npad / 256), dim3(256), 0, (const double *)d.nrm, p.N, p.npad, 16 * NCH,
+           (const float *)d.cut, (const KnnScale *)d.sc, d.QA);
+}
+
+// Candidates and neighbours of all queries, p.qper blocks of kKmWg at a time.
+template <int NCH>
+static void knn_candidates(fitsne_ctx *c, const KnnPlan &p, const KnnDev &d, int *idx, double *dist, int *redo,
+                           int *nredo) {
+    const size_t lds = sizeof(f16x8) * 2 * kKmCt<NCH> * NCH * 2 * kWave;
+    auto rerank = p.cap == 768 ? k_knn_rerank<12> : p.cap == 1536 ? k_knn_rerank<24> : k_knn_rerank<36>;
+    for (int b = 0; b < p.qblocks; b += p.qper) {
+        const int nb = std::min(p.qper, p.qblocks - b), first = b * kKmWg;
+        launch(c, "knn_collect", k_knn_collect<NCH>, dim3(nb * p.parts), dim3(kKmThreads), lds, (const f16x8 *)d.XC,
+               (const f16x4 *)d.QA, p.N, first, nb, p.per, p.cap, d.cand, d.cnt);
+        launch(c, "knn_rerank", rerank, dim3(std::min(nb * kKmWg, p.N - first)), dim3(kWave), 0, d.X, first, p.D, p.K,
+               16 * p.nch, (const unsigned long long *)d.cand, (const int *)d.cnt, (const float *)d.cut,
+               (const double *)d.nrm, (const KnnScale *)d.sc, idx, dist, redo, nredo);
+    }
 }
 
 // Neighbours by the filter, the queries it cannot settle by the FP64 kernel (their number into *nredo).
@@ -3856,7 +3876,7 @@ static int knn_filtered(fitsne_ctx *c, const double *X, int N, int D, int K, int
     KnnSlab m;
     const size_t oX = m.need<double>(nd), oXC = m.need<f16x8>(p.npad / 32 * tile), oXS = m.need<f16x8>(p.nspad / 32 * tile);
     const size_t oQA = m.need<f16x4>(p.npad), oN = m.need<double>(N), oCut = m.need<float>(N);
-    const size_t oCand = m.need<unsigned long long>((size_t)N * p.cap), oCnt = m.need<int>(N);
+    const size_t oCand = m.need<unsigned long long>((size_t)std::min(N, p.qper * kKmWg) * p.cap), oCnt = m.need<int>(N);
     const size_t oI = m.need<int>(nk), oD = m.need<double>(nk), oR = m.need<int>((size_t)N + 1);
     const size_t oPart = m.need<double>(std::max((size_t)cblk * D + eblk, (size_t)tblk)), oMean = m.need<double>(D), oSc = m.need<KnnScale>(1);
     TRY(ensure(m.b, m.at));
@@ -3878,21 +3898,21 @@ static int knn_filtered(fitsne_ctx *c, const double *X, int N, int D, int K, int
     launch(c, "knn_prep", k_knn_prep, dim3(tblk), dim3(256), 0, d.X, N, D, p.nch, (const double *)mean,
            (const KnnScale *)d.sc, p.stride, p.NS, p.nspad, d.XC, d.XS, d.nrm, part);
     launch(c, "knn_nmax", k_knn_nmax, dim3(1), dim3(1024), 0, (const double *)part, tblk, d.sc);
+    auto run = [&](auto nch) {
+        knn_thresholds<decltype(nch)::value>(c, p, d);
+        knn_candidates<decltype(nch)::value>(c, p, d, di, dd, redo, nr);
+    };
     switch (p.nch) {
-    case 1: knn_passes<1>(c, p, d); break;
-    case 2: knn_passes<2>(c, p, d); break;
-    case 3: knn_passes<3>(c, p, d); break;
-    case 4: knn_passes<4>(c, p, d); break;
-    case 5: knn_passes<5>(c, p, d); break;
-    case 6: knn_passes<6>(c, p, d); break;
-    case 7: knn_passes<7>(c, p, d); break;
-    case 8: knn_passes<8>(c, p, d); break;
-    default: knn_passes<9>(c, p, d); break;
+    case 1: run(std::integral_constant<int, 1>{}); break;
+    case 2: run(std::integral_constant<int, 2>{}); break;
+    case 3: run(std::integral_constant<int, 3>{}); break;
+    case 4: run(std::integral_constant<int, 4>{}); break;
+    case 5: run(std::integral_constant<int, 5>{}); break;
+    case 6: run(std::integral_constant<int, 6>{}); break;
+    case 7: run(std::integral_constant<int, 7>{}); break;
+    case 8: run(std::integral_constant<int, 8>{}); break;
+    default: run(std::integral_constant<int, 9>{}); break;
     }
-    auto rerank = p.cap == 768 ? k_knn_rerank<12> : p.cap == 1536 ? k_knn_rerank<24> : k_knn_rerank<36>;
-    launch(c, "knn_rerank", rerank, dim3(N), dim3(kWave), 0, d.X, N, D, K, 16 * p.nch,
-           (const unsigned long long *)d.cand, (const int *)d.cnt, (const float *)d.cut, (const double *)d.nrm,
-           (const KnnScale *)d.sc, di, dd, redo, nr);
     HIPTRY(hipGetLastError());
     int n = 0;
     HIPTRY(hipMemcpyAsync(&n, nr, sizeof(int), hipMemcpyDeviceToHost, c->stream));

@@ -278,7 +278,7 @@ __global__ __launch_bounds__(256) void k_knn_query(const double *__restrict__ nr
 // one barrier and 6 KB NCH of LDS reads (half the LDS rate at eight wavefronts per CU); the next stage is
 // loaded straight to LDS meanwhile.
 template <int NCH, int TS, typename V, typename S>
-__device__ __forceinline__ void knn_sweep(const f16x8 *__restrict__ XQ, const f16x4 *__restrict__ QA, int D, int q0,
+__device__ __forceinline__ void knn_sweep(const f16x8 *__restrict__ XQ, const f16x4 *__restrict__ QA, int q0,
                                           const f16x8 *__restrict__ XC, int t0, int t1, f16x8 *stage, V &&visit,
                                           S &&step) {
     constexpr int CT = kKmCt<NCH>, TILE = NCH * 2 * kWave;  // f16x8 per tile
@@ -378,7 +378,7 @@ __device__ __forceinline__ float knn_unbits(unsigned u) {
 // takes 8.4 ms.)
 template <int NCH>
 __global__ __launch_bounds__(kKmThreads, NCH <= 7 ? 2 : 1) void k_knn_tau(const f16x8 *__restrict__ XC,
-                                                           const f16x4 *__restrict__ QA, int N, int D,
+                                                           const f16x4 *__restrict__ QA, int N,
                                                            const f16x8 *__restrict__ XS, int NS, int stride,
                                                            float *__restrict__ cut) {
     extern __shared__ f16x8 knn_stage[];
@@ -402,11 +402,11 @@ __global__ __launch_bounds__(kKmThreads, NCH <= 7 ? 2 : 1) void k_knn_tau(const 
     };
     const int tiles = (NS + 31) / 32;
     knn_sweep<NCH, 2>(
-        XC, QA, D, q0, XS, 0, tiles, knn_stage,
+        XC, QA, q0, XS, 0, tiles, knn_stage,
         [&](auto T, int j0, const f32x16 &acc) { keep(T.value == 0 ? b00 : b01, T.value, j0, acc); }, [](int) {});
     __syncthreads();  // the stage is free
     knn_sweep<NCH, 2>(
-        XC, QA, D, q0, XS, 1, tiles, knn_stage,
+        XC, QA, q0, XS, 1, tiles, knn_stage,
         [&](auto T, int j0, const f32x16 &acc) { keep(T.value == 0 ? b10 : b11, T.value, j0, acc); }, [](int) {});
     auto finish = [&](int t, const f32x16 &v0, const f32x16 &v1) {
 #pragma unroll
@@ -430,8 +430,8 @@ __global__ __launch_bounds__(kKmThreads, NCH <= 7 ? 2 : 1) void k_knn_tau(const 
     finish(1, b01, b11);
 }
 
-// Candidate pass: every point j != q whose accumulator (the constant of QA holds the threshold) is above 0
-// into cand[q][0 .. cap) as (~accumulator bits, j): ascending keys are ascending distances; count[q]
+// Candidate pass of the queries first .. first + kKmWg qblocks: every point j != q whose accumulator (the constant of QA
+// holds the threshold) is above 0 into cand[q - first][0 .. cap) as (~accumulator bits, j): ascending keys are ascending distances; count[q]
 // (zeroed by the caller) = how many there were.  Workgroup (query block, part of the points).  Hits are
 // queued in LDS and written out when the queue is half full: ranks within the queue by LDS atomics, then
 // one global atomic per query; what the queue cannot take goes out by itself, unless the query's list has overflowed
@@ -439,8 +439,9 @@ __global__ __launch_bounds__(kKmThreads, NCH <= 7 ? 2 : 1) void k_knn_tau(const 
 // query (5,000 points in 30 places: 4.7 ms a call with a global atomic for each, 1.9 so).
 template <int NCH>
 __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__restrict__ XC,
-                                                            const f16x4 *__restrict__ QA, int N, int D, int qblocks,
-                                                            int per, int cap, unsigned long long *__restrict__ cand,
+                                                            const f16x4 *__restrict__ QA, int N, int first,
+                                                            int qblocks, int per, int cap,
+                                                            unsigned long long *__restrict__ cand,
                                                             int *__restrict__ count) {
     extern __shared__ f16x8 knn_stage[];
     __shared__ unsigned long long qkey[kKmQueue];
@@ -450,7 +451,8 @@ __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__re
     __shared__ int qn, qflag[2];
     static_assert(kKmWg <= 256, "a queued hit's query is one byte");
     const int w = threadIdx.x / kWave, l = threadIdx.x % kWave, tid = threadIdx.x;
-    const int q0 = (blockIdx.x % qblocks) * kKmWg, part = blockIdx.x / qblocks;
+    const int q0 = first + (blockIdx.x % qblocks) * kKmWg, part = blockIdx.x / qblocks;
+    unsigned long long *mine_at = cand + (long)(q0 - first) * cap;  // the workgroup's lists
     const int tiles = (N + 31) / 32;
     const int t0 = part * per, t1 = min(tiles, t0 + per);
     if (!__syncthreads_or((float)QA[q0 + tid][0] > 0.5f * (float)kKmNever)) return;  // none of the queries can pass
@@ -483,7 +485,7 @@ __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__re
             const int e = i * kKmThreads + tid;
             if (e < n) {
                 const int pos = hist[qq_[e]] + rank[i];
-                if (pos < cap && q0 + qq_[e] < N) cand[(long)(q0 + qq_[e]) * cap + pos] = qkey[e];
+                if (pos < cap && q0 + qq_[e] < N) mine_at[qq_[e] * cap + pos] = qkey[e];
             }
         }
         __syncthreads();
@@ -491,7 +493,7 @@ __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__re
         __syncthreads();
     };
     knn_sweep<NCH, 1>(
-        XC, QA, D, q0, XC, t0, t1, knn_stage,
+        XC, QA, q0, XC, t0, t1, knn_stage,
         [&](auto T, int j0, const f32x16 &acc) {
             constexpr int t = T.value;
             if (!__any(knn_max16(acc) > 0.f)) return;
@@ -522,7 +524,7 @@ __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__re
                         qq_[pos] = (unsigned char)qq;
                     } else if (q0 + qq < N && !(*(volatile unsigned *)&full[qq / 32] >> qq % 32 & 1u)) {
                         const int p = atomicAdd(&count[q0 + qq], 1);
-                        if (p < cap) cand[(long)(q0 + qq) * cap + p] = key;
+                        if (p < cap) mine_at[qq * cap + p] = key;
                         else atomicOr(&full[qq / 32], 1u << qq % 32);
                     }
                 }
@@ -538,7 +540,7 @@ __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__re
     flush();
 }
 
-// Exact pass: one workgroup of one wavefront per query.  Of its candidates, those whose accumulator is
+// Exact pass: one workgroup of one wavefront per query, from `first` on.  Of its candidates, those whose accumulator is
 // within two error bounds of the K-th largest (nearest) are evaluated: FP64 squared distances
 // (coordinate order, no fused multiply-add, as the FP64 kernel), sorted by (distance, index); the first K
 // go to out_idx / out_dist (square root correctly rounded).  A query
@@ -546,7 +548,7 @@ __global__ __launch_bounds__(kKmThreads, 2) void k_knn_collect(const f16x8 *__re
 // bound, is appended to redo[] instead.
 constexpr int kKmExact = 512;  // FP64 distances per query
 template <int CAPL>
-__global__ __launch_bounds__(kWave) void k_knn_rerank(const double *__restrict__ X, int N, int D, int K, int kp,
+__global__ __launch_bounds__(kWave) void k_knn_rerank(const double *__restrict__ X, int first, int D, int K, int kp,
                                                       const unsigned long long *__restrict__ cand,
                                                       const int *__restrict__ count, const float *__restrict__ cut,
                                                       const double *__restrict__ nrm,
@@ -557,7 +559,7 @@ __global__ __launch_bounds__(kWave) void k_knn_rerank(const double *__restrict__
     __shared__ int ii[kKmExact];
     constexpr int CAP = CAPL * kWave;
     const int l = threadIdx.x;
-    const int q = blockIdx.x;
+    const int q = first + blockIdx.x;
     const int n = count[q];
     auto give_up = [&]() {
         if (l == 0) redo[atomicAdd(nredo, 1)] = q;
@@ -573,7 +575,7 @@ __global__ __launch_bounds__(kWave) void k_knn_rerank(const double *__restrict__
         if (s * kWave < n) {
             const int e = s * kWave + l;
             if (e < n) {
-                const unsigned long long key = cand[(long)q * CAP + e];
+                const unsigned long long key = cand[(long)blockIdx.x * CAP + e];
                 hi[s] = (unsigned)(key >> 32);
                 id[s] = (int)(unsigned)key;
             }

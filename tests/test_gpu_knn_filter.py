@@ -105,3 +105,24 @@ def test_filter_where_queries_cannot_pass(name, N):
     print(f"[gpu] knn filter {name} N={N}", flush=True)
     check(X, 40, fg.knn_mfma(X, 40)[:2])
     check(X, 40, fg.knn_exact(X, 40))
+
+
+@pytest.mark.parametrize("N", [524288, 524289, 600001])
+def test_queries_in_rounds(N):
+    """As many queries as their lists are kept for at once (2^19), and more: the neighbours of some of every round,
+    those at its ends among them, by distances added in coordinate order."""
+    D, K = 3, 12
+    X = mixture(N, D, N, k=40)
+    print(f"[gpu] knn filter rounds N={N}", flush=True)
+    idx, dist, redo = fg.knn_mfma(X, K)
+    assert redo <= N // 100
+    half = (N + 511) // 512 * 256
+    for q in [0, 1, half - 1, half, half + 1, N - 257, N - 2, N - 1] + list(np.random.default_rng(1).integers(0, N, 40)):
+        d2 = np.zeros(N)
+        for d in range(D):
+            d2 += (X[q, d] - X[:, d]) ** 2
+        d2[q] = np.inf
+        near = np.argpartition(d2, K + 8)[: K + 9]
+        near = near[np.lexsort((near, d2[near]))][:K]
+        assert np.array_equal(idx[q], near)
+        assert np.array_equal(dist[q], np.sqrt(d2[near]))
