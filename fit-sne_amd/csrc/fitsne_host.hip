@@ -3947,13 +3947,24 @@ static int knn_plain(fitsne_ctx *c, const double *X, int N, int D, int K, int32_
     return sync_ctx(c);
 }
 
-// The filter's fewest points (its sample must hit kKmRank classes), and the least work fitsne_knn_exact
-// takes it for.  The filter's dozen launches cost 0.5 to 0.7 ms whatever the size; the FP64 kernel's time
-// goes with N (D + 40) while N is small (whole calls, D = 50, K = 90: 0.79 against 0.80 ms at N = 1,500, 1.92
-// against 0.89 at 5,000; D = 20, K = 30: 0.41 against 0.55 ms at 2,000, 0.79 against 0.54 at 5,000; D = 100,
-// K = 30: 0.63 against 0.59 ms at 1,024).
+// The filter's fewest points (its sample must hit kKmRank classes).
 constexpr int kKnnFilterMinN = 1024;
-constexpr long kKnnFilterWork = 150000;
+// Whether fitsne_knn_exact takes it.  Its dozen launches and its lists cost 0.45 to 0.8 ms a call whatever the size; the
+// FP64 kernel's time goes with N (D + a number that grows with K) while N is small.  Whole calls, us, FP64 kernel / filter:
+//   K = 15  N = 4,000 D = 35 523 / 514, D = 60 638 / 535; 7,000 D = 20 592 / 476; 12,000 D = 12 739 / 844, D = 20 920 / 849;
+//           20,000 D = 8 1100 / 1058, D = 12 1301 / 1105; 30,000 D = 2 1444 / 1342, D = 1 1263 / 2085
+//   K = 30  2,500 D = 60 549 / 567; 4,000 D = 20 491 / 496, D = 35 603 / 534; 10,000 D = 4 747 / 874; 12,000 D = 8 813 / 861,
+//           D = 12 901 / 895; 20,000 D = 2 1129 / 1103, D = 8 1362 / 1164; 30,000 D = 2 1866 / 1491, D = 1 1706 / 2522
+//   K = 60  1,100 D = 1 664 / 599, D = 100 837 / 621; 4,000 D = 2 1295 / 527  (the FP64 kernel's buffer is cut often)
+//   K = 90  1,600 D = 35 576 / 617, D = 60 634 / 646; 2,500 D = 4 596 / 613, D = 35 757 / 657; 4,000 D = 1 682 / 599
+//   K = 250 1,600 D = 20 923 / 963, D = 60 1039 / 990; 2,500 D = 1 1113 / 1036
+// (D = 1 at small K: the neighbours are so near each other that the filter passes many queries on.)
+static bool knn_filter_pays(int N, int D, int K) {
+    const long nd = (long)N * D;
+    if (K > 64) return N >= 3000 || nd >= 90000;
+    if (K > 32) return true;
+    return nd >= (K > 20 ? 140000 : 220000) || (N >= 25000 && D >= 2);
+}
 
 extern "C" int fitsne_knn_exact(const double *X, int N, int D, int K, int32_t *idx, double *dist) {
     TRY(knn_args(X, N, D, K, idx, dist));
@@ -3961,7 +3972,7 @@ extern "C" int fitsne_knn_exact(const double *X, int N, int D, int K, int32_t *i
     fitsne_ctx *c;
     TRY(mirror_ctx(&c, 1, 3, 1.0, 1, 1.0));
     HIPTRY(hipSetDevice(c->device));
-    if (N >= kKnnFilterMinN && D <= kKmMaxD && K <= kKmMaxK && (long)N * (D + 40) >= kKnnFilterWork) {
+    if (N >= kKnnFilterMinN && D <= kKmMaxD && K <= kKmMaxK && knn_filter_pays(N, D, K)) {
         const int rc = knn_filtered(c, X, N, D, K, idx, dist, nullptr);
         if (rc != FITSNE_E_ALLOC) return rc;
         (void)hipGetLastError();  // no room for the candidate lists: the FP64 kernel needs none

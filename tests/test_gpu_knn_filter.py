@@ -126,3 +126,18 @@ def test_queries_in_rounds(N):
         near = near[np.lexsort((near, d2[near]))][:K]
         assert np.array_equal(idx[q], near)
         assert np.array_equal(dist[q], np.sqrt(d2[near]))
+
+
+@pytest.mark.parametrize("N,D,K", [
+    (1024, 1, 33), (1024, 3, 64), (1100, 60, 65), (1400, 64, 65), (1407, 64, 65), (2999, 5, 70), (3000, 5, 70),
+    (2188, 64, 21), (2187, 64, 21), (2000, 110, 20), (1999, 110, 20), (1500, 40, 32), (25000, 2, 8), (25000, 1, 8)])
+def test_either_side_of_the_routes(N, D, K):
+    """fitsne_knn_exact where it goes over from the FP64 kernel to the filter."""
+    X = mixture(N, D, N + K)
+    print(f"[gpu] knn_exact routes N={N} D={D} K={K}", flush=True)
+    got = fg.knn_exact(X, K)
+    if N <= 3000:
+        check(X, K, got)
+    i_e, d_e = fg.knn_exact(X, 257)
+    assert np.array_equal(got[0], i_e[:, :K])
+    assert np.array_equal(got[1], d_e[:, :K])
