@@ -334,12 +334,18 @@ static int att_lanes(long long nnz, int N) {
 // other, and large ones have several threads for the memcpy (fresh pages: 4.8 GB/s with one thread, 21 with
 // eight; DMA 57).
 
-// Threads that copy their share of a piece beside the caller's; they last for one stage_copy.
+// Threads that copy their share of a piece beside the caller's; they last for one stage_copy.  All copies of the
+// process that run at once share kCopyHelpers of them.
+constexpr int kCopyHelpers = 7;
+static std::atomic<int> g_copy_helpers{0};
 class CopyTeam {
   public:
     explicit CopyTeam(int helpers) {
+        int busy = g_copy_helpers.load(std::memory_order_relaxed);
+        do mine_ = std::max(0, std::min(helpers, kCopyHelpers - busy));
+        while (mine_ > 0 && !g_copy_helpers.compare_exchange_weak(busy, busy + mine_, std::memory_order_relaxed));
         try {
-            for (int i = 0; i < helpers; i++) th_.emplace_back([this, i] { work(i + 1); });
+            for (int i = 0; i < mine_; i++) th_.emplace_back([this, i] { work(i + 1); });
         } catch (...) {  // no more threads: copy with those that started
         }
     }
@@ -347,6 +353,7 @@ class CopyTeam {
         stop_ = true;
         gen_.fetch_add(1, std::memory_order_release);
         for (auto &t : th_) t.join();
+        if (mine_ > 0) g_copy_helpers.fetch_sub(mine_, std::memory_order_relaxed);
     }
     void copy(char *dst, const char *src, size_t len) {
         dst_ = dst;
@@ -380,6 +387,7 @@ class CopyTeam {
         }
     }
     std::vector<std::thread> th_;
+    int mine_ = 0;
     std::atomic<int> gen_{0}, left_{0};
     bool stop_ = false;
     char *dst_ = nullptr;
@@ -418,7 +426,7 @@ constexpr size_t kStageDirect = 1 << 20;
 // bytes from device memory dev to host (out) or back, on c->stream behind what is queued there; done when it
 // returns.  Pieces: a quarter of the copy, from 512 KB (uploads of 404 and 829 KB in pieces of 256 KB 20 to 25 us longer: a
 // DMA of its own each) to half the buffer.
-// Helpers: one per 4 MB (starting one costs 20 us), at most seven.
+// Helpers: one per 4 MB (starting one costs 20 us), at most kCopyHelpers.
 static int stage_copy(fitsne_ctx *c, char *host, char *dev, size_t bytes, bool out) {
     if (!bytes) return FITSNE_OK;
     const size_t piece = std::min(std::max((bytes / 4 + 4095) & ~(size_t)4095, (size_t)512 << 10), kStage / 2);
@@ -431,7 +439,7 @@ static int stage_copy(fitsne_ctx *c, char *host, char *dev, size_t bytes, bool o
                    : hipMemcpyAsync(dev + k * piece, half(k), len(k), hipMemcpyHostToDevice, c->stream);
     };
     if (out) HIPTRY(dma(0));
-    CopyTeam team(bytes >> 22 ? (int)std::min<size_t>({bytes >> 22, 7, std::max(1u, std::thread::hardware_concurrency()) - 1}) : 0);
+    CopyTeam team(bytes >> 22 ? (int)std::min<size_t>({bytes >> 22, kCopyHelpers, std::max(1u, std::thread::hardware_concurrency()) - 1}) : 0);
     for (size_t k = 0; k < n; k++) {
         if (out) {
             HIPTRY(hipStreamSynchronize(c->stream));

@@ -101,3 +101,32 @@ def test_small_P(nnz, prec):
     want, _ = orc.gradient((row, col, val), Y)
     r = np.linalg.norm(g - want) / np.linalg.norm(want)
     assert r <= (1e-9 if prec == "fp64" else 1e-4), r
+
+
+def test_contexts_copying_at_once():
+    """Several threads, each with its own context and large copies, share the helper threads."""
+    import threading
+
+    N = 1300003
+    print("[gpu] copies from four threads", flush=True)
+    bad = []
+
+    def work(k):
+        try:
+            Y = fixed_order(np.random.default_rng(k).normal(size=(N, 2)))
+            c = fg.Context(no_dims=2, precision=fg.FP64_PLAIN)
+            c.set_P(*chain_P(N))
+            for r in range(3):
+                c.set_Y(Y * (r + 1))
+                if not np.array_equal(c.get_Y().reshape(N, 2), Y * (r + 1)):
+                    bad.append((k, r))
+            c.close()
+        except Exception as e:  # (a thread's exception would not fail the test)
+            bad.append((k, repr(e)))
+
+    th = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not bad
