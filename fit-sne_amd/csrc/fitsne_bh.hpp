@@ -26,8 +26,8 @@
 //      beside everything else.
 // Coinciding points, points closer than 2 kBhLevels halvings and points that rounding leaves outside every
 // child, and keys that the exact root changes, are recognised, and that iteration's tree is built on the
-// host by the reference's insertions (BhTree).  Contraction is off and sqrt / divisions are correctly rounded, so the result is the
-// reference's to the bit either way.
+// host by the reference's insertions (BhTree), as it is for few points.  Contraction is off and sqrt / divisions
+// are correctly rounded, so the result is the reference's to the bit either way.
 #pragma once
 
 #include <cfloat>

@@ -1205,8 +1205,9 @@ struct SpreadWaveLds {
 // step, 60 entries per row, table with its streams / straight on one stream): 3 nodes N = 5,000 97 / 72, 20,000 118
 // / 86, 30,000 119 / 100, 40,000 117 / 111, 50,000 114 / 125, 70,000 129 / 156 (captured 30,000 145 / 135, 40,000 147 /
 // 150, 70,000 157 / 197); 2 nodes 40,000 95 / 83, 70,000 103 / 106.  With 4 and 5 nodes the values of a box fill the
-// table's slots sooner: 70,000 303 / 165 and 472 / 237, 140,000 460 / 270 and 816 / 414 (points still in their sorted
-// order 188 / 204 and 194 / 281).  In 1D straight is no faster from 10,000 points on (70,000 88 / 102, captured 92 /
+// table's slots sooner: 70,000 303 / 165 and 472 / 237, 140,000 460 / 270 and 816 / 414.  (From a PCA start the points
+// stay in order longer: 3 nodes 45,000 106 / 94, 70,000 111 / 110, 140,000 126 / 150; 4 nodes 140,000 168 / 183, 5
+// nodes 100,000 174 / 213.)  In 1D straight is no faster from 10,000 points on (70,000 88 / 102, captured 92 /
 // 109) and within 3% below: always the table.
 constexpr int kSpreadWaveN = 40000, kSpreadWaveNWide = 150000;  // up to 3 nodes per box and side, and more
 constexpr bool spread_waves(int D, int p, int N) { return D == 2 && N < (p <= 3 ? kSpreadWaveN : kSpreadWaveNWide); }

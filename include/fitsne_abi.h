@@ -288,14 +288,15 @@ int fitsne_autotune_stats(fitsne_ctx *ctx, int *spread_points, int *attractive_r
  * rows (8192 in 1D) cut so that their modelled times match, one per CU; else a multiple of 64 up to 4096
  * (8192 in 1D)).  The forces are bitwise the same for every value. */
 int fitsne_set_attractive_rows(fitsne_ctx *ctx, int rows);
-/* Set the spread's points per workgroup directly (a multiple of 512 in [512, 8192]; default 1024). */
+/* Set the spread's points per workgroup directly (a multiple of 512 in [512, 8192]; default 1024).  Small 2D
+ * contexts (below 40,000 points, 150,000 with 4 or 5 nodes per box) use it only as members of a batch. */
 int fitsne_set_spread_points(fitsne_ctx *ctx, int points);
 
 /* Batched embeddings (no reference counterpart): one optimisation step of every context of the batch
  * (FP32 contexts on one device, each with its own P and Y): each context's captured step is launched
  * on its own stream, so the embeddings' steps overlap on the device.  prm[n] holds each context's
- * parameters.  Results are bitwise those of stepping each context alone.  Creating a batch runs the
- * autotuner on each context. */
+ * parameters.  Results are bitwise those of stepping each context alone.  Creating a batch tunes
+ * each context's spread. */
 typedef struct fitsne_batch fitsne_batch;
 int fitsne_batch_create(fitsne_batch **batch, fitsne_ctx **ctxs, int n);
 int fitsne_batch_step(fitsne_batch *batch, const fitsne_step_params *prm);
