@@ -398,7 +398,7 @@ class CopyTeam {
 
 constexpr size_t kStage = 4u << 20;
 // The context's first pinned allocation: h_mm in 256 bytes, then the stage (it costs 12 us, of 16 KB as of 4 MB).
-constexpr size_t kStageFirst = (512 << 10) + 256;
+constexpr size_t kStageFirst = (1 << 20) + 256;
 static char *first_stage(const fitsne_ctx *c) { return reinterpret_cast<char *>(c->h_mm) + 256; }
 
 // At least `need` (<= kStage) bytes of pinned buffer; nothing may be in flight in it.
@@ -426,7 +426,8 @@ constexpr size_t kStageDirect = 1 << 20;
 // bytes from device memory dev to host (out) or back, on c->stream behind what is queued there; done when it
 // returns.  Pieces: a quarter of the copy, from 512 KB (uploads of 404 and 829 KB in pieces of 256 KB 20 to 25 us longer: a
 // DMA of its own each) to half the buffer.
-// Helpers: one per 4 MB (starting one costs 20 us), at most kCopyHelpers.
+// Helpers: one per 4 MB (starting one costs 20 us), at most kCopyHelpers; uploads, whose pages are there, have them
+// from 16 MB on (8 MB 266 us a call with one helper, 237 without; the runtime's own copy 231).
 static int stage_copy(fitsne_ctx *c, char *host, char *dev, size_t bytes, bool out) {
     if (!bytes) return FITSNE_OK;
     const size_t piece = std::min(std::max((bytes / 4 + 4095) & ~(size_t)4095, (size_t)512 << 10), kStage / 2);
@@ -439,7 +440,7 @@ static int stage_copy(fitsne_ctx *c, char *host, char *dev, size_t bytes, bool o
                    : hipMemcpyAsync(dev + k * piece, half(k), len(k), hipMemcpyHostToDevice, c->stream);
     };
     if (out) HIPTRY(dma(0));
-    CopyTeam team(bytes >> 22 ? (int)std::min<size_t>({bytes >> 22, kCopyHelpers, std::max(1u, std::thread::hardware_concurrency()) - 1}) : 0);
+    CopyTeam team(bytes >> (out ? 22 : 24) ? (int)std::min<size_t>({bytes >> 22, kCopyHelpers, std::max(1u, std::thread::hardware_concurrency()) - 1}) : 0);
     for (size_t k = 0; k < n; k++) {
         if (out) {
             HIPTRY(hipStreamSynchronize(c->stream));
